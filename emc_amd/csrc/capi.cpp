@@ -283,7 +283,7 @@ extern "C" emc_status emc_create(const emc_dims *d, const emc_options *o, emc_ct
         if (st == EMC_OK) A(dalloc(&c->pdirty, Sp * (int64_t)p_segments(c)), "pdirty");
         if (st == EMC_OK) A(hipMemset(c->pdirty, 1, sizeof(uint8_t) * Sp * p_segments(c)), "pdirty");
         if (st == EMC_OK) A(dalloc(&c->runmax, Ip), "runmax");
-        if (st == EMC_OK) A(dalloc(&c->blk, (int64_t)softmax_fused_bands(c) * Ip), "blk");
+        if (st == EMC_OK) A(dalloc(&c->blk, (int64_t)softmax_fused_bands_max(c) * Ip), "blk");
         if (st == EMC_OK) A(dalloc(&c->colsum, 2 * (int64_t)PpMax), "colsum");
         if (st == EMC_OK) A(dalloc(&c->colp, colp_len(c->S, PpMax)), "colp");
         if (st == EMC_OK) A(dalloc(&c->colpart, colpart_len(PpMax)), "colpart");
@@ -335,7 +335,7 @@ extern "C" emc_status emc_create(const emc_dims *d, const emc_options *o, emc_ct
     // gives them p = exp(x - inf) = 0, which needs finite x: nothing else writes them
     if (st == EMC_OK) A(hipMemset(c->R, 0, sizeof(float) * Sp * Ip), "R");
     if (st == EMC_OK) A(dalloc(&c->lse, Ip), "lse");
-    c->part_len = std::max<int64_t>(emc::softmax_part_len(c->S, c->I, softmax_fused_bands(c)), 4096);
+    c->part_len = std::max<int64_t>(emc::softmax_part_len(c->S, c->I, softmax_fused_bands_max(c)), 4096);
     if (st == EMC_OK) A(dalloc(&c->part, c->part_len), "part");
     if (st == EMC_OK) A(dalloc(&c->red, kRedLen), "red");
     if (st == EMC_OK) A(dalloc(&c->T, Sp), "T");

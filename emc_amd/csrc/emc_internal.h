@@ -257,9 +257,11 @@ hipError_t launch_square_counts(const emc_ctx *c, hipStream_t st);
 // MFMA contractions.
 hipError_t launch_logl_mfma(const emc_ctx *c, int s0, int cs, hipStream_t st);
 // C [chunkp][Ip] (=, or += with accumulate) sum over pixels of A [chunkp][Pp] (na BF16 terms) and
-// the counts-like operand B [Ip][Pp] (BF16, or bytes when B8 is given): the large-tile kernel.
-hipError_t launch_gemm_store_mfma(const emc_ctx *c, int na, const bf16_t *A0, const bf16_t *A1, const bf16_t *A2,
-                                  const bf16_t *B16, const uint8_t *B8, float *C, bool accumulate, hipStream_t st);
+// the counts-like operand B [Ip][Pp] (nb BF16 terms; B8: the same as bytes, which the register-staged
+// kernels read), term pairs a + b < max(na, nb).
+hipError_t launch_gemm_store_mfma(const emc_ctx *c, int na, const bf16_t *A0, const bf16_t *A1, const bf16_t *A2, int nb,
+                                  const bf16_t *B0, const bf16_t *B1, const uint8_t *B8, float *C, bool accumulate,
+                                  hipStream_t st);
 // chi^2 logits of rotations [s0, s0+cs) on the MFMA path, from the chunk's FP32 slices (A0 = W,
 // A1 = the pixel weight a): D = sum a W^2 - 2 ip sum a W K + ip^2 sum a K^2 over the valid pixels,
 // ip = 1/phi (options.scaling: sum W K / sum K^2 over W > 1e-10; else 1); R = log w_s - D rscale_s.
@@ -280,9 +282,12 @@ constexpr int kSparseMaxPp = 16384;
 hipError_t launch_mstep_sparse(const emc_ctx *c, int s0, int cs, const double *gate, double gate_thr, hipStream_t st);
 
 // Responsibilities.  When logl_fuses_softmax(c), the logL contraction's epilogue writes the
-// per-band softmax partials (one band per 256 rotation rows) and launch_softmax skips its pass.
+// per-band softmax partials (one band per logl_band_rows rotation rows: the contraction's tile, 256 or, for
+// smaller shapes, 128 or 64) and launch_softmax skips its pass.
 bool logl_fuses_softmax(const emc_ctx *c);
+int logl_band_rows(const emc_ctx *c);
 int softmax_fused_bands(const emc_ctx *c);
+int softmax_fused_bands_max(const emc_ctx *c);  // over the pattern sets the context may be given (buffer sizes)
 // The logL pass leaves out the stores of negligible bands' logits (c->skip_logits on the DMA kernel).
 bool logl_skips_stores(const emc_ctx *c);
 int64_t softmax_part_len(int S, int I, int fused_bands);

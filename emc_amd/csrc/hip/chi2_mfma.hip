@@ -106,22 +106,18 @@ hipError_t launch_logl_chi2_mfma(const emc_ctx *c, int s0, int cs, hipStream_t s
     hipError_t e = hipGetLastError();
     auto op = [&](int p, int q) { return c->Cx + (int64_t)(p * NT + q) * plane; };
     auto with_counts = [&](int p, float *C) {  // C = X_p . K^T (hi + lo counts above 256)
-        hipError_t err = launch_gemm_store_mfma(c, NT, op(p, 0), op(p, 1), NT == 3 ? op(p, 2) : nullptr, c->K16, c->K8,
-                                                C, false, st);
+        hipError_t err = launch_gemm_store_mfma(c, NT, op(p, 0), op(p, 1), NT == 3 ? op(p, 2) : nullptr, 1, c->K16,
+                                                nullptr, c->K8, C, false, st);
         if (err == hipSuccess && c->k_split)
-            err = launch_gemm_store_mfma(c, NT, op(p, 0), op(p, 1), NT == 3 ? op(p, 2) : nullptr, c->K16lo, nullptr, C,
-                                         true, st);
+            err = launch_gemm_store_mfma(c, NT, op(p, 0), op(p, 1), NT == 3 ? op(p, 2) : nullptr, 1, c->K16lo, nullptr,
+                                         nullptr, C, true, st);
         return err;
     };
     // C = X_p . (K^2)^T with na terms of X_p; the low half of K^2 meets na - 1 of them (at least
     // one): the dropped product of the two lowest terms is below 2^-16 of the sum's terms.
     auto with_squares = [&](int p, int na, float *C) {
-        hipError_t err = launch_gemm_store_mfma(c, na, op(p, 0), op(p, 1), na == 3 ? op(p, 2) : nullptr, c->K2h,
-                                                nullptr, C, false, st);
-        const int nl = na > 1 ? na - 1 : 1;
-        if (err == hipSuccess && c->k2_split)
-            err = launch_gemm_store_mfma(c, nl, op(p, 0), op(p, 1), nullptr, c->K2l, nullptr, C, true, st);
-        return err;
+        return launch_gemm_store_mfma(c, na, op(p, 0), op(p, 1), na == 3 ? op(p, 2) : nullptr, c->k2_split ? 2 : 1,
+                                      c->K2h, c->K2l, nullptr, C, false, st);
     };
     float *R = c->R + (size_t)s0 * c->Ip;
     if (e == hipSuccess) e = with_counts(0, R);

@@ -133,7 +133,7 @@ constexpr int kApplyCols = 1024; // pattern columns per workgroup (4 per thread)
 // OUT = 1 skips the store of a wave's 256-pattern row segment when every value in it is zero and
 // pdirty says the segment already holds only zeros (P is mostly zeros once the posteriors are
 // sharp); pdirty is then updated to whether the segment holds a non-zero value.
-// pm (the logL epilogue's band maxima, [band][I], band of row s = (s / chunk) bpc + (s % chunk) / 256;
+// pm (the logL epilogue's band maxima, [band][I], band of row s = (s / chunk) bpc + (s % chunk) / brows;
 // null without them): a pattern's logits in a band whose maximum lies more than kSkipApplyNats below
 // its lse are not read and count as -inf, which gives the P = 0 that they give (exp of less than -110
 // is 0 in FP32).  blk (the skipping logL pass's record, [band][I]; null when every logit is in
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256) void k_sm_apply(float *__restrict__ R, int64_t
                                                   bf16_t *__restrict__ Pl, double *__restrict__ Tpart,
                                                   double *__restrict__ nnz, const float *__restrict__ iphi,
                                                   uint8_t *__restrict__ pdirty, int nseg, const float *__restrict__ pm,
-                                                  const int16_t *__restrict__ blk, int chunk, int bpc)
+                                                  const int16_t *__restrict__ blk, int chunk, int bpc, int brows)
 {
     static_assert(kApplyRows == 8, "8 rows: two per wave in the row sums, 8 floats per block read");
     constexpr float kLog2e = 1.4426950408889634f;
@@ -190,10 +190,10 @@ __global__ __launch_bounds__(256) void k_sm_apply(float *__restrict__ R, int64_t
     bool one_band = false;
     if (OUT == 1 && pm) {
         const int rl = min(r0 + kApplyRows - 1, S - 1);
-        b0 = (r0 / chunk) * bpc + (r0 % chunk) / 256;
-        one_band = b0 == (rl / chunk) * bpc + (rl % chunk) / 256;
+        b0 = (r0 / chunk) * bpc + (r0 % chunk) / brows;
+        one_band = b0 == (rl / chunk) * bpc + (rl % chunk) / brows;
         if (one_band) {  // the workgroup's rows lie in one band (always, when blk is given)
-            brow0 = (r0 / chunk) * chunk + ((r0 % chunk) / 256) * 256;
+            brow0 = (r0 / chunk) * chunk + ((r0 % chunk) / brows) * brows;
             float pv[4];
             int cv[4] = {-2, -2, -2, -2};
             const size_t o = (size_t)b0 * I + c0;
@@ -506,10 +506,10 @@ hipError_t launch_softmax(const emc_ctx *c, hipStream_t st)
         hipLaunchKernelGGL(k_sm_apply<1>, ga, dim3(256), 0, st, c->R, (int64_t)c->Ip, S, I, c->lse, c->Ph, c->Pl,
                            Tpart, nzpart, c->opt.scaling ? c->iphi : nullptr, c->pdirty, p_segments(c),
                            fused ? pm : nullptr, fused && c->logits_partial ? c->blk : nullptr, c->chunk,
-                           c->chunkp / 256);
+                           c->chunkp / logl_band_rows(c), logl_band_rows(c));
     else
         hipLaunchKernelGGL(k_sm_apply<0>, ga, dim3(256), 0, st, c->R, (int64_t)c->Ip, S, I, c->lse, nullptr, nullptr,
-                           Tpart, nullptr, nullptr, nullptr, 0, nullptr, nullptr, 1, 1);
+                           Tpart, nullptr, nullptr, nullptr, 0, nullptr, nullptr, 1, 1, 1);
     hipLaunchKernelGGL(k_T_final, dim3((c->Sp + 255) / 256), dim3(256), 0, st, Tpart, ncb, S, c->Sp, c->T);
     if (c->mfma) hipLaunchKernelGGL(k_sum_f64, dim3(1), dim3(1024), 0, st, nzpart, (int)(ga.x * ga.y), c->scal + SC_NNZ);
     return hipGetLastError();

@@ -100,13 +100,14 @@ typedef struct emc_options {
                                 precision).  0 = phi = 1 (known_intensity = true) */
     int32_t tile_rows;       /* large-tile MFMA contractions: row panels per group of consecutive tiles
                                 (L2 reuse within an XCD); 0 = the built-in default */
-    int32_t mfma_staging;    /* 256-row MFMA contractions of a two-term operand with a one-term one
-                                (logL, dense M-step, chi^2 sums): 0 = operands staged in LDS by direct
+    int32_t mfma_staging;    /* 256-row MFMA contractions with a one-term counts operand (logL, dense
+                                M-step, chi^2 sums): 0 = operands staged in LDS by direct
                                 global->LDS loads (BF16 counts), 1 = staged through registers (byte
                                 counts widened in registers).  Same products in the same order:
                                 identical results */
     int32_t keep_logits;     /* emc_iterate with the MFMA likelihood: 0 = the logL kernel leaves out
-                                the stores of a 256-rotation band's logits for a pattern when the
+                                the stores of a rotation band's (its tile's rows: 64 to 256
+                                rotations) logits for a pattern when the
                                 band's largest logit lies more than 128 below a largest logit
                                 already found for that pattern (its responsibilities there are
                                 exactly 0; the softmax reads those logits as -inf).  The iteration's
@@ -151,7 +152,7 @@ typedef struct emc_iter_stats {
                               responsibility mass inside the cells the network would keep; else -1 */
     double train_loss;     /* mean cross-entropy of the last training pass; -1 if none ran */
     double work_fraction;  /* scored (rotation, pattern) pairs / (S * I) */
-    double logits_skipped; /* fraction of the (256-rotation band, pattern) logit blocks whose stores
+    double logits_skipped; /* fraction of the (rotation band, pattern) logit blocks whose stores
                               the logL kernel left out (options.keep_logits = 0); 0 otherwise */
 } emc_iter_stats;
 
