@@ -444,8 +444,10 @@ int softmax_fused_bands_max(const emc_ctx *c)
 
 bool logl_skips_stores(const emc_ctx *c)
 {
-    // the softmax's 8-row groups must not straddle a band (chunks of a multiple of 8 rotations)
-    return c->skip_logits && logl_fuses_softmax(c) && c->opt.mfma_staging == 0 && c->chunk % 8 == 0;
+    // the softmax's 8-row groups must not straddle a band (chunks of a multiple of 8 rotations); three-term
+    // slices and two-term counts keep every logit, which a caller may read after an iteration
+    return c->skip_logits && logl_fuses_softmax(c) && c->la_terms == 2 && !c->k_split && c->opt.mfma_staging == 0 &&
+           c->chunk % 8 == 0;
 }
 
 // One contraction by the kernel of its tile (with more terms than one launch of the larger tiles takes, the
