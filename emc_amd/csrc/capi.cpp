@@ -897,8 +897,8 @@ static emc_status compress_enqueue(emc_ctx *c)
     ev_start(c, EMC_STAGE_COMPRESS);
     // divide, normalise over the voxels that received weight, blur (the numerator, free after the
     // divide, is the blur's second buffer)
-    HIP_TRY(c, launch_compress_buffers(c->L, c->opt.blur_sigma > 0.0, c->Mnum, c->Wt, c->model, c->taps, c->tmp3,
-                                       c->Mnum, c->red, c->scal, c->stream));
+    HIP_TRY(c, launch_compress_buffers(c->L, c->opt.blur_sigma, false, c->Mnum, c->Wt, c->model, c->taps, c->tmp3,
+                                       c->Mnum, c->red, c->scal, nullptr, c->stream));
     ev_stop(c, EMC_STAGE_COMPRESS);
     return EMC_OK;
 }

@@ -304,10 +304,12 @@ hipError_t launch_normalize(const emc_ctx *c, bool apply, bool support, hipStrea
 // Blur taps of side L (FP64 sums, stored as float).
 hipError_t launch_blur_taps(int L, double sigma, float *taps, hipStream_t st);
 // Compress on explicit buffers: divide, normalise over the voxels with weight (FP64 partials in
-// red [kRedLen], scalars in scal [SC_N]), blur when asked (t1, t2: two L^3 volumes; t2 may be
-// Mnum, which the divide has consumed).
-hipError_t launch_compress_buffers(int L, bool blur, const float *Mnum, const float *Wt, float *model,
-                                   const float *taps, float *t1, float *t2, double *red, double *scal, hipStream_t st);
+// red [kRedLen], scalars in scal [SC_N], the average to avg_out too when given), blur when blur_sigma > 0
+// (taps [L], formed here with new_taps; t1, t2: two L^3 volumes; t2 may be Mnum, which the divide has
+// consumed).
+hipError_t launch_compress_buffers(int L, double blur_sigma, bool new_taps, const float *Mnum, const float *Wt,
+                                   float *model, float *taps, float *t1, float *t2, double *red, double *scal,
+                                   double *avg_out, hipStream_t st);
 // Deterministic single-workgroup sum of n doubles into *out.
 hipError_t launch_sum_f64(const double *x, int n, double *out, hipStream_t st);
 

@@ -272,6 +272,7 @@ hipError_t pick(const Contraction &g, hipStream_t st)
     case kTile256: return launch<EPI, NA, NB, 4, 4>(g, st);
     case kTile256x128: return launch<EPI, NA, NB, 4, 2>(g, st);
     case kTile128: return launch<EPI, NA, NB, 2, 2>(g, st);
+    case kTile64: break;
     }
     return hipErrorInvalidValue;
 }

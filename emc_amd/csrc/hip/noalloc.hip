@@ -45,17 +45,6 @@ hipError_t scratch_of_current_device(void **out)
     return hipSuccess;
 }
 
-// The scalars keep the last call's values: the ones the compress flags must start at zero.
-__global__ void k_clear_scalars(double *__restrict__ scal)
-{
-    if (threadIdx.x < SC_N) scal[threadIdx.x] = 0.0;
-}
-
-__global__ void k_copy_avg(const double *__restrict__ scal, double *__restrict__ out)
-{
-    if (threadIdx.x == 0) *out = scal[SC_AVG];
-}
-
 emc_status fail(emc_status st, const std::string &msg)
 {
     emc_host_fail(st, msg.c_str());
@@ -84,15 +73,7 @@ extern "C" emc_status emc_compress_device(int32_t L, double blur_sigma, const fl
     float *t1 = reinterpret_cast<float *>(base), *t2 = reinterpret_cast<float *>(base + kVolBytes);
     double *red = reinterpret_cast<double *>(base + kOffRed), *scal = reinterpret_cast<double *>(base + kOffScal);
     float *taps = reinterpret_cast<float *>(base + kOffTaps);
-    const bool blur = blur_sigma > 0.0;
-    hipLaunchKernelGGL(k_clear_scalars, dim3(1), dim3(64), 0, st, scal);
-    e = hipGetLastError();
-    if (e == hipSuccess && blur) e = launch_blur_taps(L, blur_sigma, taps, st);
-    if (e == hipSuccess) e = launch_compress_buffers(L, blur, Mnum, Wt, model, taps, t1, t2, red, scal, st);
-    if (e == hipSuccess && avg) {
-        hipLaunchKernelGGL(k_copy_avg, dim3(1), dim3(64), 0, st, scal, avg);
-        e = hipGetLastError();
-    }
+    e = launch_compress_buffers(L, blur_sigma, true, Mnum, Wt, model, taps, t1, t2, red, scal, avg, st);
     if (e != hipSuccess) return fail(EMC_E_HIP, std::string("compress_device: ") + hipGetErrorString(e));
     return EMC_OK;
 }
