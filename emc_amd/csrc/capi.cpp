@@ -280,8 +280,6 @@ extern "C" emc_status emc_create(const emc_dims *d, const emc_options *o, emc_ct
         if (st == EMC_OK && c->la_terms == 3) A(dalloc(&c->Lm, cp * PpMax), "Lm");
         if (st == EMC_OK) A(dalloc(&c->Ph, Sp * Ip), "Ph");
         if (st == EMC_OK) A(dalloc(&c->Pl, Sp * Ip), "Pl");
-        if (st == EMC_OK) A(dalloc(&c->pdirty, Sp * (int64_t)p_segments(c)), "pdirty");
-        if (st == EMC_OK) A(hipMemset(c->pdirty, 1, sizeof(uint8_t) * Sp * p_segments(c)), "pdirty");
         if (st == EMC_OK) A(dalloc(&c->runmax, Ip), "runmax");
         if (st == EMC_OK) A(dalloc(&c->blk, (int64_t)softmax_fused_bands_max(c) * Ip), "blk");
         if (st == EMC_OK) A(dalloc(&c->colsum, 2 * (int64_t)PpMax), "colsum");
@@ -331,6 +329,8 @@ extern "C" emc_status emc_create(const emc_dims *d, const emc_options *o, emc_ct
     if (st == EMC_OK) A(dalloc(&c->rscale, Sp), "rscale");
     if (st == EMC_OK) A(dalloc(&c->cst, Ip), "cst");
     if (st == EMC_OK) A(dalloc(&c->R, Sp * Ip), "R");
+    if (st == EMC_OK) A(dalloc(&c->pdirty, Sp * (int64_t)p_segments(c)), "pdirty");
+    if (st == EMC_OK) A(hipMemset(c->pdirty, 1, sizeof(uint8_t) * Sp * p_segments(c)), "pdirty");
     // the responsibilities pass reads the padding columns [I, Ip) of a row beside the real ones and
     // gives them p = exp(x - inf) = 0, which needs finite x: nothing else writes them
     if (st == EMC_OK) A(hipMemset(c->R, 0, sizeof(float) * Sp * Ip), "R");
@@ -757,6 +757,7 @@ static emc_status softmax_enqueue(emc_ctx *c)
 {
     ev_start(c, EMC_STAGE_SOFTMAX);
     HIP_TRY(c, launch_softmax(c, c->stream));
+    c->pphi_stale = false;
     ev_stop(c, EMC_STAGE_SOFTMAX);
     return EMC_OK;
 }
@@ -802,8 +803,14 @@ extern "C" emc_status emc_set_resp(emc_ctx *c, const float *resp)
         T[s] = t;
     }
     if (!c->mfma) {
+        double nnz = 0.0;  // read by the M-step's choice of form, as after an E-step
+        for (size_t k = 0; k < (size_t)S * I; ++k) nnz += resp[k] != 0.0f;
+        HIP_TRY(c, hipMemcpy(c->scal + SC_NNZ, &nnz, sizeof(double), hipMemcpyHostToDevice));
         HIP_TRY(c, hipMemcpy2D(c->R, sizeof(float) * c->Ip, resp, sizeof(float) * I, sizeof(float) * I, S,
                                hipMemcpyHostToDevice));
+        HIP_TRY(c, launch_mark_p_dirty(c, c->stream));
+        HIP_TRY(c, hipStreamSynchronize(c->stream));
+        c->pphi_stale = true;
         c->has_logl = false;
     } else {
         std::vector<bf16_t> h((size_t)S * I), l((size_t)S * I);
@@ -854,12 +861,15 @@ static emc_status mstep_enqueue(emc_ctx *c)
         HIP_TRY(c, launch_fill_f32(c->Wt, 0.0f, c->N3, st));
     }
     const bool fused = c->mfma && c->opt.insert == EMC_INSERT_FUSED;
-    // MFMA M-step form: both kernels are enqueued in AUTO mode and the one not chosen by the
+    // M-step form: both kernels are enqueued in AUTO mode and the one not chosen by the
     // E-step's non-zero count (scal[SC_NNZ]) returns at once, so the host never waits for it
     const int mode = fused || c->Pp > kSparseMaxPp ? EMC_MSTEP_DENSE : c->opt.mstep;
     const double thr = 0.02 * (double)c->S * (double)c->I;
     const double *gate = c->scal + SC_NNZ;
-    if (!c->mfma && c->opt.scaling) HIP_TRY(c, launch_pscale_f32(c, st));  // the M-step sums K P / phi
+    if (!c->mfma && c->opt.scaling && c->pphi_stale) {  // the M-step sums K P / phi
+        HIP_TRY(c, launch_pscale_f32(c, st));
+        c->pphi_stale = false;
+    }
     for (int s0 = 0; s0 < c->S; s0 += c->chunk) {
         const int cs = std::min(c->chunk, c->S - s0);
         const int k = s0 / c->chunk;
@@ -870,7 +880,10 @@ static emc_status mstep_enqueue(emc_ctx *c)
             if (mode != EMC_MSTEP_SPARSE)
                 HIP_TRY(c, launch_mstep_mfma(c, s0, cs, fused, mode == EMC_MSTEP_AUTO ? gate : nullptr, thr, st));
         } else {
-            HIP_TRY(c, launch_mstep_f32(c, s0, cs, st));
+            if (mode != EMC_MSTEP_DENSE)
+                HIP_TRY(c, launch_mstep_sparse(c, s0, cs, mode == EMC_MSTEP_AUTO ? gate : nullptr, thr, st));
+            if (mode != EMC_MSTEP_SPARSE)
+                HIP_TRY(c, launch_mstep_f32(c, s0, cs, mode == EMC_MSTEP_AUTO ? gate : nullptr, thr, st));
         }
         gev_rec(c, 1, k, 1);
         if (c->opt.insert == EMC_INSERT_BINNED) HIP_TRY(c, launch_insert_binned(c, s0, cs, st));

@@ -183,7 +183,8 @@ struct emc_ctx {
     // responsibilities
     float *R = nullptr;                                // [Sp][Ip] logits (P in place on FP32 path)
     emc::bf16_t *Ph = nullptr, *Pl = nullptr;          // [Sp][Ip] BF16 hi/lo P (MFMA path)
-    uint8_t *pdirty = nullptr;  // [Sp][ceil(I/256)]: 0 = that 256-pattern segment of Ph/Pl holds only zeros
+    uint8_t *pdirty = nullptr;  // [Sp][ceil(I/256)]: 0 = that 256-pattern segment of P (Ph/Pl; R) holds only zeros
+    bool pphi_stale = false;    // emc_set_resp replaced P: Pphi does not follow from it yet
     int32_t *runmax = nullptr;  // [Ip] per pattern, the largest band maximum of the logits found so far in
                                 // this logL pass (order-preserving integer form of a float)
     int16_t *blk = nullptr;     // [fused bands][Ip] where the skipping logL pass put each band's logits of
@@ -244,9 +245,10 @@ hipError_t launch_slice_bf16(const emc_ctx *c, int s0, int cs, hipStream_t st);
 hipError_t launch_expand(const emc_ctx *c, int s0, int cs, float *out, hipStream_t st);
 
 // FP32 contractions (plain path).  With options.scaling the logits use iphi (launch_scaling_f32
-// first) and the M-step reads P/phi from iphi (launch_pscale_f32 after the responsibilities).
+// first) and the M-step reads P/phi from Pphi (the responsibilities pass writes it; launch_pscale_f32 after
+// emc_set_resp).  The dense M-step returns at once when gate is non-null and *gate <= gate_thr.
 hipError_t launch_logl_f32(const emc_ctx *c, int s0, int cs, hipStream_t st);
-hipError_t launch_mstep_f32(const emc_ctx *c, int s0, int cs, hipStream_t st);
+hipError_t launch_mstep_f32(const emc_ctx *c, int s0, int cs, const double *gate, double gate_thr, hipStream_t st);
 // 1/phi of rotations [s0, s0+cs) from the chunk's FP32 slices: sum K^2 and sum K W over
 // {W > 1e-10} as two contractions over pixels, then the quotient (1 where either sum is 0).
 hipError_t launch_scaling_f32(const emc_ctx *c, int s0, int cs, hipStream_t st);

@@ -24,6 +24,7 @@ __device__ __forceinline__ T wave_sum(T v)
     return v;
 }
 
+constexpr int kPartialRows = 8;
 __global__ __launch_bounds__(256) void k_sm_partial(const float *__restrict__ R, int64_t ldr, int S, int I,
                                                     int rows_per_band, float *__restrict__ pm,
                                                     double *__restrict__ ps)
@@ -35,14 +36,21 @@ __global__ __launch_bounds__(256) void k_sm_partial(const float *__restrict__ R,
     float m = -1.0e10f;
     double sum = 0.0;
     const float *col = R + i;
-    for (int s = r0; s < r1; ++s) {
-        const float v = col[(size_t)s * ldr];
-        if (v > m) {
-            sum = sum * (double)expf(m - v) + 1.0;
-            m = v;
-        } else {
-            const float d = v - m;
-            if (d > -1.0e10f) sum += (double)expf(d);
+    for (int s = r0; s < r1; s += kPartialRows) {  // the rows' loads in flight together, one rescale for them
+        float v[kPartialRows];
+#pragma unroll
+        for (int q = 0; q < kPartialRows; ++q) v[q] = col[(size_t)min(s + q, r1 - 1) * ldr];
+        float mx = m;
+#pragma unroll
+        for (int q = 0; q < kPartialRows; ++q) mx = fmaxf(mx, v[q]);
+        if (mx > m) {
+            sum *= (double)expf(m - mx);
+            m = mx;
+        }
+#pragma unroll
+        for (int q = 0; q < kPartialRows; ++q) {
+            const float d = v[q] - m;
+            if (d > -1.0e10f && s + q < r1) sum += (double)expf(d);
         }
     }
     pm[(size_t)band * I + i] = m;
@@ -128,7 +136,8 @@ __device__ __forceinline__ uint32_t pk_bf16(float a, float b)
 }
 constexpr int kApplyCols = 1024; // pattern columns per workgroup (4 per thread)
 
-// OUT = 0: P in place (FP32).  OUT = 1: BF16 hi/lo pair, of P * iphi when iphi is given (the
+// OUT = 0: P in place (FP32), and P * iphi to Pphi when iphi is given; pdirty says which 256-pattern segments
+// hold a non-zero.  OUT = 1: BF16 hi/lo pair, of P * iphi when iphi is given (the
 // M-step's P/phi under intensity scaling; the slice sums T stay sums of P).
 // OUT = 1 skips the store of a wave's 256-pattern row segment when every value in it is zero and
 // pdirty says the segment already holds only zeros (P is mostly zeros once the posteriors are
@@ -148,11 +157,12 @@ __global__ __launch_bounds__(256) void k_sm_apply(float *__restrict__ R, int64_t
                                                   bf16_t *__restrict__ Pl, double *__restrict__ Tpart,
                                                   double *__restrict__ nnz, const float *__restrict__ iphi,
                                                   uint8_t *__restrict__ pdirty, int nseg, const float *__restrict__ pm,
-                                                  const int16_t *__restrict__ blk, int chunk, int bpc, int brows)
+                                                  const int16_t *__restrict__ blk, int chunk, int bpc, int brows,
+                                                  float *__restrict__ Pphi)
 {
     static_assert(kApplyRows == 8, "8 rows: two per wave in the row sums, 8 floats per block read");
     constexpr float kLog2e = 1.4426950408889634f;
-    int nz = 0;  // OUT = 1: entries with a non-zero hi or lo term (for the choice of the M-step)
+    int nz = 0;  // entries of non-zero P (OUT = 1: hi or lo term; for the choice of the M-step)
     // per-thread row sums: each is a float (a float sum of the thread's four values, or one value),
     // kept as such and widened when the row sums are formed
     __shared__ float rs[kApplyRows][256];
@@ -351,6 +361,14 @@ __global__ __launch_bounds__(256) void k_sm_apply(float *__restrict__ R, int64_t
                 acc = (p[0] + p[1]) + (p[2] + p[3]);
                 if (OUT == 0) {
                     *reinterpret_cast<float4 *>(src) = make_float4(p[0], p[1], p[2], p[3]);
+                    if (iphi) {
+                        const size_t o = (size_t)s * ldr + c0;
+                        const float4 f = *reinterpret_cast<const float4 *>(iphi + o);
+                        *reinterpret_cast<float4 *>(Pphi + o) = make_float4(p[0] * f.x, p[1] * f.y, p[2] * f.z, p[3] * f.w);
+                    }
+                    const int mine = (p[0] != 0.0f) + (p[1] != 0.0f) + (p[2] != 0.0f) + (p[3] != 0.0f);
+                    nz += mine;
+                    any_nz = mine != 0;
                 } else {
                     const size_t o = (size_t)s * ldr + c0;
                     float q[4] = {p[0], p[1], p[2], p[3]};
@@ -373,6 +391,10 @@ __global__ __launch_bounds__(256) void k_sm_apply(float *__restrict__ R, int64_t
                     any_nz = mine != 0;
                 }
             }
+            if (OUT == 0 && s < S && seg_live) {
+                const bool seg_nz = __any(any_nz) != 0;
+                if (lane == 0) pdirty[(size_t)s * nseg + seg] = seg_nz ? 1 : 0;
+            }
             if (OUT == 1 && s < S && seg_live) {  // s and seg_live are uniform over the wave
                 const bool seg_nz = __any(any_nz) != 0;
                 const size_t fo = (size_t)s * nseg + seg;
@@ -390,10 +412,8 @@ __global__ __launch_bounds__(256) void k_sm_apply(float *__restrict__ R, int64_t
     // row sums over the workgroup's 1,024 patterns through LDS: wave w adds rows 2w and 2w + 1 (one
     // per 32-lane half, eight values a lane, then five shuffle steps), in a fixed order
     __shared__ int nzw[4];
-    if (OUT == 1) {
-        nz = wave_sum(nz);
-        if (lane == 0) nzw[wave] = nz;
-    }
+    nz = wave_sum(nz);
+    if (lane == 0) nzw[wave] = nz;
     __syncthreads();
     {
         const int row = 2 * wave + (lane >> 5), part = lane & 31;
@@ -428,7 +448,7 @@ __global__ __launch_bounds__(256) void k_sm_apply(float *__restrict__ R, int64_t
         }
     }
     // per-workgroup non-zero count, summed by one deterministic pass afterwards
-    if (OUT == 1 && threadIdx.x == 0)
+    if (threadIdx.x == 0)
         nnz[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = (double)(nzw[0] + nzw[1] + nzw[2] + nzw[3]);
 }
 
@@ -506,12 +526,13 @@ hipError_t launch_softmax(const emc_ctx *c, hipStream_t st)
         hipLaunchKernelGGL(k_sm_apply<1>, ga, dim3(256), 0, st, c->R, (int64_t)c->Ip, S, I, c->lse, c->Ph, c->Pl,
                            Tpart, nzpart, c->opt.scaling ? c->iphi : nullptr, c->pdirty, p_segments(c),
                            fused ? pm : nullptr, fused && c->logits_partial ? c->blk : nullptr, c->chunk,
-                           c->chunkp / logl_band_rows(c), logl_band_rows(c));
+                           c->chunkp / logl_band_rows(c), logl_band_rows(c), nullptr);
     else
         hipLaunchKernelGGL(k_sm_apply<0>, ga, dim3(256), 0, st, c->R, (int64_t)c->Ip, S, I, c->lse, nullptr, nullptr,
-                           Tpart, nullptr, nullptr, nullptr, 0, nullptr, nullptr, 1, 1, 1);
+                           Tpart, nzpart, c->opt.scaling ? c->iphi : nullptr, c->pdirty, p_segments(c), nullptr, nullptr, 1,
+                           1, 1, c->Pphi);
     hipLaunchKernelGGL(k_T_final, dim3((c->Sp + 255) / 256), dim3(256), 0, st, Tpart, ncb, S, c->Sp, c->T);
-    if (c->mfma) hipLaunchKernelGGL(k_sum_f64, dim3(1), dim3(1024), 0, st, nzpart, (int)(ga.x * ga.y), c->scal + SC_NNZ);
+    hipLaunchKernelGGL(k_sum_f64, dim3(1), dim3(1024), 0, st, nzpart, (int)(ga.x * ga.y), c->scal + SC_NNZ);
     return hipGetLastError();
 }
 

@@ -9,7 +9,9 @@
 // so the result is deterministic), in as many batches as the list needs, and each full list (and
 // the last) has its count rows added to registers, 16 pixels per thread and pass.  Counts as
 // bytes (KT 0), BF16 (KT 1) or BF16 hi + lo (KT 2); NPASS 16-pixel chunks per thread (Pp <=
-// 4096 * NPASS).  FP32 accumulation.
+// 4096 * NPASS).  FP32 accumulation, one fused multiply-add per entry and pixel, in ascending entry order: the
+// chain of the dense FP32 contraction without its zero entries.
+// KT 3 is the FP32 precision: the row is float (ph; pl unused) and so are the counts.
 #pragma once
 
 #include "../emc_internal.h"
@@ -19,8 +21,7 @@ namespace emc {
 namespace sparse_row_detail {
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kCap = 2048;        // LDS list entries per batch
-constexpr int kV = 4;             // 16-byte loads of hi per thread and step
-constexpr int kPer = 8 * kV;      // consecutive entries per thread and step
+constexpr int kPer = 32;          // consecutive entries per thread and step
 constexpr int kStep = 256 * kPer; // entries scanned per step
 static_assert(256 % kPer == 0, "a thread's entries lie in one 256-entry segment");
 
@@ -33,12 +34,24 @@ __device__ __forceinline__ bool nonzero(const u32x4 &v) { return (v[0] | v[1] | 
 // 16-byte aligned.  seg (or nullptr): one flag per 256 entries of the row, 0 where those entries are
 // known to be zero (their loads are skipped).
 template <int KT, int NPASS>
-__device__ __forceinline__ void sparse_row(const bf16_t *__restrict__ ph, const bf16_t *__restrict__ pl, int n,
+__device__ __forceinline__ void sparse_row(const void *__restrict__ ph, const bf16_t *__restrict__ pl, int n,
                                            const int32_t *__restrict__ pat, const void *__restrict__ Kv,
                                            const bf16_t *__restrict__ Klo, int Pp, float *__restrict__ out,
                                            const uint8_t *__restrict__ seg = nullptr)
 {
     using namespace sparse_row_detail;
+    constexpr int E = KT == 3 ? 4 : 8;  // entries per 16-byte load
+    constexpr int kV = kPer / E;        // loads per thread and step
+    auto load16 = [&](int i) {
+        return *reinterpret_cast<const u32x4 *>(reinterpret_cast<const unsigned char *>(ph) + (size_t)i * (16 / E));
+    };
+    // entry k of a load: its bits (0: not listed) and value
+    auto bits_of = [&](const u32x4 &h, const u32x4 &l, int k) -> uint32_t {
+        return KT == 3 ? h[k & 3] << 1 : ((h[(k >> 1) & 3] | l[(k >> 1) & 3]) >> (16 * (k & 1))) & 0xffffu;
+    };
+    auto value_of = [&](const u32x4 &h, const u32x4 &l, int k) {
+        return KT == 3 ? __uint_as_float(h[k & 3]) : half16(h, k & 7) + half16(l, k & 7);
+    };
     __shared__ int li[kCap];
     __shared__ float lp[kCap];
     __shared__ int wsum[4];
@@ -64,7 +77,18 @@ __device__ __forceinline__ void sparse_row(const bf16_t *__restrict__ ph, const 
                 if (KT == 0) {
                     const u32x4 v = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const uint8_t *>(Kv) + row);
 #pragma unroll
-                    for (int k = 0; k < 16; ++k) acc[q][k] += p * (float)((v[k >> 2] >> (8 * (k & 3))) & 0xffu);
+                    for (int k = 0; k < 16; ++k)
+                        acc[q][k] = __builtin_fmaf(p, (float)((v[k >> 2] >> (8 * (k & 3))) & 0xffu), acc[q][k]);
+                } else if (KT == 3) {
+                    const float4 *kr = reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(Kv) + row);
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) {
+                        const float4 v = kr[w];
+                        acc[q][4 * w] = __builtin_fmaf(p, v.x, acc[q][4 * w]);
+                        acc[q][4 * w + 1] = __builtin_fmaf(p, v.y, acc[q][4 * w + 1]);
+                        acc[q][4 * w + 2] = __builtin_fmaf(p, v.z, acc[q][4 * w + 2]);
+                        acc[q][4 * w + 3] = __builtin_fmaf(p, v.w, acc[q][4 * w + 3]);
+                    }
                 } else {
                     const bf16_t *kr = reinterpret_cast<const bf16_t *>(Kv) + row;
                     const u32x4 a = *reinterpret_cast<const u32x4 *>(kr), b = *reinterpret_cast<const u32x4 *>(kr + 8);
@@ -80,8 +104,8 @@ __device__ __forceinline__ void sparse_row(const bf16_t *__restrict__ ph, const 
                             k0 += half16(al, k);
                             k1 += half16(bl, k);
                         }
-                        acc[q][k] += p * k0;
-                        acc[q][8 + k] += p * k1;
+                        acc[q][k] = __builtin_fmaf(p, k0, acc[q][k]);
+                        acc[q][8 + k] = __builtin_fmaf(p, k1, acc[q][8 + k]);
                     }
                 }
             }
@@ -98,19 +122,16 @@ __device__ __forceinline__ void sparse_row(const bf16_t *__restrict__ ph, const 
         for (int v = 0; v < kV; ++v) {
             h[v] = u32x4{0u, 0u, 0u, 0u};
             l[v] = u32x4{0u, 0u, 0u, 0u};
-            if (live && ib + 8 * v < n) h[v] = *reinterpret_cast<const u32x4 *>(ph + ib + 8 * v);
+            if (live && ib + E * v < n) h[v] = load16(ib + E * v);
             any |= nonzero(h[v]);
         }
         if (!__syncthreads_or(any)) continue;
         int cnt = 0;
 #pragma unroll
         for (int v = 0; v < kV; ++v) {
-            if (nonzero(h[v])) l[v] = *reinterpret_cast<const u32x4 *>(pl + ib + 8 * v);
+            if (KT != 3 && nonzero(h[v])) l[v] = *reinterpret_cast<const u32x4 *>(pl + ib + E * v);
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const uint32_t bits = ((h[v][k >> 1] | l[v][k >> 1]) >> (16 * (k & 1))) & 0xffffu;
-                cnt += (bits != 0u && ib + 8 * v + k < n) ? 1 : 0;
-            }
+            for (int k = 0; k < E; ++k) cnt += (bits_of(h[v], l[v], k) != 0u && ib + E * v + k < n) ? 1 : 0;
         }
         int incl = cnt;  // inclusive scan over the wave
 #pragma unroll
@@ -131,18 +152,15 @@ __device__ __forceinline__ void sparse_row(const bf16_t *__restrict__ ph, const 
 #pragma unroll
             for (int v = 0; v < kV; ++v)
 #pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    const uint16_t hb = (uint16_t)(h[v][k >> 1] >> (16 * (k & 1)));
-                    const uint16_t lb = (uint16_t)(l[v][k >> 1] >> (16 * (k & 1)));
-                    if ((hb | lb) != 0 && ib + 8 * v + k < n) {
+                for (int k = 0; k < E; ++k)
+                    if (bits_of(h[v], l[v], k) != 0u && ib + E * v + k < n) {
                         const int q = rank - base;
                         if (q >= 0 && q < take) {
-                            li[m + q] = pat ? pat[ib + 8 * v + k] : ib + 8 * v + k;
-                            lp[m + q] = bf2f(hb) + bf2f(lb);
+                            li[m + q] = pat ? pat[ib + E * v + k] : ib + E * v + k;
+                            lp[m + q] = value_of(h[v], l[v], k);
                         }
                         ++rank;
                     }
-                }
             m += take;
             base += take;
             __syncthreads();

@@ -44,7 +44,7 @@ enum { EMC_DIFF_ABSOLUTE = 0, EMC_DIFF_POISSON = 1, EMC_DIFF_RELATIVE = 2, EMC_D
 enum { EMC_INTERP_NEAREST = 0, EMC_INTERP_TRILINEAR = 1 };
 
 /* Arithmetic of the two contractions (logL and the M-step sum).
- *   FP32   : direct FP32 (vector ALU), the plain path.
+ *   FP32   : FP32 operands, products and accumulation, the plain path.
  *   BF16X2 : MFMA, counts exact in BF16, log W and P each split into BF16 hi+lo, FP32 accumulate.
  *   BF16X3 : as BF16X2 with log W split into three BF16 terms (hi+mid+lo).
  * Counts above 256 and non-integer patterns are split into two BF16 terms on the MFMA modes.
@@ -60,7 +60,7 @@ enum { EMC_PREC_FP32 = 0, EMC_PREC_BF16X2 = 1, EMC_PREC_BF16X3 = 2 };
  *            accumulated per brick in LDS and flushed once (no contended global atomics). */
 enum { EMC_INSERT_ATOMIC = 0, EMC_INSERT_FUSED = 1, EMC_INSERT_BINNED = 2 };
 
-/* How the MFMA path forms U = P^T.K (emc_options.mstep).  SPARSE sums, per rotation, only the
+/* How the M-step forms U = P^T.K (emc_options.mstep).  SPARSE sums, per rotation, only the
  * patterns whose responsibility is non-zero (the same sums up to their order); AUTO uses it when
  * at most 2 % of the responsibilities are non-zero.  FUSED insertion always uses DENSE. */
 enum { EMC_MSTEP_AUTO = 0, EMC_MSTEP_DENSE = 1, EMC_MSTEP_SPARSE = 2 };
@@ -87,7 +87,7 @@ typedef struct emc_options {
     int32_t mfma_tile;       /* MFMA contraction tiling: 0 = 256-row tiles (default), 1 = 128x128 */
     int32_t count_bytes;     /* counts operand of the 256-row MFMA kernels: 0 = one byte per count when
                                 every count <= 255 (exact; widened to BF16 in registers), 2 = BF16 */
-    int32_t mstep;           /* MFMA M-step sum P^T.K: EMC_MSTEP_AUTO (default) chooses on the device,
+    int32_t mstep;           /* M-step sum P^T.K: EMC_MSTEP_AUTO (default) chooses on the device,
                                 from the E-step's count of non-zero responsibilities, between the
                                 dense contraction and the sparse one (only the non-zero P); or
                                 EMC_MSTEP_DENSE / EMC_MSTEP_SPARSE */
