@@ -201,16 +201,18 @@ struct emc_ctx {
     double *scal = nullptr;                            // [SC_N] device scalars
     double *scal_h = nullptr;                          // pinned host mirror
     // binned insertion: valid (s, j) pairs sorted by (chunk, model brick), cut into units of at most
-    // 4,096 pairs; per unit a base-voxel permutation; partial halo bricks per block (<= 4 units of a
-    // brick, one workgroup) and per group of blocks
+    // bin_unit pairs; per unit a base-voxel permutation; partial halo bricks per block (consecutive units of a
+    // brick, one workgroup) and, unless bin_direct, per group of blocks
+    int bin_unit = 0;
+    bool bin_direct = false;                           // every brick has few blocks: the last pass adds them itself
     uint32_t *bin_vals = nullptr;                      // [S * Pa] packed s << jbits | j, (s, j) order per brick
     uint16_t *bin_perm = nullptr;                      // [S * Pa] each pair's position in base-voxel order in its unit
     uint16_t *bin_vbeg = nullptr;                      // [n_units][520] start of each base voxel's run
-    float *bin_frac = nullptr;                         // [n_units][3][4096] trilinear fractions (base-voxel order)
+    float *bin_frac = nullptr;                         // [n_units][3][bin_unit] trilinear fractions (base-voxel order)
     int32_t *bin_units = nullptr;                      // [n_units][4] = key, begin, end, 0
     int32_t *bin_blocks = nullptr;                     // [n_blocks][4] = key, first unit, end unit, 0 (one workgroup)
     int32_t *bin_groups = nullptr;                     // [n_groups][4] = key, first block, end block (per chunk), 0
-    int32_t *bin_gbeg = nullptr;                       // [chunks][bricks + 1] first group of each brick
+    int32_t *bin_gbeg = nullptr;                       // [chunks][bricks + 1] first group (bin_direct: block) of each brick
     float *bin_part = nullptr;                         // [blocks of a chunk][2][9^3] block partials
     float *bin_gpart = nullptr;                        // [groups of a chunk][2][9^3] group partials
     std::vector<int> bin_chunk_blocks, bin_chunk_groups; // block / group range of each rotation chunk

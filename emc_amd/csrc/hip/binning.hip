@@ -5,7 +5,7 @@
 // iteration.  Once per geometry the valid (rotation s, active pixel j) pairs are sorted by the
 // model brick (kBrick^3 voxels) that holds their base voxel, per rotation chunk, with a stable
 // radix sort (rocPRIM), so each brick lists its pairs in (s, j) order; each brick's list is cut
-// into units of at most kUnit pairs, and inside a unit the pairs are ranked once more by base
+// into units of at most c->bin_unit pairs, and inside a unit the pairs are ranked once more by base
 // voxel (a 16-bit permutation, the start of each base voxel's run, and for trilinear the pairs'
 // fractions in base-voxel order, laid out for coalesced reads).  Per pair the iteration then reads
 // 4 bytes of list (the packed pair), 2 of permutation and 12 of fractions.  Every iteration:
@@ -13,12 +13,12 @@
 //      consecutive pixels, and writes U and T_s into LDS at the pair's position in base-voxel order;
 //   2. every thread sums an equal share of the positions into per-base-voxel corner sums (the
 //      pieces of a voxel's run that crosses threads are added in thread order);
-//   3. a workgroup runs steps 1-2 for up to kUnitsPerBlock units of one brick in turn, then every
+//   3. a workgroup runs steps 1-2 for a few units of one brick in turn, then every
 //      voxel of the halo brick ((kBrick+1)^3) gathers the corner sums in a fixed order, and the
 //      halo brick is stored as the block's partial (no atomics);
-//   4. a grouping pass sums the partials of up to kGroup consecutive blocks of one brick, and a
-//      last pass gives every model voxel the sum, in order, of the groups of the (at most 8)
-//      bricks whose halo covers it.
+//   4. a grouping pass sums the partials of up to kGroup consecutive blocks of one brick (left out where no brick
+//      has more than kDirect), and a last pass gives every model voxel the sum, in order, of the groups
+//      of the (at most 8) bricks whose halo covers it.
 // No sum depends on scheduling, so repeated runs give bit-identical models.  This replaces the 16
 // global atomics per (s, j) of the reference's insert_slices_kernel (emc_atomic.cu:33-85,
 // 183-200); the skip rules (T_s > 1e-10, emc_atomic.cu:190; U >= 0, emc_atomic.cu:56) and the
@@ -38,15 +38,13 @@ namespace {
 
 constexpr int kBrick = 8;
 constexpr int kBrick3 = kBrick * kBrick * kBrick;  // base voxels of a brick
-constexpr int kUnit = 4096;                        // pairs per workgroup (positions fit 16 bits)
 constexpr int kVbeg = 520;                         // run starts per unit: kBrick3 + 1, padded to 16 bytes
-constexpr int kUnitsPerBlock = 4;                  // units one insertion workgroup processes in turn
 constexpr int kGroup = 32;                         // blocks whose partials one grouping workgroup sums
+constexpr int kDirect = 8;                         // up to this many blocks per brick: no grouping pass (a launch;
+                                                   // at 12 the last pass takes longer by as much)
 constexpr int kHalo = kBrick + 1;
 constexpr int kHalo3 = kHalo * kHalo * kHalo;      // voxels a brick's pairs reach
-constexpr int kStage = 8;                          // pairs per thread whose loads are issued together
-constexpr int kThreads = 512;  // 8 waves; with 67 KB of LDS two workgroups (16 waves) fit a CU
-static_assert(kUnit % kThreads == 0, "step 2 gives every thread the same share");
+constexpr int kThreads = 512;  // 8 waves; with 67 KB of LDS and 128 registers two workgroups (16 waves) fit a CU
 
 struct BinGeom {
     int L, nb, S, Pa, Pp, chunk, interp, jbits;
@@ -135,19 +133,17 @@ __global__ __launch_bounds__(kThreads) void k_unit_keys(const int32_t *__restric
 // Per unit: each pair's position in base-voxel order (a stable order, so (s, j) order within a base
 // voxel), stored at the pair's place in (s, j) order; the start of each base voxel's run
 // (kBrick3 + 1 entries); for trilinear, the fractions of the pair at base-voxel position k, stored
-// at frac[(u * 3 + axis) * kUnit + (k % kPer) * kThreads + k / kPer], where the insertion's thread
-// k / kPer reads them in step (k % kPer) of its share, all lanes of a wave on consecutive words.
+// at frac[(u * 3 + axis) * unit + (k % per) * kThreads + k / per], where the insertion's thread
+// k / per reads them in step (k % per) of its share, all lanes of a wave on consecutive words.
 __global__ __launch_bounds__(kThreads) void k_unit_perm(const int32_t *__restrict__ units,
                                                         const uint32_t *__restrict__ skeys,
                                                         const uint32_t *__restrict__ spos,
                                                         const uint32_t *__restrict__ vals,
-                                                        const float *__restrict__ rotm,
-                                                        const float *__restrict__ axyz, BinGeom g,
-                                                        uint16_t *__restrict__ inv, uint16_t *__restrict__ vbeg,
-                                                        float *__restrict__ frac)
+                                                        const float *__restrict__ rotm, const float *__restrict__ axyz,
+                                                        BinGeom g, int per, uint16_t *__restrict__ inv,
+                                                        uint16_t *__restrict__ vbeg, float *__restrict__ frac)
 {
-    constexpr int kPer = kUnit / kThreads;
-    const int u = blockIdx.x;
+    const int u = blockIdx.x, unit = per * kThreads;
     const int begin = units[4 * u + 1], end = units[4 * u + 2];
     for (int t = begin + threadIdx.x; t < end; t += kThreads) {
         const int k = t - begin;
@@ -157,8 +153,7 @@ __global__ __launch_bounds__(kThreads) void k_unit_perm(const int32_t *__restric
             float f[3];
             unpack(vals[spos[t]], g.jbits, s, j);
             item_cell(rotm, axyz, g, s, j, bx, by, bz, f[0], f[1], f[2]);
-            for (int a = 0; a < 3; ++a)
-                frac[((size_t)u * 3 + a) * kUnit + (k % kPer) * kThreads + k / kPer] = f[a];
+            for (int a = 0; a < 3; ++a) frac[((size_t)u * 3 + a) * unit + (k % per) * kThreads + k / per] = f[a];
         }
     }
     for (int lv = threadIdx.x; lv <= kBrick3; lv += kThreads) {
@@ -173,24 +168,32 @@ __global__ __launch_bounds__(kThreads) void k_unit_perm(const int32_t *__restric
     }
 }
 
-// Steps 1-3 for one block: up to kUnitsPerBlock consecutive units of one brick, one after the other,
-// whose corner sums accumulate in LDS; the block's halo brick is stored as its partial
+// Steps 1-3 for one block: consecutive units of one brick, one after the other, whose corner sums accumulate in
+// LDS; the block's halo brick is stored as its partial
 // (part: [block - first block of the chunk][2][kHalo3], numerator then weight).
-// Step 1 reads a unit's pairs in (s, j) order (coalesced: runs of pixels of one rotation) and
-// writes U (or -1: skipped) and T_s into LDS at the pair's position in base-voxel order.  Step 2
-// gives every thread the same share of the unit, kPer consecutive positions, with the trilinear
+// Step 1 writes U (or -1: skipped) and T_s into LDS at the pair's position in base-voxel order.  Step 2
+// gives every thread the same share of the unit, KPER consecutive positions, with the trilinear
 // fractions read from the precomputed coalesced planes (a thread per base voxel would wait on the
 // brick's heaviest voxel: at 64^3 / 25,680 the slowest thread of a unit would sum 2.5 times the
 // mean, up to 32 times).  A base voxel's run that crosses a thread boundary is summed piecewise: a
 // piece that continues into the next thread is handed over as a tail, and the thread holding the
 // run's last position adds the pieces in thread order.  Corner c = dx + 2 dy + 4 dz, weights
-// (1-f or f) per axis.  LDS layouts avoid bank conflicts: position k sits at k ^ ((k >> 3) & 7) (a
-// thread's kPer = 8 positions are consecutive, so the 64 lanes of a read fall on 64 banks), the
+// (1-f or f) per axis.  LDS layouts avoid bank conflicts: position k sits at k ^ ((k >> 6) % KPER) (a
+// thread's KPER positions are consecutive, so the 64 lanes of a read fall on 64 banks), the
 // corner sums are corner-major, the tails value-major.
-__device__ __forceinline__ int rswz(int k) { return k ^ ((k >> 3) & 7); }
+//
+// What bounds it: memory, 22 bytes a pair with U, and the latency of list -> U, which the list read one unit ahead
+// halves.  64^3 / 25,680: 820 -> 607 us with that and the swizzle above (k ^ ((k >> 3) & 7) before, which left eight
+// lanes on each bank), 3.0 TB/s.  Forming the fractions here instead of reading them: 985 us (the vector units,
+// then); U, T and the fractions one unit ahead too: 17 to 31 registers spilled, 856 us.
+template <int KPER>
+__device__ __forceinline__ int rswz(int k)
+{
+    return k ^ ((k >> 6) & (KPER - 1));
+}
 
-template <int INTERP>
-__global__ __launch_bounds__(kThreads, 2) void k_insert_binned(const int32_t *__restrict__ blocks,
+template <int INTERP, int KPER>
+__global__ __launch_bounds__(kThreads, 4) void k_insert_binned(const int32_t *__restrict__ blocks,
                                                                const int32_t *__restrict__ units,
                                                                const uint32_t *__restrict__ vals,
                                                                const uint16_t *__restrict__ inv,
@@ -201,66 +204,72 @@ __global__ __launch_bounds__(kThreads, 2) void k_insert_binned(const int32_t *__
                                                                float *__restrict__ part)
 {
     constexpr int NC = INTERP == EMC_INTERP_NEAREST ? 1 : 8;
-    constexpr int kPer = kUnit / kThreads;  // positions per thread in step 2
-    static_assert(kPer == 8, "the position swizzle assumes 8 consecutive positions per thread");
-    static_assert(2 * kUnit >= kThreads * 2 * NC, "the tails reuse the staging space");
-    __shared__ float sv[2][kUnit];  // U (-1: skipped) and T_s by base-voxel position
+    constexpr int kUnit = kThreads * KPER;
+    constexpr int kBuf = 2 * kUnit > 2 * NC * kThreads ? 2 * kUnit : 2 * NC * kThreads;
+    __shared__ float buf[kBuf];  // a unit's U (-1: skipped) and T_s by base-voxel position, then the tails
     __shared__ uint16_t svb[kBrick3 + 1];
-    __shared__ float cM[NC][kBrick3], cW[NC][kBrick3];
+    __shared__ __attribute__((aligned(16))) float cM[NC][kBrick3], cW[NC][kBrick3];
     __shared__ int tail_lv[kThreads];
-    float(*tail)[kThreads] = reinterpret_cast<float(*)[kThreads]>(&sv[0][0]);  // [2 NC][kThreads]
+    float(*sv)[kUnit] = reinterpret_cast<float(*)[kUnit]>(buf);
+    float(*tail)[kThreads] = reinterpret_cast<float(*)[kThreads]>(buf);  // [2 NC][kThreads]
     const int b = blockIdx.x;
     const int ub = blocks[4 * b + 1], ue = blocks[4 * b + 2];
     const int tid = threadIdx.x;
-    for (int k = tid; k < NC * kBrick3; k += kThreads) {
-        (&cM[0][0])[k] = 0.0f;
-        (&cW[0][0])[k] = 0.0f;
+    for (int k = tid; k < NC * kBrick3 / 4; k += kThreads) {
+        reinterpret_cast<float4 *>(&cM[0][0])[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        reinterpret_cast<float4 *>(&cW[0][0])[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
+    // the pairs of a unit, read one unit ahead (past the end of a unit: a valid pair, not stored)
+    uint32_t pv[KPER];
+    uint16_t pos[KPER];
+    int begin = units[4 * ub + 1], n = units[4 * ub + 2] - begin;
+    auto load_pairs = [&] {
+#pragma unroll
+        for (int q = 0; q < KPER; ++q) {
+            const int k = begin + min(tid + q * kThreads, n - 1);
+            pv[q] = vals[k];
+            pos[q] = inv[k];
+        }
+    };
+    load_pairs();
     for (int u = ub; u < ue; ++u) {
-        const int begin = units[4 * u + 1], end = units[4 * u + 2];
-        const int n = end - begin;
-        // this thread's fractions (issued before the barrier: they do not depend on LDS)
-        const int k0 = tid * kPer, k1 = min(n, k0 + kPer);
-        float fr[kPer][3];
+        const int k0 = tid * KPER, k1 = min(n, k0 + KPER);
+        // 1. U and T_s by base-voxel position, from the pairs in (s, j) order
+        double Td[KPER];
+        float val[KPER];
+#pragma unroll
+        for (int q = 0; q < KPER; ++q) {
+            int s, j;
+            unpack(pv[q], g.jbits, s, j);
+            Td[q] = T[s];
+            val[q] = U[(size_t)(s - s0) * g.Pp + j];
+        }
+        // this thread's fractions (used after the barriers)
+        float fr[KPER][3];
         if constexpr (INTERP == EMC_INTERP_TRILINEAR) {
 #pragma unroll
-            for (int i = 0; i < kPer; ++i)
+            for (int i = 0; i < KPER; ++i)
 #pragma unroll
                 for (int a = 0; a < 3; ++a) fr[i][a] = frac[((size_t)u * 3 + a) * kUnit + i * kThreads + tid];
         }
         __syncthreads();  // the previous unit's tails and run starts are consumed
         for (int k = tid; k <= kBrick3; k += kThreads) svb[k] = vbeg[(size_t)u * kVbeg + k];
-        // 1. U and T_s by base-voxel position, from the pairs in (s, j) order
-        for (int q0 = tid; q0 < n; q0 += kThreads * kStage) {
-            uint32_t pv[kStage];
-            uint16_t pos[kStage];
 #pragma unroll
-            for (int q = 0; q < kStage; ++q) {
-                const int k = begin + min(q0 + q * kThreads, n - 1);  // past the end: a valid pair, not stored
-                pv[q] = vals[k];
-                pos[q] = inv[k];
-            }
-            double Td[kStage];
-            float val[kStage];
-#pragma unroll
-            for (int q = 0; q < kStage; ++q) {
-                int s, j;
-                unpack(pv[q], g.jbits, s, j);
-                Td[q] = T[s];
-                val[q] = U[(size_t)(s - s0) * g.Pp + j];
-            }
-#pragma unroll
-            for (int q = 0; q < kStage; ++q) {
-                if (q0 + q * kThreads >= n) break;
-                const int p = rswz(pos[q]);
-                sv[0][p] = (Td[q] > 1e-10 && val[q] >= 0.0f) ? val[q] : -1.0f;  // emc_atomic.cu:190, :56
-                sv[1][p] = (float)Td[q];
-            }
+        for (int q = 0; q < KPER; ++q) {
+            if (tid + q * kThreads >= n) break;
+            const int p = rswz<KPER>(pos[q]);
+            sv[0][p] = (Td[q] > 1e-10 && val[q] >= 0.0f) ? val[q] : -1.0f;  // emc_atomic.cu:190, :56
+            sv[1][p] = (float)Td[q];
+        }
+        if (u + 1 < ue) {  // the next unit's pairs
+            begin = units[4 * (u + 1) + 1];
+            n = units[4 * (u + 1) + 2] - begin;
+            load_pairs();
         }
         __syncthreads();
         // 2. positions [k0, k1); lv = the base voxel of the current run
         int lv = 0;
-        if (k0 < n) {  // the voxel whose run holds k0: the last lv with svb[lv] <= k0
+        if (k0 < k1) {  // the voxel whose run holds k0: the last lv with svb[lv] <= k0
             int lo = 0, hi = kBrick3 - 1;
             while (lo < hi) {
                 const int mid = (lo + hi + 1) >> 1;
@@ -294,14 +303,14 @@ __global__ __launch_bounds__(kThreads, 2) void k_insert_binned(const int32_t *__
             for (int c = 0; c < 2 * NC; ++c) acc[c] = 0.0f;
         };
 #pragma unroll
-        for (int i = 0; i < kPer; ++i) {
+        for (int i = 0; i < KPER; ++i) {
             const int k = k0 + i;
             if (k >= k1) break;
             if (k >= svb[lv + 1]) {
                 close_run(k);
                 while (svb[lv + 1] <= k) ++lv;  // skip base voxels without pairs
             }
-            const int p = rswz(k);
+            const int p = rswz<KPER>(k);
             const float v = sv[0][p];
             if (v < 0.0f) continue;
             const float Ts = sv[1][p];
@@ -387,7 +396,8 @@ __global__ __launch_bounds__(kThreads) void k_bin_group(const int32_t *__restric
 
 // Step 4b: every voxel adds the groups of the bricks whose halo covers it: its own brick and, on
 // a brick's low face, the neighbour below on that axis (whose halo index there is kBrick); in a
-// fixed order.  gbeg: [key - key0] first group of each brick of the chunk (kBricks + 1 entries).
+// fixed order.  gbeg: [key - key0] first group of each brick of the chunk (kBricks + 1 entries);
+// without a grouping pass, blocks and their partials take the place of the groups.
 __global__ __launch_bounds__(kThreads) void k_insert_reduce(const float *__restrict__ gpart,
                                                             const int32_t *__restrict__ gbeg, BinGeom g,
                                                             float *__restrict__ Mnum, float *__restrict__ Wt,
@@ -406,7 +416,22 @@ __global__ __launch_bounds__(kThreads) void k_insert_reduce(const float *__restr
             for (int dx = 0; dx < nx; ++dx) {
                 const int key = ((bz - dz) * g.nb + (by - dy)) * g.nb + (bx - dx);
                 const int hv = ((dz ? kBrick : lz) * kHalo + (dy ? kBrick : ly)) * kHalo + (dx ? kBrick : lx);
-                for (int gi = gbeg[key]; gi < gbeg[key + 1]; ++gi) {
+                const int g1 = gbeg[key + 1];
+                int gi = gbeg[key];
+                for (; gi + 4 <= g1; gi += 4) {  // independent loads, added in order
+                    float a[4], w[4];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        a[q] = gpart[(size_t)(gi + q) * 2 * kHalo3 + hv];
+                        w[q] = gpart[(size_t)(gi + q) * 2 * kHalo3 + kHalo3 + hv];
+                    }
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        sm += a[q];
+                        sw += w[q];
+                    }
+                }
+                for (; gi < g1; ++gi) {
                     sm += gpart[(size_t)gi * 2 * kHalo3 + hv];
                     sw += gpart[(size_t)gi * 2 * kHalo3 + kHalo3 + hv];
                 }
@@ -452,6 +477,17 @@ hipError_t build_bins(emc_ctx *c, std::string &err)
     const int nch = (c->S + c->chunk - 1) / c->chunk;
     const uint32_t nbr = (uint32_t)g.nb * g.nb * g.nb;
     const uint32_t nkeys = (uint32_t)nch * nbr;
+    // Unit size and units per workgroup, from the pairs of a chunk (longer workgroups write fewer partial halo
+    // bricks of 5.8 KB, shorter ones fill the chip's 512 workgroup slots).  Insertion and its two reductions, us,
+    // at 2,048 x 1 / 4,096 x 2 / 4,096 x 4 pairs a workgroup: 0.17M pairs (24^3 / 420 rotations) 27 / 36 / 44,
+    // 1.5M (45^3 nearest, 1,000) 30 / 38 / 41, 2.4M (32^3 / 3,240) 56 / 51 / 69, 20M (64^3 / 6,300) 241 / 185 / 190,
+    // 82M (64^3 / 25,680) 953 / 648 / 633 and (128^3 / 6,300) 913 / 668 / 662.
+    const int64_t pairs = (int64_t)std::min(c->chunk, c->S) * c->Pa;
+    // (the unit keys have 32 bits: with very many bricks over all chunks the fewest units)
+    const bool small = pairs < (2 << 20) && nkeys < (1u << 22);
+    const int kUnit = c->bin_unit = small ? 2048 : 4096;
+    const int kUnitsPerBlock = small ? 1 : pairs < (32 << 20) ? 2 : 4;
+    int max_brick_blocks = 0;
     int end_bit = 1;
     while (end_bit < 32 && ((uint64_t)1 << end_bit) <= nkeys) ++end_bit;
     uint32_t *kin = nullptr, *vin = nullptr, *kout = nullptr, *pout = nullptr;
@@ -504,7 +540,7 @@ hipError_t build_bins(emc_ctx *c, std::string &err)
     // workgroup each, numbered per chunk (unit indices global); groups (key, first block, end
     // block, 0): at most kGroup consecutive blocks of one brick, numbered per chunk, with each
     // brick's first group in gbeg
-    std::vector<int32_t> units, blocks, groups, gbeg;
+    std::vector<int32_t> units, blocks, groups, gbeg, bbeg;  // bbeg: each brick's first block
     c->bin_chunk_blocks.assign(nch + 1, 0);
     c->bin_chunk_groups.assign(nch + 1, 0);
     int max_blocks = 0, max_groups = 0;
@@ -530,6 +566,8 @@ hipError_t build_bins(emc_ctx *c, std::string &err)
                 blocks.push_back(0);
             }
             const int be = (int)(blocks.size() / 4) - b_first;
+            max_brick_blocks = std::max(max_brick_blocks, be - bb);
+            bbeg.push_back(bb);
             for (int bl = bb; bl < be; bl += kGroup) {
                 groups.push_back((int32_t)k);
                 groups.push_back(bl);
@@ -538,19 +576,22 @@ hipError_t build_bins(emc_ctx *c, std::string &err)
             }
         }
         gbeg.push_back((int32_t)(groups.size() / 4) - g_first);
+        bbeg.push_back((int32_t)(blocks.size() / 4) - b_first);
         c->bin_chunk_blocks[ch + 1] = (int)(blocks.size() / 4);
         c->bin_chunk_groups[ch + 1] = (int)(groups.size() / 4);
         max_blocks = std::max(max_blocks, c->bin_chunk_blocks[ch + 1] - c->bin_chunk_blocks[ch]);
         max_groups = std::max(max_groups, c->bin_chunk_groups[ch + 1] - c->bin_chunk_groups[ch]);
     }
     const uint32_t n_units = (uint32_t)(units.size() / 4);
+    c->bin_direct = max_brick_blocks <= kDirect;
+    if (c->bin_direct) gbeg = bbeg;
     if (e == hipSuccess && n_units > 0) {
         chk(hipMalloc((void **)&c->bin_units, sizeof(int32_t) * units.size()));
         chk(hipMalloc((void **)&c->bin_blocks, sizeof(int32_t) * blocks.size()));
         chk(hipMalloc((void **)&c->bin_groups, sizeof(int32_t) * groups.size()));
         chk(hipMalloc((void **)&c->bin_gbeg, sizeof(int32_t) * gbeg.size()));
         chk(hipMalloc((void **)&c->bin_part, sizeof(float) * 2 * kHalo3 * (size_t)max_blocks));
-        chk(hipMalloc((void **)&c->bin_gpart, sizeof(float) * 2 * kHalo3 * (size_t)max_groups));
+        if (!c->bin_direct) chk(hipMalloc((void **)&c->bin_gpart, sizeof(float) * 2 * kHalo3 * (size_t)max_groups));
         chk(hipMalloc((void **)&c->bin_perm, sizeof(uint16_t) * n));
         chk(hipMalloc((void **)&c->bin_vbeg, sizeof(uint16_t) * kVbeg * (size_t)n_units));
         if (c->opt.interp == EMC_INTERP_TRILINEAR)
@@ -593,7 +634,7 @@ hipError_t build_bins(emc_ctx *c, std::string &err)
             chk(rocprim::radix_sort_pairs(tmp, tmp_bytes, kin, kout, vin, pout, (size_t)n, 0, end_bit2, st));
         if (e == hipSuccess) {
             hipLaunchKernelGGL(k_unit_perm, dim3(n_units), dim3(kThreads), 0, st, c->bin_units, kout, pout, c->bin_vals,
-                               c->rotm, c->axyz, g, c->bin_perm, c->bin_vbeg, c->bin_frac);
+                               c->rotm, c->axyz, g, kUnit / kThreads, c->bin_perm, c->bin_vbeg, c->bin_frac);
             chk(hipGetLastError());
         }
         if (e == hipSuccess) chk(hipStreamSynchronize(st));
@@ -623,18 +664,22 @@ hipError_t launch_insert_binned(const emc_ctx *c, int s0, int cs, hipStream_t st
     }
     const BinGeom g = geom_of(c);
     const int32_t *blocks = c->bin_blocks + 4 * (size_t)b0;
+    const auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(b1 - b0), dim3(kThreads), 0, st, blocks, c->bin_units, c->bin_vals, c->bin_perm,
+                           c->bin_vbeg, c->bin_frac, c->U, s0, c->T, g, c->bin_part);
+    };
+    const bool small = c->bin_unit == 2048;
     if (c->opt.interp == EMC_INTERP_NEAREST)
-        hipLaunchKernelGGL(k_insert_binned<EMC_INTERP_NEAREST>, dim3(b1 - b0), dim3(kThreads), 0, st, blocks,
-                           c->bin_units, c->bin_vals, c->bin_perm, c->bin_vbeg, nullptr, c->U, s0, c->T, g, c->bin_part);
+        run(small ? k_insert_binned<EMC_INTERP_NEAREST, 4> : k_insert_binned<EMC_INTERP_NEAREST, 8>);
     else
-        hipLaunchKernelGGL(k_insert_binned<EMC_INTERP_TRILINEAR>, dim3(b1 - b0), dim3(kThreads), 0, st, blocks,
-                           c->bin_units, c->bin_vals, c->bin_perm, c->bin_vbeg, c->bin_frac, c->U, s0, c->T, g,
-                           c->bin_part);
-    hipLaunchKernelGGL(k_bin_group, dim3(g1 - g0), dim3(kThreads), 0, st, c->bin_groups + 4 * (size_t)g0, c->bin_part,
-                       c->bin_gpart);
+        run(small ? k_insert_binned<EMC_INTERP_TRILINEAR, 4> : k_insert_binned<EMC_INTERP_TRILINEAR, 8>);
+    if (!c->bin_direct)
+        hipLaunchKernelGGL(k_bin_group, dim3(g1 - g0), dim3(kThreads), 0, st, c->bin_groups + 4 * (size_t)g0, c->bin_part,
+                           c->bin_gpart);
     const int nbr = g.nb * g.nb * g.nb;
     hipLaunchKernelGGL(k_insert_reduce, dim3((unsigned)((c->N3 + kThreads - 1) / kThreads)), dim3(kThreads), 0, st,
-                       c->bin_gpart, c->bin_gbeg + (size_t)k * (nbr + 1), g, c->Mnum, c->Wt, k == 0);
+                       c->bin_direct ? c->bin_part : c->bin_gpart, c->bin_gbeg + (size_t)k * (nbr + 1), g, c->Mnum,
+                       c->Wt, k == 0);
     return hipGetLastError();
 }
 
