@@ -197,7 +197,7 @@ extern "C" void emc_destroy(emc_ctx *c)
     dfree(c->K32); dfree(c->KT32); dfree(c->K16); dfree(c->K16lo); dfree(c->KT16); dfree(c->KT16lo); dfree(c->sumK);
     dfree(c->K8); dfree(c->KT8);
     dfree(c->model); dfree(c->Mnum); dfree(c->Wt); dfree(c->tmp3); dfree(c->modelq); dfree(c->taps);
-    dfree(c->sumW); dfree(c->ns); dfree(c->colsum); dfree(c->colp); dfree(c->colpart); dfree(c->colmean); dfree(c->bias); dfree(c->rscale); dfree(c->cst);
+    dfree(c->sumW); dfree(c->ns); dfree(c->colp); dfree(c->colpart); dfree(c->colmean); dfree(c->bias); dfree(c->rscale); dfree(c->cst);
     dfree(c->A0); dfree(c->A1); dfree(c->Am); dfree(c->AWm); dfree(c->K2); dfree(c->iphi); dfree(c->Pphi); dfree(c->Lh); dfree(c->Lm); dfree(c->Ll); dfree(c->lw32);
     dfree(c->Cx); dfree(c->K2h); dfree(c->K2l); dfree(c->Aw); dfree(c->G2); dfree(c->G3); dfree(c->G4);
     dfree(c->R); dfree(c->Ph); dfree(c->Pl); dfree(c->pdirty); dfree(c->runmax); dfree(c->blk); dfree(c->lse); dfree(c->part); dfree(c->red); dfree(c->T); dfree(c->U); dfree(c->scal);
@@ -282,14 +282,11 @@ extern "C" emc_status emc_create(const emc_dims *d, const emc_options *o, emc_ct
         if (st == EMC_OK) A(dalloc(&c->Pl, Sp * Ip), "Pl");
         if (st == EMC_OK) A(dalloc(&c->runmax, Ip), "runmax");
         if (st == EMC_OK) A(dalloc(&c->blk, (int64_t)softmax_fused_bands_max(c) * Ip), "blk");
-        if (st == EMC_OK) A(dalloc(&c->colsum, 2 * (int64_t)PpMax), "colsum");
         if (st == EMC_OK) A(dalloc(&c->colp, colp_len(c->S, PpMax)), "colp");
         if (st == EMC_OK) A(dalloc(&c->colpart, colpart_len(PpMax)), "colpart");
         if (st == EMC_OK) A(dalloc(&c->lw32, Sp * PpMax), "lw32");
         if (c->chi2_mfma) {
             const int64_t nops = (opt.scaling ? 4 : 2) * (int64_t)c->la_terms;
-            if (st == EMC_OK) A(dalloc(&c->A0, cp * PpMax), "A0");
-            if (st == EMC_OK) A(dalloc(&c->A1, cp * PpMax), "A1");
             if (st == EMC_OK) A(dalloc(&c->Cx, nops * cp * PpMax), "Cx");
             if (st == EMC_OK) A(dalloc(&c->K2h, Ip * PpMax), "K2h");
             if (st == EMC_OK) A(dalloc(&c->K2l, Ip * PpMax), "K2l");
@@ -700,9 +697,8 @@ static emc_status slice_prepare(emc_ctx *c, float sigma)
 {
     hipStream_t st = c->stream;
     ev_start(c, EMC_STAGE_SLICE);
-    HIP_TRY(c, launch_slice_stats(c, c->mfma, st));
+    HIP_TRY(c, launch_slice_stats(c, st));
     HIP_TRY(c, launch_bias(c, sigma, st));
-    HIP_TRY(c, launch_pattern_const(c, c->mfma && !c->chi2_mfma, st));
     ev_stop(c, EMC_STAGE_SLICE);
     return EMC_OK;
 }
@@ -716,7 +712,6 @@ static emc_status logl_enqueue(emc_ctx *c, float sigma)
         const int cs = std::min(c->chunk, c->S - s0);
         const int k = s0 / c->chunk;
         if (c->chi2_mfma) {
-            HIP_TRY(c, launch_slice_f32(c, s0, cs, st));
             gev_rec(c, 0, k, 0);
             HIP_TRY(c, launch_logl_chi2_mfma(c, s0, cs, st));
             gev_rec(c, 0, k, 1);
@@ -744,7 +739,6 @@ extern "C" emc_status emc_logl(emc_ctx *c, float sigma)
         return fail(c, EMC_E_STATE, "logl: needs rotations, coords, mask, patterns and model");
     if (c->opt.diff != EMC_DIFF_TRUE_POISSON && !(sigma > 0.0f)) return fail(c, EMC_E_INVALID, "logl: sigma must be > 0");
     HIP_TRY(c, hipSetDevice(c->opt.device));
-    HIP_TRY(c, launch_fill_f64(c->scal + SC_NONFINITE, 0.0, 1, c->stream));
     c->skip_logits = c->logits_partial = false;  // the caller may read every logit
     EMC_TRY(logl_enqueue(c, sigma));
     HIP_TRY(c, hipStreamSynchronize(c->stream));
@@ -762,17 +756,6 @@ static emc_status softmax_enqueue(emc_ctx *c)
     return EMC_OK;
 }
 
-static emc_status total_logl_host(emc_ctx *c, double *total)
-{
-    // sum_i lse_i = sum_i lse'_i + sum_i cst_i (FP64)
-    std::vector<double> cst(c->I);
-    HIP_TRY(c, hipMemcpy(cst.data(), c->cst, sizeof(double) * c->I, hipMemcpyDeviceToHost));
-    double t = c->scal_h[SC_TOTAL];
-    for (double v : cst) t += v;
-    *total = t;
-    return EMC_OK;
-}
-
 extern "C" emc_status emc_normalize_resp(emc_ctx *c, double *total_logl)
 {
     if (!c) return fail(c, EMC_E_INVALID, "normalize_resp: null context");
@@ -783,7 +766,7 @@ extern "C" emc_status emc_normalize_resp(emc_ctx *c, double *total_logl)
     c->has_resp = c->has_lse = true;
     if (!c->mfma) c->has_logl = false;  // P overwrote the logits
     if (c->scal_h[SC_NONFINITE] != 0.0) return fail(c, EMC_E_NONFINITE, "normalize_resp: non-finite log-sum-exp");
-    if (total_logl) EMC_TRY(total_logl_host(c, total_logl));
+    if (total_logl) *total_logl = c->scal_h[SC_TOTAL];
     return EMC_OK;
 }
 
@@ -990,7 +973,6 @@ extern "C" emc_status emc_iterate(emc_ctx *c, int32_t iteration, emc_iter_stats 
     HIP_TRY(c, hipSetDevice(c->opt.device));
     const double sigma = emc_sigma_schedule(iteration, c->opt.sigma_start, c->opt.sigma_final, c->opt.sigma_half_life);
     if (c->opt.timing) (void)hipEventRecord(c->ev[2 * EMC_STAGE_TOTAL], c->stream);
-    HIP_TRY(c, launch_fill_f64(c->scal + SC_NONFINITE, 0.0, 1, c->stream));
 
     // search policy: full search until the network has trained, during the warm-up, on every
     // full_every-th iteration after it, and when too many patterns would fall back
@@ -1086,7 +1068,7 @@ extern "C" emc_status emc_iterate(emc_ctx *c, int32_t iteration, emc_iter_stats 
         stats->fluence = c->scal_h[SC_PHI0];
         stats->model_avg = c->scal_h[SC_AVG];
         stats->weight_sum = c->scal_h[SC_WSUM];
-        EMC_TRY(total_logl_host(c, &stats->total_logl));
+        stats->total_logl = c->scal_h[SC_TOTAL];
         stats->search = full ? EMC_SEARCH_FULL : EMC_SEARCH_PROPOSAL;
         stats->n_fallback = predicted ? n_fb : 0;
         stats->predicted_mass = pmass_mean;

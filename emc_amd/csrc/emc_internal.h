@@ -25,7 +25,7 @@ inline int64_t round_up(int64_t a, int64_t b) { return (a + b - 1) / b * b; }
 enum {
     SC_PHI0 = 0,      // global fluence used this iteration
     SC_LOGPHI0 = 1,   // log(phi0)
-    SC_TOTAL = 2,     // sum_i lse'_i (without the per-pattern constants)
+    SC_TOTAL = 2,     // sum_i lse_i (lse'_i and the per-pattern constants)
     SC_AVG = 3,       // model average before normalisation
     SC_INV = 4,       // 1/avg applied
     SC_COUNT = 5,     // positive voxel count
@@ -156,7 +156,6 @@ struct emc_ctx {
     // slicing stage
     double *sumW = nullptr;   // [Sp]
     int32_t *ns = nullptr;    // [Sp]
-    double *colsum = nullptr; // [Pp][2] per pixel: sum over rotations of log W, valid count
     float2 *colp = nullptr;   // [ceil(S / 16)][Pp] per statistics block: (sum of log W, valid count)
     double2 *colpart = nullptr; // [32][Pp] fixed-order partial column sums
     float *colmean = nullptr; // [Pp]
@@ -230,18 +229,17 @@ hipError_t launch_fill_f32(float *p, float v, int64_t n, hipStream_t st);
 hipError_t launch_fill_f64(double *p, double v, int64_t n, hipStream_t st);
 hipError_t launch_fill_i32(int32_t *p, int32_t v, int64_t n, hipStream_t st);
 
-// Slicing statistics over rotations [0, S): sumW, ns and (if colsum) sum of log W per pixel.
-// colp / colpart hold colp_len / colpart_len elements.
+// Slicing statistics over rotations [0, S): sumW, ns, the slices that a later pass reads and (BF16
+// Poisson) the column sums of log W; clears the E-step's non-finite flag.  colp / colpart hold colp_len / colpart_len elements.
 int64_t colp_len(int S, int Pp);
 int64_t colpart_len(int Pp);
-hipError_t launch_slice_stats(const emc_ctx *c, bool want_colsum, hipStream_t st);
-// Fluence, per-rotation bias / chi^2 scale, column means.
+hipError_t launch_slice_stats(const emc_ctx *c, hipStream_t st);
+// Fluence, per-rotation bias / chi^2 scale, column means (without centring: the pattern constants).
 hipError_t launch_bias(const emc_ctx *c, float sigma, hipStream_t st);
-// Per-pattern constant: cst[i] = sum_j K[i,j] colmean[j] (MFMA path) - B0.
-hipError_t launch_pattern_const(const emc_ctx *c, bool centred, hipStream_t st);
 // FP32 slices of rotations [s0, s0+cs) into A0/A1 (rows up to chunkp zero-padded).
 hipError_t launch_slice_f32(const emc_ctx *c, int s0, int cs, hipStream_t st);
-// BF16-split centred log-slices into Lh/Lm/Ll.
+// BF16-split centred log-slices into Lh/Lm/Ll; with the first chunk (s0 = 0) also the patterns' constants
+// cst[i] = sum_j K[i,j] colmean[j] - B0.
 hipError_t launch_slice_bf16(const emc_ctx *c, int s0, int cs, hipStream_t st);
 // Full-detector slice values of rotations [s0, s0+cs) into out [cs][P] (-1 invalid/masked).
 hipError_t launch_expand(const emc_ctx *c, int s0, int cs, float *out, hipStream_t st);
@@ -315,7 +313,8 @@ hipError_t launch_compress_buffers(int L, double blur_sigma, bool new_taps, cons
                                    float *model, float *taps, float *t1, float *t2, double *red, double *scal,
                                    double *avg_out, hipStream_t st);
 // Deterministic single-workgroup sum of n doubles into *out.
-hipError_t launch_sum_f64(const double *x, int n, double *out, hipStream_t st);
+hipError_t launch_sm_sums(const emc_ctx *c, const double *nz, int nnz, const double *blk, int nblk, const double *Tpart,
+                          int ncb, hipStream_t st);
 
 // ---- learned proposal ------------------------------------------------------------------------
 // Grouped (per coarse cell) contractions and softmax over the work lists in c->prop.

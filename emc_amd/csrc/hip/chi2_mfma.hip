@@ -9,6 +9,7 @@
 // over the same pixels.  The FP32 products go through the large-tile kernel's store epilogue; one
 // elementwise pass combines them into the logits (in double) and 1/phi.
 #include "../emc_internal.h"
+#include "geom.h"
 
 namespace emc {
 namespace {
@@ -20,43 +21,63 @@ __device__ __forceinline__ T wave_sum(T v)
     return v;
 }
 
-// x -> NT BF16 terms whose sum carries ~8 NT significant bits of x.
+// x -> NT BF16 terms whose sum carries ~8 NT significant bits of x; two values, packed, per store.
 template <int NT>
-__device__ __forceinline__ void split(float x, bf16_t *t0, bf16_t *t1, bf16_t *t2, size_t o)
+__device__ __forceinline__ void split(const float *x, uint32_t *const *t, size_t o)
 {
-    const bf16_t h = f2bf(x);
-    const float r1 = x - bf2f(h);
-    const bf16_t m = f2bf(r1);
-    t0[o] = h;
-    t1[o] = m;
-    if (NT == 3) t2[o] = f2bf(r1 - bf2f(m));
+    uint32_t h[2], m[2], l[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const bf16_t hb = f2bf(x[q]);
+        const float r1 = x[q] - bf2f(hb);
+        const bf16_t mb = f2bf(r1);
+        h[q] = hb;
+        m[q] = mb;
+        l[q] = f2bf(r1 - bf2f(mb));
+    }
+    t[0][o] = h[0] | (h[1] << 16);
+    if (NT > 1) t[1][o] = m[0] | (m[1] << 16);
+    if (NT > 2) t[2][o] = l[0] | (l[1] << 16);
 }
 
-// One workgroup per chunk row r: the four operands from the FP32 slices (A0 = W, A1 = a; both 0 on
-// invalid samples, masked pixels and padding rows) and Aw[r] = sum a W^2.
+// One workgroup per chunk row r: the four operands from the slices kept by the statistics pass (W, 0 on
+// invalid samples; masked pixels and padding rows count as 0) and Aw[r] = sum a W^2.  Two pixels per thread.
 template <int NT>
-__global__ __launch_bounds__(256) void k_chi2_operands(const float *__restrict__ A0, const float *__restrict__ A1,
-                                                       int Pp, int64_t plane, bool scaling, bf16_t *__restrict__ Cx,
+__global__ __launch_bounds__(256) void k_chi2_operands(const float *__restrict__ Wk, int cs, int Pa, int Pp, int kind,
+                                                       int64_t plane, bool scaling, bf16_t *__restrict__ Cx,
                                                        double *__restrict__ Aw)
 {
     __shared__ double red[4];
     const int r = blockIdx.x;
     double acc = 0.0;
-    bf16_t *t[4][3];
+    uint32_t *t[4][3];
 #pragma unroll
     for (int p = 0; p < 4; ++p)
 #pragma unroll
-        for (int q = 0; q < 3; ++q) t[p][q] = Cx + (int64_t)(p * NT + (q < NT ? q : 0)) * plane;
-    for (int j = threadIdx.x; j < Pp; j += 256) {
-        const size_t o = (size_t)r * Pp + j;
-        const float W = A0[o], a = A1[o];
-        acc += (double)a * W * W;
-        split<NT>(a * W, t[0][0], t[0][1], t[0][2], o);
-        split<NT>(a, t[1][0], t[1][1], t[1][2], o);
+        for (int q = 0; q < 3; ++q)
+            t[p][q] = reinterpret_cast<uint32_t *>(Cx + (int64_t)(p * NT + (q < NT ? q : 0)) * plane);
+    for (int j = 2 * threadIdx.x; j < Pp; j += 512) {  // Pp is even
+        const size_t o = ((size_t)r * Pp + j) / 2;
+        float W[2] = {0.0f, 0.0f}, a[2], aW[2], in[2], Wi[2];
+        if (r < cs) {
+            const float2 v = *reinterpret_cast<const float2 *>(Wk + (size_t)r * Pp + j);
+            if (j < Pa) W[0] = v.x;
+            if (j + 1 < Pa) W[1] = v.y;
+        }
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            a[q] = W[q] > 0.0f ? chi2_weight(W[q], kind) : 0.0f;
+            aW[q] = a[q] * W[q];
+            acc += (double)a[q] * W[q] * W[q];
+            const bool ok = W[q] > 1.0e-10f;  // emc_cuda.cu:444 (a zero count adds nothing to either sum)
+            in[q] = ok ? 1.0f : 0.0f;
+            Wi[q] = ok ? W[q] : 0.0f;
+        }
+        split<NT>(aW, t[0], o);
+        split<NT>(a, t[1], o);
         if (scaling) {
-            const bool in = W > 1.0e-10f;  // emc_cuda.cu:444 (a zero count adds nothing to either sum)
-            t[2][0][o] = f2bf(in ? 1.0f : 0.0f);  // the indicator is exact in one term
-            split<NT>(in ? W : 0.0f, t[3][0], t[3][1], t[3][2], o);
+            split<1>(in, t[2], o);  // the indicator is exact in one term
+            split<NT>(Wi, t[3], o);
         }
     }
     acc = wave_sum(acc);
@@ -97,12 +118,13 @@ hipError_t launch_logl_chi2_mfma(const emc_ctx *c, int s0, int cs, hipStream_t s
     const int NT = c->la_terms;
     const int64_t plane = (int64_t)c->chunkp * c->Pp;
     const bool scaling = c->opt.scaling != 0;
-    if (NT == 3)
-        hipLaunchKernelGGL(k_chi2_operands<3>, dim3(c->chunkp), dim3(256), 0, st, c->A0, c->A1, c->Pp, plane, scaling,
+    const float *Wk = c->lw32 + (size_t)s0 * c->Pp;
+    const auto operands = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(c->chunkp), dim3(256), 0, st, Wk, cs, c->Pa, c->Pp, (int)c->opt.diff, plane, scaling,
                            c->Cx, c->Aw);
-    else
-        hipLaunchKernelGGL(k_chi2_operands<2>, dim3(c->chunkp), dim3(256), 0, st, c->A0, c->A1, c->Pp, plane, scaling,
-                           c->Cx, c->Aw);
+    };
+    if (NT == 3) operands(k_chi2_operands<3>);
+    else operands(k_chi2_operands<2>);
     hipError_t e = hipGetLastError();
     auto op = [&](int p, int q) { return c->Cx + (int64_t)(p * NT + q) * plane; };
     auto with_counts = [&](int p, float *C) {  // C = X_p . K^T (hi + lo counts above 256)

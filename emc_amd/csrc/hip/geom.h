@@ -109,6 +109,12 @@ __device__ __forceinline__ float sample_quad(const float4 *__restrict__ modelq, 
     return c0 * gz + c1 * fz;
 }
 
+// Pixel weight of the chi^2 kinds: poisson (reference chi^2) 1/(W+0.02), absolute 1, relative 1/W^2.
+__device__ __forceinline__ float chi2_weight(float W, int kind)
+{
+    return kind == EMC_DIFF_POISSON ? 1.0f / (W + 0.02f) : (kind == EMC_DIFF_ABSOLUTE ? 1.0f : 1.0f / (W * W));
+}
+
 __device__ __forceinline__ void load_rot(const float *__restrict__ rotm, int s, float *m)
 {
     const float4 a = *reinterpret_cast<const float4 *>(rotm + 12 * (size_t)s);

@@ -486,16 +486,14 @@ hipError_t launch_grouped_softmax(const emc_ctx *c, hipStream_t st)
     const int ncol = (c->I + 255) / 256;
     double *blk = c->part;
     hipLaunchKernelGGL(k_gsm_final, dim3(ncol), dim3(256), 0, st, p->slot_pm, p->slot_ps, g, c->I, c->lse, blk, c->scal);
-    hipError_t e = launch_sum_f64(blk, ncol, c->scal + SC_TOTAL, st);
-    if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_slot_lse, dim3((unsigned)((p->n_slots + 255) / 256)), dim3(256), 0, st, g.slot_pat, c->lse,
                        p->n_slots, p->slot_lse);
     double *nzrow = c->part + blk_pad(c);  // one non-zero count per fine rotation
     hipLaunchKernelGGL(k_gsm_apply, dim3((c->S + 3) / 4), dim3(256), 0, st, c->R, g, c->S, p->slot_lse, c->Ph, c->Pl,
                        c->T, nzrow);
-    e = launch_mark_p_dirty(c, st);  // Ph / Pl now hold the grouped layout
+    hipError_t e = launch_mark_p_dirty(c, st);  // Ph / Pl now hold the grouped layout
     if (e != hipSuccess) return e;
-    return launch_sum_f64(nzrow, c->S, c->scal + SC_NNZ, st);
+    return launch_sm_sums(c, nzrow, c->S, blk, ncol, nullptr, 0, st);
 }
 
 hipError_t launch_recall_grouped(const emc_ctx *c, hipStream_t st)

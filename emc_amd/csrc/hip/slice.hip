@@ -52,8 +52,10 @@ __global__ void k_fill(T *__restrict__ p, T v, int64_t n)
 // log W and number of rotations with a valid sample (colp[block][j] = (sum, count); summed over
 // the blocks in a fixed order by k_colsum_*, so the column sums are deterministic).
 // kStatsG rotations per workgroup; each thread walks pixels j = tid, tid+256, ... and keeps the
-// kStatsG partial sums in registers.  With lw, the pass also keeps log W ([Sp][Pp], -inf where
-// W <= 0) for the operand split, which then needs no second gather from the model.
+// kStatsG partial sums in registers.  KEEP_LOG keeps log W ([S][Pp], -inf where W <= 0) for the
+// operand split, KEEP_W keeps W (0 where invalid) for the chi^2 operands, KEEP_WA the FP32 chi^2
+// contraction's operands W and a themselves: a second gather from the model costs as much as this one
+// (64^3 / 6,300 rotations 125 us), reading back what was kept 20 to 50 us.
 // modelq[v] = (model[v], model[v + 1], model[v + L], model[v + L + 1]), 0 past an edge (the trilinear
 // statistics pass reads the 8 corners of a sample as two 16-byte loads).
 __global__ void k_quad_model(const float *__restrict__ model, int L, float4 *__restrict__ modelq)
@@ -66,13 +68,17 @@ __global__ void k_quad_model(const float *__restrict__ model, int L, float4 *__r
     }
 }
 
-template <int INTERP>
+// What the statistics pass keeps of its samples, so that no later pass gathers from the model again.
+enum { KEEP_NONE, KEEP_LOG, KEEP_W, KEEP_WA };
+
+template <int INTERP, int KEEP>
 __global__ __launch_bounds__(256) void k_slice_stats(const float *__restrict__ model,
                                                      const float4 *__restrict__ modelq, int L,
                                                      const float *__restrict__ rotm, int S,
-                                                     const float *__restrict__ axyz, int Pa, int Pp,
+                                                     const float *__restrict__ axyz, int Pa, int Pp, int kind,
                                                      double *__restrict__ sumW, int32_t *__restrict__ ns,
-                                                     float2 *__restrict__ colp, float *__restrict__ lw)
+                                                     float2 *__restrict__ colp, float *__restrict__ out0,
+                                                     float *__restrict__ out1, double *__restrict__ scal)
 {
     __shared__ float rm[kStatsG][9];
     __shared__ double red_w[kStatsG][256];
@@ -86,10 +92,17 @@ __global__ __launch_bounds__(256) void k_slice_stats(const float *__restrict__ m
     }
     __syncthreads();
     const int ng = min(kStatsG, S - s0);
+    if (blockIdx.x == 0 && tid == 0) scal[SC_NONFINITE] = 0.0;  // the first kernel of an E-step
     float sw[kStatsG];
     int cnt[kStatsG];
 #pragma unroll
     for (int g = 0; g < kStatsG; ++g) { sw[g] = 0.0f; cnt[g] = 0; }
+    if (KEEP == KEEP_WA)  // the contraction reads whole tiles: padding pixels and rotations are zeros
+        for (int g = 0; g < kStatsG; ++g)
+            for (int j = (g < ng ? Pa : 0) + tid; j < Pp; j += 256) {
+                out0[(size_t)(s0 + g) * Pp + j] = 0.0f;
+                out1[(size_t)(s0 + g) * Pp + j] = 0.0f;
+            }
     for (int j = tid; j < Pa; j += 256) {
         const float X = axyz[j], Y = axyz[Pp + j], Z = axyz[2 * Pp + j];
         float col = 0.0f;
@@ -99,18 +112,25 @@ __global__ __launch_bounds__(256) void k_slice_stats(const float *__restrict__ m
             if (g < ng) {
                 const float W = INTERP == EMC_INTERP_TRILINEAR ? sample_quad(modelq, L, rm[g], X, Y, Z)
                                                                : sample<INTERP>(model, L, rm[g], X, Y, Z);
-                float l = -INFINITY;
+                const size_t o = (size_t)(s0 + g) * Pp + j;
+                float v0 = KEEP == KEEP_LOG ? -INFINITY : 0.0f, v1 = 0.0f;
                 if (W > 0.0f) {
-                    l = logf(W);
                     sw[g] += W;
                     cnt[g] += 1;
-                    col += l;
-                    colv += 1;
+                    if (KEEP == KEEP_LOG) {
+                        v0 = logf(W);
+                        col += v0;
+                        colv += 1;
+                    } else {
+                        v0 = W;
+                        if (KEEP == KEEP_WA) v1 = chi2_weight(W, kind);
+                    }
                 }
-                if (lw) lw[(size_t)(s0 + g) * Pp + j] = l;
+                if (KEEP != KEEP_NONE) out0[o] = v0;
+                if (KEEP == KEEP_WA) out1[o] = v1;
             }
         }
-        if (colp) colp[(size_t)blockIdx.x * Pp + j] = make_float2(col, (float)colv);
+        if (KEEP == KEEP_LOG && colp) colp[(size_t)blockIdx.x * Pp + j] = make_float2(col, (float)colv);
     }
     // per-rotation sums over the workgroup's 256 threads through LDS, in a fixed order: 32 lanes per
     // rotation add 8 values each, then five shuffle steps
@@ -143,7 +163,7 @@ __global__ __launch_bounds__(256) void k_slice_stats(const float *__restrict__ m
 }
 
 // Column sums of the statistics pass, in two fixed-order steps: part r of the blocks
-// [r * per, (r + 1) * per) per pixel, then the kColParts parts in order.
+// [r * per, (r + 1) * per) per pixel here, then the kColParts parts in order (k_bias).
 constexpr int kColParts = 32;
 
 __global__ __launch_bounds__(256) void k_colsum_part(const float2 *__restrict__ colp, int nblk, int Pa, int Pp,
@@ -171,22 +191,6 @@ __global__ __launch_bounds__(256) void k_colsum_part(const float2 *__restrict__ 
     cpart[(size_t)r * Pp + j] = make_double2(a, n);
 }
 
-__global__ __launch_bounds__(256) void k_colsum_final(const double2 *__restrict__ cpart, int Pa, int Pp,
-                                                      double *__restrict__ colsum)
-{
-    const int j = blockIdx.x * 256 + threadIdx.x;
-    if (j >= Pp) return;
-    double a = 0.0, n = 0.0;
-    if (j < Pa)
-        for (int r = 0; r < kColParts; ++r) {
-            const double2 v = cpart[(size_t)r * Pp + j];
-            a += v.x;
-            n += v.y;
-        }
-    colsum[2 * j] = a;
-    colsum[2 * j + 1] = n;
-}
-
 // FP32 slice rows for the plain contraction.  KIND: TRUE_POISSON -> A0 = log(phi0 W) (0 if
 // invalid; log phi0 is read from the device scalars written by k_bias);
 // chi^2 kinds -> A0 = W, A1 = pixel weight a (0 if invalid):
@@ -212,8 +216,7 @@ __global__ __launch_bounds__(256) void k_slice_f32(const float *__restrict__ mod
                     a0 = logf(W) + logphi0;
                 } else {
                     a0 = W;
-                    a1 = KIND == EMC_DIFF_POISSON ? 1.0f / (W + 0.02f)
-                                                  : (KIND == EMC_DIFF_ABSOLUTE ? 1.0f : 1.0f / (W * W));
+                    a1 = chi2_weight(W, KIND);
                 }
             }
         }
@@ -222,45 +225,70 @@ __global__ __launch_bounds__(256) void k_slice_f32(const float *__restrict__ mod
     }
 }
 
-// Centred log-slice x = (W > 0 ? log(phi0 W) : 0) - colmean[j] split into NT BF16 terms
-// (hi, [mid,] lo) whose sum carries ~8*NT significant bits of x.
-template <int INTERP, int NT>
-__global__ __launch_bounds__(256) void k_slice_bf16(const float *__restrict__ model, int L,
-                                                    const float *__restrict__ rotm, int s0, int cs,
-                                                    const float *__restrict__ axyz, int Pa, int Pp,
-                                                    const float *__restrict__ colmean,
-                                                    const double *__restrict__ scal,
-                                                    bf16_t *__restrict__ Lh, bf16_t *__restrict__ Lm,
-                                                    bf16_t *__restrict__ Ll)
+// log W kept by the statistics pass -> A0 = log(phi0 W) (0 where invalid and in the padding), in place.
+__global__ __launch_bounds__(256) void k_log_phi0(float *__restrict__ A0, int cs, int rows, int Pa, int Pp,
+                                                  const double *__restrict__ scal)
 {
-    const int r = blockIdx.x;
-    const bool row_ok = r < cs;
     const float logphi0 = (float)scal[SC_LOGPHI0];
-    float m[9];
-    if (row_ok) load_rot(rotm, s0 + r, m);
-    for (int j = threadIdx.x; j < Pp; j += 256) {
-        float x = 0.0f;
-        if (row_ok && j < Pa) {
-            const float W = sample<INTERP>(model, L, m, axyz[j], axyz[Pp + j], axyz[2 * Pp + j]);
-            x = (W > 0.0f ? logf(W) + logphi0 : 0.0f) - colmean[j];
-        }
-        const bf16_t h = f2bf(x);
-        const float r1 = x - bf2f(h);
-        const bf16_t mi = f2bf(r1);
-        const size_t o = (size_t)r * Pp + j;
-        Lh[o] = h;
-        if (NT == 2) {
-            Ll[o] = mi;
-        } else {
-            Lm[o] = mi;
-            Ll[o] = f2bf(r1 - bf2f(mi));
-        }
+    const int quads = Pp / 4;  // Pp is a multiple of 128
+    const int64_t n = (int64_t)rows * quads;
+    for (int64_t t = blockIdx.x * 256 + threadIdx.x; t < n; t += (int64_t)gridDim.x * 256) {
+        const int r = (int)(t / quads), j = (int)(t % quads) * 4;
+        float4 *p = reinterpret_cast<float4 *>(A0) + t;
+        const float4 v = *p;
+        const float l[4] = {v.x, v.y, v.z, v.w};
+        float x[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[q] = r < cs && j + q < Pa && l[q] > -INFINITY ? l[q] + logphi0 : 0.0f;
+        *p = make_float4(x[0], x[1], x[2], x[3]);
     }
 }
 
-// The same operand split from the log W kept by the statistics pass: x = (log W + log phi0, or 0
-// where W <= 0) - colmean[j], the same float operations as k_slice_bf16, so the terms are
-// bit-identical.  Four pixels per thread and kSplitRows rows per workgroup, whose loads are issued
+// cst_i = sum_j K_ij colmean_j - B0 (FP64), one wavefront per pattern.
+__device__ __forceinline__ void pattern_const(const bf16_t *__restrict__ K16, const bf16_t *__restrict__ K16lo,
+                                              const uint8_t *__restrict__ K8, int i, int Pp,
+                                              const float *__restrict__ colmean, double B0,
+                                              double *__restrict__ cst)
+{
+    const int lane = threadIdx.x & 63;
+    double acc = 0.0;
+    if (K8) {  // byte counts (exact): 16 per lane and 16-byte load (Pp % 16 == 0)
+        for (int j = lane * 16; j < Pp; j += 64 * 16) {
+            const uint4 v = *reinterpret_cast<const uint4 *>(K8 + (size_t)i * Pp + j);
+            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float4 m = *reinterpret_cast<const float4 *>(colmean + j + 4 * q);
+                acc = fma((double)(w[q] & 0xffu), (double)m.x, acc);
+                acc = fma((double)((w[q] >> 8) & 0xffu), (double)m.y, acc);
+                acc = fma((double)((w[q] >> 16) & 0xffu), (double)m.z, acc);
+                acc = fma((double)(w[q] >> 24), (double)m.w, acc);
+            }
+        }
+    } else {  // eight per lane and 16-byte load
+        for (int j = lane * 8; j < Pp; j += 64 * 8) {
+            const uint4 v = *reinterpret_cast<const uint4 *>(K16 + (size_t)i * Pp + j);
+            const uint4 u = K16lo ? *reinterpret_cast<const uint4 *>(K16lo + (size_t)i * Pp + j) : make_uint4(0, 0, 0, 0);
+            const uint32_t w[4] = {v.x, v.y, v.z, v.w}, l[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float2 m = *reinterpret_cast<const float2 *>(colmean + j + 2 * q);
+                const float k0 = __uint_as_float(w[q] << 16) + __uint_as_float(l[q] << 16);
+                const float k1 = __uint_as_float(w[q] & 0xffff0000u) + __uint_as_float(l[q] & 0xffff0000u);
+                acc = fma((double)k0, (double)m.x, acc);
+                acc = fma((double)k1, (double)m.y, acc);
+            }
+        }
+    }
+    acc = wave_sum(acc);
+    if (lane == 0) cst[i] = acc - B0;
+}
+
+// Centred log-slice x = (log W + log phi0, or 0 where W <= 0) - colmean[j], from the log W kept by the
+// statistics pass, split into NT BF16 terms (hi, [mid,] lo) whose sum carries ~8*NT significant bits
+// of x.  The workgroups past the first nsplit rows of the grid form the patterns' constants, which
+// depend on the same column means (a launch of their own took 13 us at 32^3 / 1,000 patterns and 60 us with
+// split counts read element by element).  Four pixels per thread and kSplitRows rows per workgroup, whose loads are issued
 // together (the column means are read once for all of them).  Pp is a multiple of 128.
 constexpr int kSplitRows = 8;
 
@@ -268,8 +296,15 @@ template <int NT>
 __global__ __launch_bounds__(256) void k_split_bf16(const float *__restrict__ lw, int s0, int cs, int Pa, int Pp,
                                                     const float *__restrict__ colmean,
                                                     const double *__restrict__ scal, bf16_t *__restrict__ Lh,
-                                                    bf16_t *__restrict__ Lm, bf16_t *__restrict__ Ll)
+                                                    bf16_t *__restrict__ Lm, bf16_t *__restrict__ Ll, int nsplit,
+                                                    const bf16_t *__restrict__ K16, const bf16_t *__restrict__ K16lo,
+                                                    const uint8_t *__restrict__ K8, int I, double *__restrict__ cst)
 {
+    if ((int)blockIdx.y >= nsplit) {
+        const int i = (((int)blockIdx.y - nsplit) * (int)gridDim.x + (int)blockIdx.x) * 4 + (int)(threadIdx.x >> 6);
+        if (i < I) pattern_const(K16, K16lo, K8, i, Pp, colmean, scal[SC_B0], cst);  // a whole wavefront
+        return;
+    }
     const int r0 = blockIdx.y * kSplitRows;
     const int j0 = (blockIdx.x * 256 + threadIdx.x) * 4;
     if (j0 >= Pp) return;
@@ -335,9 +370,10 @@ __global__ __launch_bounds__(256) void k_expand(const float *__restrict__ model,
 __global__ __launch_bounds__(1024) void k_bias(const double *__restrict__ sumW, const int32_t *__restrict__ ns,
                                                const float *__restrict__ logw, int S, int Sp, int I,
                                                double sumK_total, double fluence, int diff, float sigma,
-                                               const double *__restrict__ colsum, int Pa, int Pp,
+                                               const double2 *__restrict__ cpart, int Pa, int Pp,
                                                float *__restrict__ bias, float *__restrict__ rscale,
-                                               float *__restrict__ colmean, double *__restrict__ scal)
+                                               float *__restrict__ colmean, double *__restrict__ cst,
+                                               double *__restrict__ scal)
 {
     __shared__ double red[16];
     const int tid = threadIdx.x;
@@ -369,8 +405,9 @@ __global__ __launch_bounds__(1024) void k_bias(const double *__restrict__ sumW, 
         scal[SC_B0] = B0;
     }
     const double inv2s2 = 1.0 / (2.0 * (double)sigma * (double)sigma);
-    const int t0 = blockIdx.x * 1024 + tid, stride = gridDim.x * 1024;
-#pragma unroll 4
+    // 256 elements per workgroup: the column sums' 32 loads a pixel then come from many compute units
+    if (tid >= 256) return;
+    const int t0 = blockIdx.x * 256 + tid, stride = gridDim.x * 256;
     for (int s = t0; s < Sp; s += stride) {
         float b = 0.0f, rs = 0.0f;
         if (s < S) {
@@ -383,51 +420,23 @@ __global__ __launch_bounds__(1024) void k_bias(const double *__restrict__ sumW, 
         bias[s] = b;
         rscale[s] = rs;
     }
+    if (!cpart) {  // no centring: the pattern constants are the shift alone
+        for (int i = t0; i < I; i += stride) cst[i] = -B0;
+        return;
+    }
     // column mean of log(phi0 W) over rotations (invalid samples count as 0)
     const double lp = log(phi0);
-    for (int j = t0; j < Pp; j += stride)
-        colmean[j] = (colsum && j < Pa && S > 0) ? (float)((colsum[2 * j] + colsum[2 * j + 1] * lp) / S) : 0.0f;
-}
-
-// cst_i = sum_j K_ij colmean_j - B0   (FP64; one wavefront per pattern, four per workgroup)
-__global__ __launch_bounds__(256) void k_pattern_const(const float *__restrict__ K32,
-                                                       const bf16_t *__restrict__ K16,
-                                                       const bf16_t *__restrict__ K16lo,
-                                                       const uint8_t *__restrict__ K8, int I, int Pp,
-                                                       const float *__restrict__ colmean,
-                                                       const double *__restrict__ sumK,
-                                                       const double *__restrict__ scal, bool centred,
-                                                       double *__restrict__ cst)
-{
-    const int lane = threadIdx.x & 63, i = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (i >= I) return;  // a whole wavefront
-    double acc = 0.0;
-    if (centred && K8) {  // byte counts (exact): 16 per lane and 16-byte load (Pp % 16 == 0)
-        for (int j = lane * 16; j < Pp; j += 64 * 16) {
-            const uint4 v = *reinterpret_cast<const uint4 *>(K8 + (size_t)i * Pp + j);
-            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const float4 m = *reinterpret_cast<const float4 *>(colmean + j + 4 * q);
-                acc = fma((double)(w[q] & 0xffu), (double)m.x, acc);
-                acc = fma((double)((w[q] >> 8) & 0xffu), (double)m.y, acc);
-                acc = fma((double)((w[q] >> 16) & 0xffu), (double)m.z, acc);
-                acc = fma((double)(w[q] >> 24), (double)m.w, acc);
+    for (int j = t0; j < Pp; j += stride) {
+        double a = 0.0, n = 0.0;
+        if (j < Pa)
+#pragma unroll 16
+            for (int r = 0; r < kColParts; ++r) {
+                const double2 v = cpart[(size_t)r * Pp + j];
+                a += v.x;
+                n += v.y;
             }
-        }
-    } else if (centred) {
-        for (int j = lane; j < Pp; j += 64) {
-            float k;
-            if (K32) k = K32[(size_t)i * Pp + j];
-            else {
-                k = bf2f(K16[(size_t)i * Pp + j]);
-                if (K16lo) k += bf2f(K16lo[(size_t)i * Pp + j]);
-            }
-            acc += (double)k * (double)colmean[j];
-        }
+        colmean[j] = j < Pa && S > 0 ? (float)((a + n * lp) / S) : 0.0f;
     }
-    acc = wave_sum(acc);
-    if (lane == 0) cst[i] = acc - scal[SC_B0];
 }
 
 }  // namespace
@@ -466,42 +475,48 @@ hipError_t launch_fill_i32(int32_t *p, int32_t v, int64_t n, hipStream_t st)
 int64_t colp_len(int S, int Pp) { return (int64_t)((S + kStatsG - 1) / kStatsG) * Pp; }
 int64_t colpart_len(int Pp) { return (int64_t)kColParts * Pp; }
 
-hipError_t launch_slice_stats(const emc_ctx *c, bool want_colsum, hipStream_t st)
+// The FP32 path's operands come from the statistics pass when one chunk covers every rotation.
+static bool f32_slices_kept(const emc_ctx *c) { return !c->mfma && c->chunk >= c->S; }
+
+template <int INTERP>
+static void slice_stats_interp(const emc_ctx *c, hipStream_t st)
 {
-    const int nblk = (c->S + kStatsG - 1) / kStatsG;
-    float2 *cp = want_colsum ? c->colp : nullptr;
+    const int nblk = (c->S + kStatsG - 1) / kStatsG, nall = c->chunkp / kStatsG;  // with the padding rows
+    const bool poisson = c->opt.diff == EMC_DIFF_TRUE_POISSON;
+    const auto run = [&](auto kernel, float2 *colp, float *out0, float *out1) {
+        hipLaunchKernelGGL(kernel, dim3(out1 ? nall : nblk), dim3(256), 0, st, c->model, c->modelq, c->L, c->rotm, c->S, c->axyz, c->Pa,
+                           c->Pp, (int)c->opt.diff, c->sumW, c->ns, colp, out0, out1, c->scal);
+    };
+    if (c->chi2_mfma) run(k_slice_stats<INTERP, KEEP_W>, nullptr, c->lw32, nullptr);
+    else if (c->mfma) run(k_slice_stats<INTERP, KEEP_LOG>, c->colp, c->lw32, nullptr);
+    else if (f32_slices_kept(c) && poisson) run(k_slice_stats<INTERP, KEEP_LOG>, nullptr, c->A0, nullptr);
+    else if (f32_slices_kept(c)) run(k_slice_stats<INTERP, KEEP_WA>, nullptr, c->A0, c->A1);
+    else run(k_slice_stats<INTERP, KEEP_NONE>, nullptr, nullptr, nullptr);
+}
+
+hipError_t launch_slice_stats(const emc_ctx *c, hipStream_t st)
+{
     if (c->opt.interp == EMC_INTERP_NEAREST) {
-        hipLaunchKernelGGL(k_slice_stats<EMC_INTERP_NEAREST>, dim3(nblk), dim3(256), 0, st, c->model, nullptr, c->L,
-                           c->rotm, c->S, c->axyz, c->Pa, c->Pp, c->sumW, c->ns, cp, c->lw32);
+        slice_stats_interp<EMC_INTERP_NEAREST>(c, st);
     } else {
         const int64_t n3 = (int64_t)c->L * c->L * c->L;
         hipLaunchKernelGGL(k_quad_model, dim3((unsigned)std::min<int64_t>((n3 + 255) / 256, 4096)), dim3(256), 0, st,
                            c->model, c->L, c->modelq);
-        hipLaunchKernelGGL(k_slice_stats<EMC_INTERP_TRILINEAR>, dim3(nblk), dim3(256), 0, st, c->model, c->modelq,
-                           c->L, c->rotm, c->S, c->axyz, c->Pa, c->Pp, c->sumW, c->ns, cp, c->lw32);
+        slice_stats_interp<EMC_INTERP_TRILINEAR>(c, st);
     }
-    if (want_colsum) {
-        hipLaunchKernelGGL(k_colsum_part, dim3((c->Pa + 255) / 256, kColParts), dim3(256), 0, st, c->colp, nblk, c->Pa,
-                           c->Pp, c->colpart);
-        hipLaunchKernelGGL(k_colsum_final, dim3((c->Pp + 255) / 256), dim3(256), 0, st, c->colpart, c->Pa, c->Pp,
-                           c->colsum);
-    }
+    if (c->mfma && !c->chi2_mfma)
+        hipLaunchKernelGGL(k_colsum_part, dim3((c->Pa + 255) / 256, kColParts), dim3(256), 0, st, c->colp,
+                           (c->S + kStatsG - 1) / kStatsG, c->Pa, c->Pp, c->colpart);
     return hipGetLastError();
 }
 
 hipError_t launch_bias(const emc_ctx *c, float sigma, hipStream_t st)
 {
-    const int nb = std::max(1, (std::max(c->Sp, c->Pp) + 1023) / 1024);
+    const int nb = std::max(1, (std::max(c->Sp, c->Pp) + 255) / 256);
     hipLaunchKernelGGL(k_bias, dim3(nb), dim3(1024), 0, st, c->sumW, c->ns, c->logw, c->S, c->Sp, c->I,
-                       c->sumK_total, c->opt.fluence, c->opt.diff, sigma, c->mfma ? c->colsum : nullptr,
-                       c->Pa, c->Pp, c->bias, c->rscale, c->colmean, c->scal);
-    return hipGetLastError();
-}
-
-hipError_t launch_pattern_const(const emc_ctx *c, bool centred, hipStream_t st)
-{
-    hipLaunchKernelGGL(k_pattern_const, dim3((c->I + 3) / 4), dim3(256), 0, st, c->K32, c->K16, c->k_split ? c->K16lo : nullptr, c->K8, c->I,
-                       c->Pp, c->colmean, c->sumK, c->scal, centred, c->cst);
+                       c->sumK_total, c->opt.fluence, c->opt.diff, sigma,
+                       c->mfma && !c->chi2_mfma ? c->colpart : nullptr, c->Pa, c->Pp, c->bias, c->rscale, c->colmean,
+                       c->cst, c->scal);
     return hipGetLastError();
 }
 
@@ -532,39 +547,28 @@ static hipError_t slice_f32_interp(const emc_ctx *c, int s0, int cs, hipStream_t
 
 hipError_t launch_slice_f32(const emc_ctx *c, int s0, int cs, hipStream_t st)
 {
+    if (f32_slices_kept(c)) {
+        const int64_t n = (int64_t)c->chunkp * c->Pp / 4;
+        if (c->opt.diff == EMC_DIFF_TRUE_POISSON)
+            hipLaunchKernelGGL(k_log_phi0, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 8192)), dim3(256), 0, st, c->A0,
+                               cs, c->chunkp, c->Pa, c->Pp, c->scal);
+        return hipGetLastError();
+    }
     return c->opt.interp == EMC_INTERP_NEAREST ? slice_f32_interp<EMC_INTERP_NEAREST>(c, s0, cs, st)
                                                : slice_f32_interp<EMC_INTERP_TRILINEAR>(c, s0, cs, st);
 }
 
 hipError_t launch_slice_bf16(const emc_ctx *c, int s0, int cs, hipStream_t st)
 {
-    if (c->lw32) {
-        const dim3 g((c->Pp / 4 + 255) / 256, (c->chunkp + kSplitRows - 1) / kSplitRows);
-        if (c->la_terms == 3)
-            hipLaunchKernelGGL(k_split_bf16<3>, g, dim3(256), 0, st, c->lw32, s0, cs, c->Pa, c->Pp, c->colmean, c->scal,
-                               c->Lh, c->Lm, c->Ll);
-        else
-            hipLaunchKernelGGL(k_split_bf16<2>, g, dim3(256), 0, st, c->lw32, s0, cs, c->Pa, c->Pp, c->colmean, c->scal,
-                               c->Lh, c->Lm, c->Ll);
-        return hipGetLastError();
-    }
-    const dim3 grid(c->chunkp), blk(256);
-    const bool nn = c->opt.interp == EMC_INTERP_NEAREST;
-    if (c->la_terms == 3) {
-        if (nn)
-            hipLaunchKernelGGL((k_slice_bf16<EMC_INTERP_NEAREST, 3>), grid, blk, 0, st, c->model, c->L, c->rotm,
-                               s0, cs, c->axyz, c->Pa, c->Pp, c->colmean, c->scal, c->Lh, c->Lm, c->Ll);
-        else
-            hipLaunchKernelGGL((k_slice_bf16<EMC_INTERP_TRILINEAR, 3>), grid, blk, 0, st, c->model, c->L, c->rotm,
-                               s0, cs, c->axyz, c->Pa, c->Pp, c->colmean, c->scal, c->Lh, c->Lm, c->Ll);
-    } else {
-        if (nn)
-            hipLaunchKernelGGL((k_slice_bf16<EMC_INTERP_NEAREST, 2>), grid, blk, 0, st, c->model, c->L, c->rotm,
-                               s0, cs, c->axyz, c->Pa, c->Pp, c->colmean, c->scal, c->Lh, c->Lm, c->Ll);
-        else
-            hipLaunchKernelGGL((k_slice_bf16<EMC_INTERP_TRILINEAR, 2>), grid, blk, 0, st, c->model, c->L, c->rotm,
-                               s0, cs, c->axyz, c->Pa, c->Pp, c->colmean, c->scal, c->Lh, c->Lm, c->Ll);
-    }
+    const int gx = (c->Pp / 4 + 255) / 256, nsplit = (c->chunkp + kSplitRows - 1) / kSplitRows;
+    const int nconst = s0 == 0 ? ((c->I + 3) / 4 + gx - 1) / gx : 0;  // the constants go with the first chunk
+    const auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(gx, nsplit + nconst), dim3(256), 0, st, c->lw32, s0, cs, c->Pa, c->Pp, c->colmean,
+                           c->scal, c->Lh, c->Lm, c->Ll, nsplit, c->K16, c->k_split ? c->K16lo : nullptr, c->K8, c->I,
+                           c->cst);
+    };
+    if (c->la_terms == 3) run(k_split_bf16<3>);
+    else run(k_split_bf16<2>);
     return hipGetLastError();
 }
 

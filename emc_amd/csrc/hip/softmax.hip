@@ -94,10 +94,9 @@ __global__ __launch_bounds__(256) void k_sm_final(const float *__restrict__ pm, 
     if (threadIdx.x == 0) blk_sum[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
 }
 
-// Deterministic single-workgroup sum of n doubles into *out.
-__global__ __launch_bounds__(1024) void k_sum_f64(const double *__restrict__ x, int n, double *__restrict__ out)
+// Deterministic sum of n doubles by one workgroup of 1,024 threads (the value in thread 0).
+__device__ __forceinline__ double block_sum(const double *__restrict__ x, int n, double *red)
 {
-    __shared__ double red[16];
     // eight partial sums per thread (eight loads in flight), added in a fixed order
     double p[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     int k = threadIdx.x;
@@ -109,13 +108,39 @@ __global__ __launch_bounds__(1024) void k_sum_f64(const double *__restrict__ x, 
         if (k + q * 1024 < n) p[q] += x[k + q * 1024];
     double a = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
     a = wave_sum(a);
+    __syncthreads();  // an earlier sum's partials are read
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = a;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double t = 0.0;
-        for (int k = 0; k < 16; ++k) t += red[k];
-        *out = t;
+    double t = 0.0;
+    for (int k = 0; k < 16; ++k) t += red[k];
+    return t;
+}
+
+// The E-step's last sums in one launch (each was a launch of its own, about 5 us of the smallest problems'
+// 200): workgroup 0 the non-zero responsibilities, workgroup 1 the total log-likelihood (log-sum-exps
+// and pattern constants), the others T_s = sum over column blocks of the partial row sums, in order.
+__global__ __launch_bounds__(1024) void k_sm_sums(const double *__restrict__ nz, int nnz, const double *__restrict__ blk,
+                                                  int nblk, const double *__restrict__ cst, int I,
+                                                  const double *__restrict__ Tpart, int ncb, int S, int Sp,
+                                                  double *__restrict__ T, double *__restrict__ scal)
+{
+    __shared__ double red[16];
+    if (blockIdx.x == 0) {
+        const double t = block_sum(nz, nnz, red);
+        if (threadIdx.x == 0) scal[SC_NNZ] = t;
+        return;
     }
+    if (blockIdx.x == 1) {
+        const double t = block_sum(blk, nblk, red) + block_sum(cst, I, red);
+        if (threadIdx.x == 0) scal[SC_TOTAL] = t;
+        return;
+    }
+    const int s = (blockIdx.x - 2) * 1024 + threadIdx.x;
+    if (s >= Sp) return;
+    double t = 0.0;
+    if (s < S)
+        for (int b = 0; b < ncb; ++b) t += Tpart[(size_t)b * S + s];
+    T[s] = t;
 }
 
 constexpr int kApplyRows = 8;    // rotation rows per workgroup (the block reads of k_sm_apply assume 8)
@@ -452,17 +477,6 @@ __global__ __launch_bounds__(256) void k_sm_apply(float *__restrict__ R, int64_t
         nnz[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = (double)(nzw[0] + nzw[1] + nzw[2] + nzw[3]);
 }
 
-// T_s = sum over column blocks of the partial row sums (deterministic order).
-__global__ void k_T_final(const double *__restrict__ Tpart, int ncb, int S, int Sp, double *__restrict__ T)
-{
-    const int s = blockIdx.x * 256 + threadIdx.x;
-    if (s >= Sp) return;
-    double t = 0.0;
-    if (s < S)
-        for (int b = 0; b < ncb; ++b) t += Tpart[(size_t)b * S + s];
-    T[s] = t;
-}
-
 }  // namespace
 
 // Partials layout inside c->part:  pm (float, nb*I) | ps (double, nb*I) | blk (double) | Tpart |
@@ -496,9 +510,12 @@ hipError_t launch_mark_p_dirty(const emc_ctx *c, hipStream_t st)
     return hipGetLastError();
 }
 
-hipError_t launch_sum_f64(const double *x, int n, double *out, hipStream_t st)
+hipError_t launch_sm_sums(const emc_ctx *c, const double *nz, int nnz, const double *blk, int nblk, const double *Tpart,
+                          int ncb, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_sum_f64, dim3(1), dim3(1024), 0, st, x, n, out);
+    const int nT = Tpart ? (c->Sp + 1023) / 1024 : 0;
+    hipLaunchKernelGGL(k_sm_sums, dim3(2 + nT), dim3(1024), 0, st, nz, nnz, blk, nblk, c->cst, c->I, Tpart, ncb, c->S, c->Sp,
+                       c->T, c->scal);
     return hipGetLastError();
 }
 
@@ -518,7 +535,6 @@ hipError_t launch_softmax(const emc_ctx *c, hipStream_t st)
     if (!fused)
         hipLaunchKernelGGL(k_sm_partial, dim3(ncol, nb), dim3(256), 0, st, c->R, (int64_t)c->Ip, S, I, rows, pm, ps);
     hipLaunchKernelGGL(k_sm_final, dim3(nfin), dim3(256), 0, st, pm, ps, nb, I, c->lse, blk, c->scal);
-    hipLaunchKernelGGL(k_sum_f64, dim3(1), dim3(1024), 0, st, blk, nfin, c->scal + SC_TOTAL);
     const int ncb = (I + kApplyCols - 1) / kApplyCols;
     const dim3 ga(ncb, (S + kApplyRows - 1) / kApplyRows);
     double *nzpart = Tpart + (int64_t)ncb * S;  // one non-zero count per apply workgroup
@@ -531,9 +547,7 @@ hipError_t launch_softmax(const emc_ctx *c, hipStream_t st)
         hipLaunchKernelGGL(k_sm_apply<0>, ga, dim3(256), 0, st, c->R, (int64_t)c->Ip, S, I, c->lse, nullptr, nullptr,
                            Tpart, nzpart, c->opt.scaling ? c->iphi : nullptr, c->pdirty, p_segments(c), nullptr, nullptr, 1,
                            1, 1, c->Pphi);
-    hipLaunchKernelGGL(k_T_final, dim3((c->Sp + 255) / 256), dim3(256), 0, st, Tpart, ncb, S, c->Sp, c->T);
-    hipLaunchKernelGGL(k_sum_f64, dim3(1), dim3(1024), 0, st, nzpart, (int)(ga.x * ga.y), c->scal + SC_NNZ);
-    return hipGetLastError();
+    return launch_sm_sums(c, nzpart, (int)(ga.x * ga.y), blk, nfin, Tpart, ncb, st);
 }
 
 }  // namespace emc
