@@ -217,8 +217,8 @@ class Engine:
 
     # outputs
     def get_model(self):
-        M = np.zeros(self.L ** 3, np.float32)
-        Wt = np.zeros(self.L ** 3, np.float32)
+        M = np.empty(self.L ** 3, np.float32)
+        Wt = np.empty(self.L ** 3, np.float32)
         self._c(lib().emc_get_model(self._h, M.ctypes.data_as(C.c_void_p), Wt.ctypes.data_as(C.c_void_p)))
         return M, Wt
 

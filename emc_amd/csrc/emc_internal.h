@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -18,6 +19,10 @@ constexpr int kPadI = 256;
 constexpr int kPadP = 128;
 // Partial sums of the model statistics (256 blocks x 4 values).
 constexpr int kRedLen = 1024;
+// emc_get_model's pinned slots: 512 KB each (a transfer of 10 us)
+constexpr int64_t kOutSlot = 1 << 17;
+constexpr int kOutSlots = 8;
+constexpr int64_t kReadOutThreaded = 4 << 20;
 
 inline int64_t round_up(int64_t a, int64_t b) { return (a + b - 1) / b * b; }
 
@@ -199,6 +204,10 @@ struct emc_ctx {
     float *U = nullptr;                                // [chunkp][Pp] (atomic insertion)
     double *scal = nullptr;                            // [SC_N] device scalars
     double *scal_h = nullptr;                          // pinned host mirror
+    float *out_h = nullptr;                            // kOutSlots pinned slots of out_slot floats (emc_get_model)
+    int64_t out_slot = 0;
+    std::mutex out_mutex;
+    hipEvent_t out_ev[emc::kOutSlots] = {};            // a slot's transfer has arrived
     // binned insertion: valid (s, j) pairs sorted by (chunk, model brick), cut into units of at most
     // bin_unit pairs; per unit a base-voxel permutation; partial halo bricks per block (consecutive units of a
     // brick, one workgroup) and, unless bin_direct, per group of blocks
@@ -225,6 +234,8 @@ namespace emc {
 // ---- launchers (each enqueues on `st`, returns hipError_t) --------------------------------
 hipError_t launch_rotmat(const float *q, const float *w, int S, int Sp, float *rotm, float *logw,
                          hipStream_t st);
+// n elements from position o on of a followed by b (N3 floats each) into pinned host memory.
+hipError_t launch_export(const float *a, const float *b, int64_t N3, int64_t o, int n, float *out, hipStream_t st);
 hipError_t launch_fill_f32(float *p, float v, int64_t n, hipStream_t st);
 hipError_t launch_fill_f64(double *p, double v, int64_t n, hipStream_t st);
 hipError_t launch_fill_i32(int32_t *p, int32_t v, int64_t n, hipStream_t st);

@@ -48,6 +48,16 @@ __global__ void k_fill(T *__restrict__ p, T v, int64_t n)
         p[i] = v;
 }
 
+// Bound by the host link; few workgroups reach its rate (32 as fast as 512).
+__global__ __launch_bounds__(256) void k_export(const float *__restrict__ a, const float *__restrict__ b, int64_t N3,
+                                                int64_t o, int n, float *__restrict__ out)
+{
+    for (int t = blockIdx.x * 256 + threadIdx.x; t < n; t += gridDim.x * 256) {
+        const int64_t k = o + t;
+        out[t] = k < N3 ? a[k] : b[k - N3];
+    }
+}
+
 // Per-rotation slice sum over V_s = {active j : W > 0}, |V_s|, and per pixel the workgroup's sum of
 // log W and number of rotations with a valid sample (colp[block][j] = (sum, count); summed over
 // the blocks in a fixed order by k_colsum_*, so the column sums are deterministic).
@@ -469,6 +479,12 @@ hipError_t launch_fill_i32(int32_t *p, int32_t v, int64_t n, hipStream_t st)
     if (n <= 0) return hipSuccess;
     const int64_t blocks = std::min<int64_t>((n + 255) / 256, 4096);
     hipLaunchKernelGGL(k_fill<int32_t>, dim3((unsigned)blocks), dim3(256), 0, st, p, v, n);
+    return hipGetLastError();
+}
+
+hipError_t launch_export(const float *a, const float *b, int64_t N3, int64_t o, int n, float *out, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_export, dim3(std::min((n + 255) / 256, 128)), dim3(256), 0, st, a, b, N3, o, n, out);
     return hipGetLastError();
 }
 
