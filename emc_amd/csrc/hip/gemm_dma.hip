@@ -2,8 +2,8 @@
 // path, global_load_lds_dwordx4): C[m, n] = sum_k sum_{a + b < max(NA, NB)} A_a[m, k] B_b[n, k] with NA and
 // NB BF16 terms per operand and FP32 accumulation.
 //
-// Tile 256 x BN (BN = 256 or 128), 8 wavefronts (4 along M x 2 along N), each a 64 x BN/2 block of
-// 2 x TN v_mfma_f32_32x32x16_bf16 tiles; BK = 32.  LDS rows are 64 B (32 BF16) without padding; the four
+// Tile 256 x BN (BN = 320, 256 or 128), 8 wavefronts (4 along M x 2 along N), each a 64 x BN/2 block of
+// 2 x TN v_mfma_f32_32x32x16_bf16 tiles; BK = 32; or 128 x 128, 4 wavefronts.  LDS rows are 64 B (32 BF16) without padding; the four
 // 16-byte chunks of row r sit at chunk ^ lds_swz(r), which spreads the fragment reads of 8 (or 16)
 // consecutive rows over distinct bank groups.  No register staging and no LDS store instructions.
 //
@@ -31,10 +31,11 @@ struct Cfg {
     static constexpr int OPA = BM * BK2 * 2, OPB = BN * BK2 * 2;  // bytes of one operand term per stage
     static constexpr int STAGE = NA * OPA + NB * OPB;
     // stages in LDS; the 128-row tiles run two workgroups per CU
-    static constexpr int ST = 3 * STAGE <= (WGM == 4 ? 147456 : 73728) ? 3 : 2;
-    static constexpr int LPW = STAGE / 1024 / (2 * WGM);            // DMA instructions per wave per step (16 rows each)
+    static constexpr int ST = 3 * STAGE <= (WGM == 4 ? 159744 : 73728) ? 3 : 2;
+    static constexpr int NG = STAGE / 1024;                         // DMA instructions per step (16 rows each)
+    static constexpr int LPW = (NG + 2 * WGM - 1) / (2 * WGM);      // per wave (the last ones may repeat one)
     static constexpr int NT = NA > NB ? NA : NB;                    // term pairs a + b < NT are multiplied
-    static_assert(STAGE % (2048 * WGM) == 0 && LPW < 16 && ST * STAGE <= 147456);
+    static_assert(STAGE % 1024 == 0 && LPW < 16 && ST * STAGE <= 159744);
 };
 
 template <int EPI, int NA, int NB, int WGM, int TN>
@@ -92,7 +93,7 @@ __global__ __launch_bounds__(128 * WGM) void k_dma(const bf16_t *__restrict__ A0
     const unsigned char *src[LPW];
 #pragma unroll
     for (int q = 0; q < LPW; ++q) {
-        const int g = wave * LPW + q;
+        const int g = min(wave * LPW + q, C::NG - 1);
         const bool isa = g < NA * (BM / 16);
         const int ga = g / (BM / 16), gb = (g - NA * (BM / 16)) / (BN / 16);
         const bf16_t *op = isa ? (ga == 0 ? A0 : ga == 1 ? A1 : A2) : (gb == 0 ? B0 : B1);
@@ -103,7 +104,7 @@ __global__ __launch_bounds__(128 * WGM) void k_dma(const bf16_t *__restrict__ A0
     auto issue = [&](int step, int stage) {
 #pragma unroll
         for (int q = 0; q < LPW; ++q) {
-            const int g = wave * LPW + q;
+            const int g = min(wave * LPW + q, C::NG - 1);
             lds_dma16(g < NA * (BM / 16) ? offA : offB, src[q] + (int64_t)step * (BK2 * 2), lds0 + stage * C::STAGE + g * 1024);
         }
     };
@@ -147,6 +148,7 @@ __global__ __launch_bounds__(128 * WGM) void k_dma(const bf16_t *__restrict__ A0
     };
 
     const int nk = Kd / BK2;
+    constexpr bool kOneFrag = NA + NB == 4 && TN == 5;  // two sets of fragments beside 160 accumulators do not fit
     Frag F0, F1;
     const float bv = EPI == EPI_LOGL && tid < BM && m0 + tid < e.m_valid ? e.bias[m0 + tid] : 0.0f;
     // running maxima of the tile's columns for the store skipping, read now (kept in LDS): a value
@@ -201,6 +203,24 @@ __global__ __launch_bounds__(128 * WGM) void k_dma(const bf16_t *__restrict__ A0
             // stage of step k: k % 2.  The barrier in step k follows this wave's wait for its loads of step
             // k + 1 (issued in step k - 1) and every wave's last fragment read of step k, so the loads
             // of step k + 2 may then overwrite its stage.
+            if constexpr (kOneFrag) {  // the other wavefront of the SIMD covers the fragment reads
+                for (int k = 0; k < nk; ++k) {
+                    if (LIVE) {
+                        mm(F0);
+                        rd(F0, k & 1, 16);
+                    }
+                    if (k + 1 < nk) {
+                        __builtin_amdgcn_s_waitcnt(kVm0);
+                        __syncthreads();
+                        if (k + 2 < nk) issue(k + 2, k & 1);
+                    }
+                    if (LIVE) {
+                        mm(F0);
+                        if (k + 1 < nk) rd(F0, (k + 1) & 1, 0);
+                    }
+                }
+                return;
+            }
             for (int k = 0; k < nk; ++k) {
                 if (LIVE) rd(F1, k & 1, 16);
                 __builtin_amdgcn_sched_barrier(0);
@@ -270,6 +290,9 @@ hipError_t pick(const Contraction &g, hipStream_t st)
 {
     switch (g.tile) {
     case kTile256: return launch<EPI, NA, NB, 4, 4>(g, st);
+    case kTile256x320:
+        if constexpr (NA == 2) return launch<EPI, NA, NB, 4, 5>(g, st);
+        break;
     case kTile256x128: return launch<EPI, NA, NB, 4, 2>(g, st);
     case kTile128: return launch<EPI, NA, NB, 2, 2>(g, st);
     case kTile64: break;
@@ -289,6 +312,9 @@ hipError_t pick(const Contraction &g, hipStream_t st)
 //   6,300 x 3,000   325/266/283/274   440/384/341/427   510/373/447/438
 //   6,300 x 4,000   435/392/381/296   605/527/490/450   679/517/622/459
 //   25,680 x 4,000  1713/1518/1377/1039
+// 256 x 320 tiles (two-term slices), against the best of the others, one-term then two-term counts:
+//   6,300 x 2,000 173/146 258/226   6,300 x 3,000 190/266 280/341   6,300 x 4,000 338/296 518/450
+//   10,860 x 4,000 544/460 801/705   25,680 x 4,000 1078/1039 1592/1798   6,300 x 3,001 (12,928 pixels) 689/1097 1073/1492
 // and at 32^3 (768 pixels) 3,240 x 1,000: 31/29/35/53, 33/37/43/74, 36/36/49/73; 1,380 x 500: 14/27/35/52.
 constexpr int64_t kSmallTiles = 56;  // up to this many 256 x 256 tiles' worth: 64 x 64 tiles
 GemmTile pick_tile(int64_t rows, int64_t cols, int na, int nb)
@@ -299,6 +325,8 @@ GemmTile pick_tile(int64_t rows, int64_t cols, int na, int nb)
     const double t256 = rounds(tiles(256, 256));
     const double t2x1 = rounds(tiles(256, 128)) * (nb == 2 ? 0.53 : na == 3 ? 0.71 : 0.65);
     const double t128 = std::max(0.66, (double)tiles(128, 128) / 512.0 * (na + nb == 4 ? 0.74 : 0.80));
+    const double t320 = na == 2 ? rounds(tiles(256, 320)) * (nb == 2 ? 1.16 : 1.27) : 1e9;
+    if (t320 < t256 && t320 < t2x1 && t320 < t128) return kTile256x320;
     return t256 <= t2x1 && t256 <= t128 ? kTile256 : t2x1 <= t128 ? kTile256x128 : kTile128;
 }
 

@@ -249,7 +249,7 @@ __device__ __forceinline__ void logl_epilogue(const f32x16 (&acc)[2][TN], const 
 // The contraction C [M][N] (row stride e.ldc) = sum over the term pairs (a, b), a + b < max(na, nb), of
 // A[a] [M][K] . B[b] [N][K]^T with FP32 accumulation (na <= 3 and nb <= 2 BF16 terms).  M is a multiple
 // of 256, N of 128, K of 128.
-enum GemmTile { kTile64, kTile128, kTile256x128, kTile256 };
+enum GemmTile { kTile64, kTile128, kTile256x128, kTile256, kTile256x320 };
 
 struct Contraction {
     GemmTile tile = kTile256;
