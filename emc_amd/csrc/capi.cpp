@@ -214,6 +214,9 @@ extern "C" void emc_destroy(emc_ctx *c)
         if (e) (void)hipEventDestroy(e);
     for (auto &e : c->gev)
         if (e) (void)hipEventDestroy(e);
+    if (c->fork_ev) (void)hipEventDestroy(c->fork_ev);
+    if (c->join_ev) (void)hipEventDestroy(c->join_ev);
+    if (c->side) (void)hipStreamDestroy(c->side);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }
@@ -278,6 +281,11 @@ extern "C" emc_status emc_create(const emc_dims *d, const emc_options *o, emc_ct
     if (st == EMC_OK) A(dalloc(&c->axyz, 3 * (int64_t)PpMax), "axyz");
     if (st == EMC_OK) A(dalloc(&c->pix, PpMax), "pix");
     if (st == EMC_OK) A(dalloc(&c->sumK, Ip), "sumK");
+    if (c->chi2_mfma) {
+        if (st == EMC_OK) A(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking), "side stream");
+        if (st == EMC_OK) A(hipEventCreateWithFlags(&c->fork_ev, hipEventDisableTiming), "event");
+        if (st == EMC_OK) A(hipEventCreateWithFlags(&c->join_ev, hipEventDisableTiming), "event");
+    }
     if (c->mfma) {
         if (st == EMC_OK) A(dalloc(&c->K16, Ip * PpMax), "K16");
         if (st == EMC_OK) A(dalloc(&c->KT16, Ip * PpMax), "KT16");
@@ -344,10 +352,14 @@ extern "C" emc_status emc_create(const emc_dims *d, const emc_options *o, emc_ct
     if (st == EMC_OK) A(dalloc(&c->T, Sp), "T");
     if (st == EMC_OK && !(c->mfma && opt.insert == EMC_INSERT_FUSED)) A(dalloc(&c->U, cp * PpMax), "U");
     if (st == EMC_OK) A(dalloc(&c->scal, SC_N), "scal");
+    // the side stream's queue comes to life with its first kernel (about 1 ms): here, not in the first pass
+    if (st == EMC_OK && c->side) A(launch_fill_f64(c->scal, 0.0, SC_N, c->side), "side stream");
     if (st == EMC_OK) A(hipHostMalloc((void **)&c->scal_h, sizeof(double) * SC_N, hipHostMallocDefault), "scal_h");
     c->out_slot = std::min<int64_t>(2 * N3, kOutSlot);
     if (st == EMC_OK)
         A(hipHostMalloc((void **)&c->out_h, sizeof(float) * c->out_slot * kOutSlots, hipHostMallocDefault), "out_h");
+    // its pages are mapped at the first touch (about 1 ms): here, not in the first emc_get_model
+    if (st == EMC_OK) std::memset(c->out_h, 0, sizeof(float) * c->out_slot * kOutSlots);
     for (auto &e : c->out_ev)
         if (st == EMC_OK) A(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event");
     if (st == EMC_OK) A(hipDeviceSynchronize(), "sync");  // every null-stream fill is done

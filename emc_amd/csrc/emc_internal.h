@@ -203,6 +203,8 @@ struct emc_ctx {
     double *T = nullptr;                               // [Sp]
     float *U = nullptr;                                // [chunkp][Pp] (atomic insertion)
     double *scal = nullptr;                            // [SC_N] device scalars
+    hipStream_t side = nullptr;                        // contractions that run beside the main stream's (the chi^2 kinds)
+    hipEvent_t fork_ev = nullptr, join_ev = nullptr;
     double *scal_h = nullptr;                          // pinned host mirror
     float *out_h = nullptr;                            // kOutSlots pinned slots of out_slot floats (emc_get_model)
     int64_t out_slot = 0;
@@ -395,5 +397,18 @@ __host__ __device__ inline float bf2f(bf16_t h) { return __builtin_bit_cast(floa
 // the two-element vector conversion, __builtin_convertvector(float2 -> __bf16 x 2), is lowered to one
 // instruction that converts the first element alone.
 __device__ inline bf16_t f2bf_dev(float x) { return __builtin_bit_cast(bf16_t, (__bf16)x); }
+
+// Work on c->side between the two runs beside st's and after everything st held at the fork.  Joined also
+// after an error: what the side stream holds uses the context's buffers.
+inline hipError_t fork_side(const emc_ctx *c, hipStream_t st)
+{
+    const hipError_t e = hipEventRecord(c->fork_ev, st);
+    return e != hipSuccess ? e : hipStreamWaitEvent(c->side, c->fork_ev, 0);
+}
+inline hipError_t join_side(const emc_ctx *c, hipStream_t st)
+{
+    const hipError_t e = hipEventRecord(c->join_ev, c->side);
+    return e != hipSuccess ? e : hipStreamWaitEvent(st, c->join_ev, 0);
+}
 
 }  // namespace emc

@@ -139,14 +139,21 @@ hipError_t launch_logl_chi2_mfma(const emc_ctx *c, int s0, int cs, hipStream_t s
     // one): the dropped product of the two lowest terms is below 2^-16 of the sum's terms.
     auto with_squares = [&](int p, int na, float *C) {
         return launch_gemm_store_mfma(c, na, op(p, 0), op(p, 1), na == 3 ? op(p, 2) : nullptr, c->k2_split ? 2 : 1,
-                                      c->K2h, c->K2l, nullptr, C, false, st);
+                                      c->K2h, c->K2l, nullptr, C, false, c->side);
     };
+    // The contractions do not depend on each other: those with the squares run on a second stream, so that the last,
+    // partly filled round of one is filled with tiles of the next (6,300 x 4,000 at 64^3: 400 tiles each, 1.56
+    // rounds of the chip).
     float *R = c->R + (size_t)s0 * c->Ip;
-    if (e == hipSuccess) e = with_counts(0, R);
-    if (e == hipSuccess) e = with_squares(1, NT, c->G2);
-    if (e == hipSuccess && scaling) e = with_squares(2, 1, c->G3);
-    if (e == hipSuccess && scaling) e = with_counts(3, c->G4);
+    if (e == hipSuccess) e = fork_side(c, st);
     if (e != hipSuccess) return e;
+    e = with_squares(1, NT, c->G2);
+    if (e == hipSuccess && scaling) e = with_squares(2, 1, c->G3);
+    hipError_t e2 = with_counts(0, R);
+    if (e2 == hipSuccess && scaling) e2 = with_counts(3, c->G4);
+    const hipError_t e3 = join_side(c, st);
+    for (hipError_t x : {e, e2, e3})
+        if (x != hipSuccess) return x;
     const int64_t n = (int64_t)cs * c->Ip;
     hipLaunchKernelGGL(k_chi2_combine, dim3(grid_for(n)), dim3(256), 0, st, R, c->G2, c->G3, c->G4, c->Aw,
                        c->bias + s0, c->rscale + s0, cs, c->I, (int64_t)c->Ip, scaling,
