@@ -205,7 +205,7 @@ extern "C" void emc_destroy(emc_ctx *c)
     dfree(c->Cx); dfree(c->K2h); dfree(c->K2l); dfree(c->Aw); dfree(c->G2); dfree(c->G3); dfree(c->G4);
     dfree(c->R); dfree(c->Ph); dfree(c->Pl); dfree(c->pdirty); dfree(c->runmax); dfree(c->blk); dfree(c->lse); dfree(c->part); dfree(c->red); dfree(c->T); dfree(c->U); dfree(c->scal);
     dfree(c->bin_vals); dfree(c->bin_perm); dfree(c->bin_vbeg); dfree(c->bin_frac); dfree(c->bin_units); dfree(c->bin_blocks); dfree(c->bin_groups);
-    dfree(c->bin_gbeg); dfree(c->bin_part); dfree(c->bin_gpart);
+    dfree(c->bin_gbeg); dfree(c->bin_part); dfree(c->bin_usum); dfree(c->bin_gpart);
     if (c->scal_h) (void)hipHostFree(c->scal_h);
     if (c->out_h) (void)hipHostFree(c->out_h);
     for (auto &e : c->out_ev)

@@ -211,21 +211,21 @@ struct emc_ctx {
     std::mutex out_mutex;
     hipEvent_t out_ev[emc::kOutSlots] = {};            // a slot's transfer has arrived
     // binned insertion: valid (s, j) pairs sorted by (chunk, model brick), cut into units of at most
-    // bin_unit pairs; per unit a base-voxel permutation; partial halo bricks per block (consecutive units of a
-    // brick, one workgroup) and, unless bin_direct, per group of blocks
-    int bin_unit = 0;
+    // 4,096 pairs; per unit a base-voxel permutation; partial halo bricks per block (up to four consecutive units
+    // of a brick) and, unless bin_direct, per group of blocks
     bool bin_direct = false;                           // every brick has few blocks: the last pass adds them itself
     uint32_t *bin_vals = nullptr;                      // [S * Pa] packed s << jbits | j, (s, j) order per brick
     uint16_t *bin_perm = nullptr;                      // [S * Pa] each pair's position in base-voxel order in its unit
     uint16_t *bin_vbeg = nullptr;                      // [n_units][520] start of each base voxel's run
-    float *bin_frac = nullptr;                         // [n_units][3][bin_unit] trilinear fractions (base-voxel order)
+    float *bin_frac = nullptr;                         // [n_units][3][4096] trilinear fractions (base-voxel order)
     int32_t *bin_units = nullptr;                      // [n_units][4] = key, begin, end, 0
-    int32_t *bin_blocks = nullptr;                     // [n_blocks][4] = key, first unit, end unit, 0 (one workgroup)
+    int32_t *bin_blocks = nullptr;                     // [n_blocks][4] = key, first unit, end unit, 0
     int32_t *bin_groups = nullptr;                     // [n_groups][4] = key, first block, end block (per chunk), 0
     int32_t *bin_gbeg = nullptr;                       // [chunks][bricks + 1] first group (bin_direct: block) of each brick
+    float *bin_usum = nullptr;                         // [units of a chunk][2][corners][512] unit sums (null: a workgroup per block)
     float *bin_part = nullptr;                         // [blocks of a chunk][2][9^3] block partials
     float *bin_gpart = nullptr;                        // [groups of a chunk][2][9^3] group partials
-    std::vector<int> bin_chunk_blocks, bin_chunk_groups; // block / group range of each rotation chunk
+    std::vector<int> bin_chunk_units, bin_chunk_blocks, bin_chunk_groups; // unit / block / group range of each rotation chunk
     bool bins_valid = false;
     // learned proposal (null when disabled)
     emc::Proposal *prop = nullptr;
@@ -298,8 +298,10 @@ hipError_t launch_mstep_sparse(const emc_ctx *c, int s0, int cs, const double *g
 
 // Responsibilities.  When logl_fuses_softmax(c), the logL contraction's epilogue writes the
 // per-band softmax partials (one band per logl_band_rows rotation rows: the contraction's tile, 256 or, for
-// smaller shapes, 128 or 64) and launch_softmax skips its pass.
+// smaller shapes, 128) and launch_softmax skips its pass.  64-row tiles leave the sums to k_sm_band, and with
+// two-term counts (no band maxima then) to the pass over every logit.
 bool logl_fuses_softmax(const emc_ctx *c);
+bool logl_band_pass(const emc_ctx *c);  // on 64-row tiles: the epilogue writes the maxima alone, k_sm_band the partials
 int logl_band_rows(const emc_ctx *c);
 int softmax_fused_bands(const emc_ctx *c);
 int softmax_fused_bands_max(const emc_ctx *c);  // over the pattern sets the context may be given (buffer sizes)

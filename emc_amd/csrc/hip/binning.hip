@@ -5,7 +5,7 @@
 // iteration.  Once per geometry the valid (rotation s, active pixel j) pairs are sorted by the
 // model brick (kBrick^3 voxels) that holds their base voxel, per rotation chunk, with a stable
 // radix sort (rocPRIM), so each brick lists its pairs in (s, j) order; each brick's list is cut
-// into units of at most c->bin_unit pairs, and inside a unit the pairs are ranked once more by base
+// into units of at most kUnit pairs, and inside a unit the pairs are ranked once more by base
 // voxel (a 16-bit permutation, the start of each base voxel's run, and for trilinear the pairs'
 // fractions in base-voxel order, laid out for coalesced reads).  Per pair the iteration then reads
 // 4 bytes of list (the packed pair), 2 of permutation and 12 of fractions.  Every iteration:
@@ -13,9 +13,10 @@
 //      consecutive pixels, and writes U and T_s into LDS at the pair's position in base-voxel order;
 //   2. every thread sums an equal share of the positions into per-base-voxel corner sums (the
 //      pieces of a voxel's run that crosses threads are added in thread order);
-//   3. a workgroup runs steps 1-2 for a few units of one brick in turn, then every
-//      voxel of the halo brick ((kBrick+1)^3) gathers the corner sums in a fixed order, and the
-//      halo brick is stored as the block's partial (no atomics);
+//   3. the corner sums of up to kUnitsPerBlock units of one brick (a block) are added in order, then every
+//      voxel of the halo brick ((kBrick+1)^3) gathers them in a fixed order, and the halo brick is stored as
+//      the block's partial (no atomics).  A workgroup takes a block's units in turn or, where the blocks
+//      are few, one unit each, and a pass over the blocks adds them: the same sums in the same order;
 //   4. a grouping pass sums the partials of up to kGroup consecutive blocks of one brick (left out where no brick
 //      has more than kDirect), and a last pass gives every model voxel the sum, in order, of the groups
 //      of the (at most 8) bricks whose halo covers it.
@@ -38,6 +39,9 @@ namespace {
 
 constexpr int kBrick = 8;
 constexpr int kBrick3 = kBrick * kBrick * kBrick;  // base voxels of a brick
+constexpr int kUnit = 4096;                        // pairs of a unit (positions fit 16 bits)
+constexpr int kUnitsPerBlock = 4;                  // units of a block
+constexpr int kSplitUnits = 1024;                  // up to this many units a chunk: one workgroup each
 constexpr int kVbeg = 520;                         // run starts per unit: kBrick3 + 1, padded to 16 bytes
 constexpr int kGroup = 32;                         // blocks whose partials one grouping workgroup sums
 constexpr int kDirect = 8;                         // up to this many blocks per brick: no grouping pass (a launch;
@@ -45,6 +49,7 @@ constexpr int kDirect = 8;                         // up to this many blocks per
 constexpr int kHalo = kBrick + 1;
 constexpr int kHalo3 = kHalo * kHalo * kHalo;      // voxels a brick's pairs reach
 constexpr int kThreads = 512;  // 8 waves; with 67 KB of LDS and 128 registers two workgroups (16 waves) fit a CU
+constexpr int kPer = kUnit / kThreads;  // positions per thread in step 2
 
 struct BinGeom {
     int L, nb, S, Pa, Pp, chunk, interp, jbits;
@@ -133,17 +138,17 @@ __global__ __launch_bounds__(kThreads) void k_unit_keys(const int32_t *__restric
 // Per unit: each pair's position in base-voxel order (a stable order, so (s, j) order within a base
 // voxel), stored at the pair's place in (s, j) order; the start of each base voxel's run
 // (kBrick3 + 1 entries); for trilinear, the fractions of the pair at base-voxel position k, stored
-// at frac[(u * 3 + axis) * unit + (k % per) * kThreads + k / per], where the insertion's thread
-// k / per reads them in step (k % per) of its share, all lanes of a wave on consecutive words.
+// at frac[(u * 3 + axis) * kUnit + (k % kPer) * kThreads + k / kPer], where the insertion's thread
+// k / kPer reads them in step (k % kPer) of its share, all lanes of a wave on consecutive words.
 __global__ __launch_bounds__(kThreads) void k_unit_perm(const int32_t *__restrict__ units,
                                                         const uint32_t *__restrict__ skeys,
                                                         const uint32_t *__restrict__ spos,
                                                         const uint32_t *__restrict__ vals,
                                                         const float *__restrict__ rotm, const float *__restrict__ axyz,
-                                                        BinGeom g, int per, uint16_t *__restrict__ inv,
+                                                        BinGeom g, uint16_t *__restrict__ inv,
                                                         uint16_t *__restrict__ vbeg, float *__restrict__ frac)
 {
-    const int u = blockIdx.x, unit = per * kThreads;
+    const int u = blockIdx.x;
     const int begin = units[4 * u + 1], end = units[4 * u + 2];
     for (int t = begin + threadIdx.x; t < end; t += kThreads) {
         const int k = t - begin;
@@ -153,7 +158,7 @@ __global__ __launch_bounds__(kThreads) void k_unit_perm(const int32_t *__restric
             float f[3];
             unpack(vals[spos[t]], g.jbits, s, j);
             item_cell(rotm, axyz, g, s, j, bx, by, bz, f[0], f[1], f[2]);
-            for (int a = 0; a < 3; ++a) frac[((size_t)u * 3 + a) * unit + (k % per) * kThreads + k / per] = f[a];
+            for (int a = 0; a < 3; ++a) frac[((size_t)u * 3 + a) * kUnit + (k % kPer) * kThreads + k / kPer] = f[a];
         }
     }
     for (int lv = threadIdx.x; lv <= kBrick3; lv += kThreads) {
@@ -170,30 +175,47 @@ __global__ __launch_bounds__(kThreads) void k_unit_perm(const int32_t *__restric
 
 // Steps 1-3 for one block: consecutive units of one brick, one after the other, whose corner sums accumulate in
 // LDS; the block's halo brick is stored as its partial
-// (part: [block - first block of the chunk][2][kHalo3], numerator then weight).
+// (part: [block - first block of the chunk][2][kHalo3], numerator then weight).  SPLIT: one unit (u0 + blockIdx.x)
+// a workgroup, whose corner sums are stored as they are for k_bin_units.
 // Step 1 writes U (or -1: skipped) and T_s into LDS at the pair's position in base-voxel order.  Step 2
-// gives every thread the same share of the unit, KPER consecutive positions, with the trilinear
+// gives every thread the same share of the unit, kPer consecutive positions, with the trilinear
 // fractions read from the precomputed coalesced planes (a thread per base voxel would wait on the
 // brick's heaviest voxel: at 64^3 / 25,680 the slowest thread of a unit would sum 2.5 times the
 // mean, up to 32 times).  A base voxel's run that crosses a thread boundary is summed piecewise: a
 // piece that continues into the next thread is handed over as a tail, and the thread holding the
 // run's last position adds the pieces in thread order.  Corner c = dx + 2 dy + 4 dz, weights
-// (1-f or f) per axis.  LDS layouts avoid bank conflicts: position k sits at k ^ ((k >> 6) % KPER) (a
-// thread's KPER positions are consecutive, so the 64 lanes of a read fall on 64 banks), the
+// (1-f or f) per axis.  LDS layouts avoid bank conflicts: position k sits at k ^ ((k >> 6) % kPer) (a
+// thread's kPer positions are consecutive, so the 64 lanes of a read fall on 64 banks), the
 // corner sums are corner-major, the tails value-major.
 //
 // What bounds it: memory, 22 bytes a pair with U, and the latency of list -> U, which the list read one unit ahead
 // halves.  64^3 / 25,680: 820 -> 607 us with that and the swizzle above (k ^ ((k >> 3) & 7) before, which left eight
 // lanes on each bank), 3.0 TB/s.  Forming the fractions here instead of reading them: 985 us (the vector units,
 // then); U, T and the fractions one unit ahead too: 17 to 31 registers spilled, 856 us.
-template <int KPER>
-__device__ __forceinline__ int rswz(int k)
+__device__ __forceinline__ int rswz(int k) { return k ^ ((k >> 6) & (kPer - 1)); }
+
+// The corner sums of a block -> its halo brick: each voxel adds those of the base voxels below it, in corner order.
+template <int NC>
+__device__ __forceinline__ void gather_halo(const float (*cM)[kBrick3], const float (*cW)[kBrick3], float *pM, float *pW)
 {
-    return k ^ ((k >> 6) & (KPER - 1));
+    for (int hv = threadIdx.x; hv < kHalo3; hv += kThreads) {
+        const int hx = hv % kHalo, hy = (hv / kHalo) % kHalo, hz = hv / (kHalo * kHalo);
+        float sm = 0.0f, sw = 0.0f;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const int bx = hx - (c & 1), by = hy - ((c >> 1) & 1), bz = hz - (c >> 2);
+            if (bx < 0 || by < 0 || bz < 0 || bx >= kBrick || by >= kBrick || bz >= kBrick) continue;
+            const int lb = (bz * kBrick + by) * kBrick + bx;
+            sm += cM[c][lb];
+            sw += cW[c][lb];
+        }
+        pM[hv] = sm;
+        pW[hv] = sw;
+    }
 }
 
-template <int INTERP, int KPER>
-__global__ __launch_bounds__(kThreads, 4) void k_insert_binned(const int32_t *__restrict__ blocks,
+template <int INTERP, bool SPLIT>
+__global__ __launch_bounds__(kThreads, 4) void k_insert_binned(const int32_t *__restrict__ blocks, int u0,
                                                                const int32_t *__restrict__ units,
                                                                const uint32_t *__restrict__ vals,
                                                                const uint16_t *__restrict__ inv,
@@ -204,7 +226,6 @@ __global__ __launch_bounds__(kThreads, 4) void k_insert_binned(const int32_t *__
                                                                float *__restrict__ part)
 {
     constexpr int NC = INTERP == EMC_INTERP_NEAREST ? 1 : 8;
-    constexpr int kUnit = kThreads * KPER;
     constexpr int kBuf = 2 * kUnit > 2 * NC * kThreads ? 2 * kUnit : 2 * NC * kThreads;
     __shared__ float buf[kBuf];  // a unit's U (-1: skipped) and T_s by base-voxel position, then the tails
     __shared__ uint16_t svb[kBrick3 + 1];
@@ -213,19 +234,19 @@ __global__ __launch_bounds__(kThreads, 4) void k_insert_binned(const int32_t *__
     float(*sv)[kUnit] = reinterpret_cast<float(*)[kUnit]>(buf);
     float(*tail)[kThreads] = reinterpret_cast<float(*)[kThreads]>(buf);  // [2 NC][kThreads]
     const int b = blockIdx.x;
-    const int ub = blocks[4 * b + 1], ue = blocks[4 * b + 2];
+    const int ub = SPLIT ? u0 + b : blocks[4 * b + 1], ue = SPLIT ? ub + 1 : blocks[4 * b + 2];
     const int tid = threadIdx.x;
     for (int k = tid; k < NC * kBrick3 / 4; k += kThreads) {
         reinterpret_cast<float4 *>(&cM[0][0])[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         reinterpret_cast<float4 *>(&cW[0][0])[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
     // the pairs of a unit, read one unit ahead (past the end of a unit: a valid pair, not stored)
-    uint32_t pv[KPER];
-    uint16_t pos[KPER];
+    uint32_t pv[kPer];
+    uint16_t pos[kPer];
     int begin = units[4 * ub + 1], n = units[4 * ub + 2] - begin;
     auto load_pairs = [&] {
 #pragma unroll
-        for (int q = 0; q < KPER; ++q) {
+        for (int q = 0; q < kPer; ++q) {
             const int k = begin + min(tid + q * kThreads, n - 1);
             pv[q] = vals[k];
             pos[q] = inv[k];
@@ -233,31 +254,31 @@ __global__ __launch_bounds__(kThreads, 4) void k_insert_binned(const int32_t *__
     };
     load_pairs();
     for (int u = ub; u < ue; ++u) {
-        const int k0 = tid * KPER, k1 = min(n, k0 + KPER);
+        const int k0 = tid * kPer, k1 = min(n, k0 + kPer);
         // 1. U and T_s by base-voxel position, from the pairs in (s, j) order
-        double Td[KPER];
-        float val[KPER];
+        double Td[kPer];
+        float val[kPer];
 #pragma unroll
-        for (int q = 0; q < KPER; ++q) {
+        for (int q = 0; q < kPer; ++q) {
             int s, j;
             unpack(pv[q], g.jbits, s, j);
             Td[q] = T[s];
             val[q] = U[(size_t)(s - s0) * g.Pp + j];
         }
         // this thread's fractions (used after the barriers)
-        float fr[KPER][3];
+        float fr[kPer][3];
         if constexpr (INTERP == EMC_INTERP_TRILINEAR) {
 #pragma unroll
-            for (int i = 0; i < KPER; ++i)
+            for (int i = 0; i < kPer; ++i)
 #pragma unroll
                 for (int a = 0; a < 3; ++a) fr[i][a] = frac[((size_t)u * 3 + a) * kUnit + i * kThreads + tid];
         }
         __syncthreads();  // the previous unit's tails and run starts are consumed
         for (int k = tid; k <= kBrick3; k += kThreads) svb[k] = vbeg[(size_t)u * kVbeg + k];
 #pragma unroll
-        for (int q = 0; q < KPER; ++q) {
+        for (int q = 0; q < kPer; ++q) {
             if (tid + q * kThreads >= n) break;
-            const int p = rswz<KPER>(pos[q]);
+            const int p = rswz(pos[q]);
             sv[0][p] = (Td[q] > 1e-10 && val[q] >= 0.0f) ? val[q] : -1.0f;  // emc_atomic.cu:190, :56
             sv[1][p] = (float)Td[q];
         }
@@ -303,14 +324,14 @@ __global__ __launch_bounds__(kThreads, 4) void k_insert_binned(const int32_t *__
             for (int c = 0; c < 2 * NC; ++c) acc[c] = 0.0f;
         };
 #pragma unroll
-        for (int i = 0; i < KPER; ++i) {
+        for (int i = 0; i < kPer; ++i) {
             const int k = k0 + i;
             if (k >= k1) break;
             if (k >= svb[lv + 1]) {
                 close_run(k);
                 while (svb[lv + 1] <= k) ++lv;  // skip base voxels without pairs
             }
-            const int p = rswz<KPER>(k);
+            const int p = rswz(k);
             const float v = sv[0][p];
             if (v < 0.0f) continue;
             const float Ts = sv[1][p];
@@ -352,22 +373,39 @@ __global__ __launch_bounds__(kThreads, 4) void k_insert_binned(const int32_t *__
         }
     }
     __syncthreads();
-    // 3. each halo voxel gathers the corner sums of the base voxels below it, in corner order
-    float *pM = part + (size_t)b * 2 * kHalo3, *pW = pM + kHalo3;
-    for (int hv = tid; hv < kHalo3; hv += kThreads) {
-        const int hx = hv % kHalo, hy = (hv / kHalo) % kHalo, hz = hv / (kHalo * kHalo);
-        float sm = 0.0f, sw = 0.0f;
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            const int bx = hx - (c & 1), by = hy - ((c >> 1) & 1), bz = hz - (c >> 2);
-            if (bx < 0 || by < 0 || bz < 0 || bx >= kBrick || by >= kBrick || bz >= kBrick) continue;
-            const int lb = (bz * kBrick + by) * kBrick + bx;
-            sm += cM[c][lb];
-            sw += cW[c][lb];
+    if constexpr (SPLIT) {  // the unit's corner sums, [2][NC][kBrick3]
+        float4 *out = reinterpret_cast<float4 *>(part + (size_t)b * 2 * NC * kBrick3);
+        for (int k = tid; k < NC * kBrick3 / 4; k += kThreads) {
+            out[k] = reinterpret_cast<const float4 *>(&cM[0][0])[k];
+            out[NC * kBrick3 / 4 + k] = reinterpret_cast<const float4 *>(&cW[0][0])[k];
         }
-        pM[hv] = sm;
-        pW[hv] = sw;
+    } else {
+        gather_halo<NC>(cM, cW, part + (size_t)b * 2 * kHalo3, part + (size_t)b * 2 * kHalo3 + kHalo3);
     }
+}
+
+// Step 3 where every unit had a workgroup of its own: the block's units [ub, ue) added in order, then its halo brick.
+template <int NC>
+__global__ __launch_bounds__(kThreads) void k_bin_units(const int32_t *__restrict__ blocks, int u0,
+                                                        const float *__restrict__ usum, float *__restrict__ part)
+{
+    __shared__ __attribute__((aligned(16))) float cs[2][NC][kBrick3];
+    const int b = blockIdx.x, ub = blocks[4 * b + 1] - u0, nu = blocks[4 * b + 2] - u0 - ub;
+    constexpr int kQuads = 2 * NC * kBrick3 / 4;
+    const float4 *in = reinterpret_cast<const float4 *>(usum) + (size_t)ub * kQuads;
+#pragma unroll 4
+    for (int k = threadIdx.x; k < kQuads; k += kThreads) {
+        float4 v[kUnitsPerBlock];
+#pragma unroll
+        for (int u = 0; u < kUnitsPerBlock; ++u) v[u] = in[(size_t)min(u, nu - 1) * kQuads + k];
+        float4 a = v[0];
+#pragma unroll
+        for (int u = 1; u < kUnitsPerBlock; ++u)
+            if (u < nu) a = make_float4(a.x + v[u].x, a.y + v[u].y, a.z + v[u].z, a.w + v[u].w);
+        reinterpret_cast<float4 *>(&cs[0][0][0])[k] = a;
+    }
+    __syncthreads();
+    gather_halo<NC>(cs[0], cs[1], part + (size_t)b * 2 * kHalo3, part + (size_t)b * 2 * kHalo3 + kHalo3);
 }
 
 // Step 4a: group g sums the partials of its blocks [gu0, gu1) (consecutive blocks of one brick), in
@@ -401,7 +439,7 @@ __global__ __launch_bounds__(kThreads) void k_bin_group(const int32_t *__restric
 __global__ __launch_bounds__(kThreads) void k_insert_reduce(const float *__restrict__ gpart,
                                                             const int32_t *__restrict__ gbeg, BinGeom g,
                                                             float *__restrict__ Mnum, float *__restrict__ Wt,
-                                                            bool first)
+                                                            bool first, bool direct)
 {
     const int64_t v = blockIdx.x * (int64_t)kThreads + threadIdx.x;
     const int L = g.L;
@@ -418,6 +456,8 @@ __global__ __launch_bounds__(kThreads) void k_insert_reduce(const float *__restr
                 const int hv = ((dz ? kBrick : lz) * kHalo + (dy ? kBrick : ly)) * kHalo + (dx ? kBrick : lx);
                 const int g1 = gbeg[key + 1];
                 int gi = gbeg[key];
+                float bm = 0.0f, bw = 0.0f;  // blocks of one brick first, as the grouping pass adds them
+                float &am = direct ? bm : sm, &aw = direct ? bw : sw;
                 for (; gi + 4 <= g1; gi += 4) {  // independent loads, added in order
                     float a[4], w[4];
 #pragma unroll
@@ -427,13 +467,17 @@ __global__ __launch_bounds__(kThreads) void k_insert_reduce(const float *__restr
                     }
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
-                        sm += a[q];
-                        sw += w[q];
+                        am += a[q];
+                        aw += w[q];
                     }
                 }
                 for (; gi < g1; ++gi) {
-                    sm += gpart[(size_t)gi * 2 * kHalo3 + hv];
-                    sw += gpart[(size_t)gi * 2 * kHalo3 + kHalo3 + hv];
+                    am += gpart[(size_t)gi * 2 * kHalo3 + hv];
+                    aw += gpart[(size_t)gi * 2 * kHalo3 + kHalo3 + hv];
+                }
+                if (direct) {
+                    sm += bm;
+                    sw += bw;
                 }
             }
     if (first) {  // the pass's first rotation chunk: the sums start here (no separate zero fill)
@@ -477,17 +521,7 @@ hipError_t build_bins(emc_ctx *c, std::string &err)
     const int nch = (c->S + c->chunk - 1) / c->chunk;
     const uint32_t nbr = (uint32_t)g.nb * g.nb * g.nb;
     const uint32_t nkeys = (uint32_t)nch * nbr;
-    // Unit size and units per workgroup, from the pairs of a chunk (longer workgroups write fewer partial halo
-    // bricks of 5.8 KB, shorter ones fill the chip's 512 workgroup slots).  Insertion and its two reductions, us,
-    // at 2,048 x 1 / 4,096 x 2 / 4,096 x 4 pairs a workgroup: 0.17M pairs (24^3 / 420 rotations) 27 / 36 / 44,
-    // 1.5M (45^3 nearest, 1,000) 30 / 38 / 41, 2.4M (32^3 / 3,240) 56 / 51 / 69, 20M (64^3 / 6,300) 241 / 185 / 190,
-    // 82M (64^3 / 25,680) 953 / 648 / 633 and (128^3 / 6,300) 913 / 668 / 662.
-    const int64_t pairs = (int64_t)std::min(c->chunk, c->S) * c->Pa;
-    // (the unit keys have 32 bits: with very many bricks over all chunks the fewest units)
-    const bool small = pairs < (2 << 20) && nkeys < (1u << 22);
-    const int kUnit = c->bin_unit = small ? 2048 : 4096;
-    const int kUnitsPerBlock = small ? 1 : pairs < (32 << 20) ? 2 : 4;
-    int max_brick_blocks = 0;
+    int max_brick_blocks = 0, max_units = 0;
     int end_bit = 1;
     while (end_bit < 32 && ((uint64_t)1 << end_bit) <= nkeys) ++end_bit;
     uint32_t *kin = nullptr, *vin = nullptr, *kout = nullptr, *pout = nullptr;
@@ -511,6 +545,7 @@ hipError_t build_bins(emc_ctx *c, std::string &err)
     release(c->bin_groups);
     release(c->bin_gbeg);
     release(c->bin_part);
+    release(c->bin_usum);
     release(c->bin_gpart);
     chk(hipMalloc((void **)&kin, sizeof(uint32_t) * n));
     chk(hipMalloc((void **)&vin, sizeof(uint32_t) * n));
@@ -542,6 +577,7 @@ hipError_t build_bins(emc_ctx *c, std::string &err)
     // brick's first group in gbeg
     std::vector<int32_t> units, blocks, groups, gbeg, bbeg;  // bbeg: each brick's first block
     c->bin_chunk_blocks.assign(nch + 1, 0);
+    c->bin_chunk_units.assign(nch + 1, 0);
     c->bin_chunk_groups.assign(nch + 1, 0);
     int max_blocks = 0, max_groups = 0;
     for (int ch = 0; ch < nch && e == hipSuccess; ++ch) {
@@ -579,11 +615,14 @@ hipError_t build_bins(emc_ctx *c, std::string &err)
         bbeg.push_back((int32_t)(blocks.size() / 4) - b_first);
         c->bin_chunk_blocks[ch + 1] = (int)(blocks.size() / 4);
         c->bin_chunk_groups[ch + 1] = (int)(groups.size() / 4);
+        c->bin_chunk_units[ch + 1] = (int)(units.size() / 4);
+        max_units = std::max(max_units, c->bin_chunk_units[ch + 1] - c->bin_chunk_units[ch]);
         max_blocks = std::max(max_blocks, c->bin_chunk_blocks[ch + 1] - c->bin_chunk_blocks[ch]);
         max_groups = std::max(max_groups, c->bin_chunk_groups[ch + 1] - c->bin_chunk_groups[ch]);
     }
     const uint32_t n_units = (uint32_t)(units.size() / 4);
     c->bin_direct = max_brick_blocks <= kDirect;
+    const bool split = max_units <= kSplitUnits;
     if (c->bin_direct) gbeg = bbeg;
     if (e == hipSuccess && n_units > 0) {
         chk(hipMalloc((void **)&c->bin_units, sizeof(int32_t) * units.size()));
@@ -591,6 +630,9 @@ hipError_t build_bins(emc_ctx *c, std::string &err)
         chk(hipMalloc((void **)&c->bin_groups, sizeof(int32_t) * groups.size()));
         chk(hipMalloc((void **)&c->bin_gbeg, sizeof(int32_t) * gbeg.size()));
         chk(hipMalloc((void **)&c->bin_part, sizeof(float) * 2 * kHalo3 * (size_t)max_blocks));
+        if (split)
+            chk(hipMalloc((void **)&c->bin_usum,
+                          sizeof(float) * 2 * kBrick3 * (c->opt.interp == EMC_INTERP_NEAREST ? 1 : 8) * (size_t)max_units));
         if (!c->bin_direct) chk(hipMalloc((void **)&c->bin_gpart, sizeof(float) * 2 * kHalo3 * (size_t)max_groups));
         chk(hipMalloc((void **)&c->bin_perm, sizeof(uint16_t) * n));
         chk(hipMalloc((void **)&c->bin_vbeg, sizeof(uint16_t) * kVbeg * (size_t)n_units));
@@ -634,7 +676,7 @@ hipError_t build_bins(emc_ctx *c, std::string &err)
             chk(rocprim::radix_sort_pairs(tmp, tmp_bytes, kin, kout, vin, pout, (size_t)n, 0, end_bit2, st));
         if (e == hipSuccess) {
             hipLaunchKernelGGL(k_unit_perm, dim3(n_units), dim3(kThreads), 0, st, c->bin_units, kout, pout, c->bin_vals,
-                               c->rotm, c->axyz, g, kUnit / kThreads, c->bin_perm, c->bin_vbeg, c->bin_frac);
+                               c->rotm, c->axyz, g, c->bin_perm, c->bin_vbeg, c->bin_frac);
             chk(hipGetLastError());
         }
         if (e == hipSuccess) chk(hipStreamSynchronize(st));
@@ -664,22 +706,31 @@ hipError_t launch_insert_binned(const emc_ctx *c, int s0, int cs, hipStream_t st
     }
     const BinGeom g = geom_of(c);
     const int32_t *blocks = c->bin_blocks + 4 * (size_t)b0;
+    const int u0 = c->bin_chunk_units[k], nu = c->bin_chunk_units[k + 1] - u0;
+    const bool split = c->bin_usum != nullptr, nearest = c->opt.interp == EMC_INTERP_NEAREST;
     const auto run = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(b1 - b0), dim3(kThreads), 0, st, blocks, c->bin_units, c->bin_vals, c->bin_perm,
-                           c->bin_vbeg, c->bin_frac, c->U, s0, c->T, g, c->bin_part);
+        hipLaunchKernelGGL(kernel, dim3(split ? nu : b1 - b0), dim3(kThreads), 0, st, blocks, u0, c->bin_units, c->bin_vals,
+                           c->bin_perm, c->bin_vbeg, c->bin_frac, c->U, s0, c->T, g, split ? c->bin_usum : c->bin_part);
     };
-    const bool small = c->bin_unit == 2048;
-    if (c->opt.interp == EMC_INTERP_NEAREST)
-        run(small ? k_insert_binned<EMC_INTERP_NEAREST, 4> : k_insert_binned<EMC_INTERP_NEAREST, 8>);
-    else
-        run(small ? k_insert_binned<EMC_INTERP_TRILINEAR, 4> : k_insert_binned<EMC_INTERP_TRILINEAR, 8>);
+    const auto add_units = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(b1 - b0), dim3(kThreads), 0, st, blocks, u0, c->bin_usum, c->bin_part);
+    };
+    if (split && nearest) {
+        run(k_insert_binned<EMC_INTERP_NEAREST, true>);
+        add_units(k_bin_units<1>);
+    } else if (split) {
+        run(k_insert_binned<EMC_INTERP_TRILINEAR, true>);
+        add_units(k_bin_units<8>);
+    } else {
+        run(nearest ? k_insert_binned<EMC_INTERP_NEAREST, false> : k_insert_binned<EMC_INTERP_TRILINEAR, false>);
+    }
     if (!c->bin_direct)
         hipLaunchKernelGGL(k_bin_group, dim3(g1 - g0), dim3(kThreads), 0, st, c->bin_groups + 4 * (size_t)g0, c->bin_part,
                            c->bin_gpart);
     const int nbr = g.nb * g.nb * g.nb;
     hipLaunchKernelGGL(k_insert_reduce, dim3((unsigned)((c->N3 + kThreads - 1) / kThreads)), dim3(kThreads), 0, st,
                        c->bin_direct ? c->bin_part : c->bin_gpart, c->bin_gbeg + (size_t)k * (nbr + 1), g, c->Mnum,
-                       c->Wt, k == 0);
+                       c->Wt, k == 0, c->bin_direct);
     return hipGetLastError();
 }
 

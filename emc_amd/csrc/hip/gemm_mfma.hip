@@ -427,7 +427,12 @@ static GemmTile logl_tile(const emc_ctx *c) { return pick_tile(c->chunkp, c->Ip,
 
 int logl_band_rows(const emc_ctx *c) { return tile_rows_of(logl_tile(c)); }
 
-bool logl_fuses_softmax(const emc_ctx *c) { return c->mfma && !c->chi2_mfma && c->opt.mfma_tile == 0; }
+bool logl_band_pass(const emc_ctx *c) { return logl_tile(c) == kTile64; }
+
+bool logl_fuses_softmax(const emc_ctx *c)
+{
+    return c->mfma && !c->chi2_mfma && c->opt.mfma_tile == 0 && !(c->k_split && logl_band_pass(c));
+}
 
 static int bands_of(const emc_ctx *c, int band_rows)
 {
@@ -481,7 +486,7 @@ hipError_t launch_logl_mfma(const emc_ctx *c, int s0, int cs, hipStream_t st)
     e.bias = c->bias + s0;
     const bf16_t *A1 = c->la_terms == 3 ? c->Lm : c->Ll;
     const bf16_t *A2 = c->Ll;
-    if (!logl_fuses_softmax(c)) {  // options.mfma_tile = 1
+    if (c->opt.mfma_tile != 0) {
         const dim3 grid(c->Ip / BN, c->chunkp / BM);
         if (c->la_terms == 3) {
             if (c->k_split) return run<3, 2, EPI_LOGL>(grid, st, c->Lh, A1, A2, c->Pp, c->K16, c->K16lo, c->Pp, c->Pp, e);
@@ -491,9 +496,10 @@ hipError_t launch_logl_mfma(const emc_ctx *c, int s0, int cs, hipStream_t st)
         return run<2, 1, EPI_LOGL>(grid, st, c->Lh, A1, nullptr, c->Pp, c->K16, nullptr, c->Pp, c->Pp, e);
     }
     // band partials in c->part: pm (floats) [bands][I] then ps (doubles) [bands][I]
-    const int64_t nb = softmax_fused_bands(c);
-    e.pm = reinterpret_cast<float *>(c->part);
-    e.ps = c->part + nb * c->I;
+    if (logl_fuses_softmax(c)) {
+        e.pm = reinterpret_cast<float *>(c->part);
+        e.ps = c->part + (int64_t)softmax_fused_bands(c) * c->I;
+    }
     e.band0 = (int64_t)(s0 / c->chunk) * (c->chunkp / logl_band_rows(c));
     e.ldp = c->I;
     if (logl_skips_stores(c)) {
@@ -536,6 +542,7 @@ hipError_t launch_gemm_store_mfma(const emc_ctx *c, int na, const bf16_t *A0, co
     g.e.m_valid = c->chunkp;
     g.e.n_valid = c->Ip;
     g.e.accumulate = accumulate;
+    g.two_sums = true;
     g.tile = pick_tile(c->chunkp, c->Ip, na, nb);
     if (g.tile >= kTile256x128 && c->opt.mfma_staging == 1 && nb == 1)
         return run_large<EPI_STORE>(c->chunkp, c->Ip, st, na, A0, A1, A2, c->Pp, B0, B8, c->Pp, c->Pp, g.e);

@@ -16,7 +16,9 @@ namespace {
 constexpr int SM = 64, SN = 64, SK = 64;
 constexpr int kTerm = 64 * SK * 2;  // LDS bytes of one operand term per stage
 
-template <int EPI, int NA, int NB>
+// TWO: the products with B[0] and with B[1] are summed apart and added at the end, as two launches of the large
+// tiles' store epilogue would (the second adding to the first).
+template <int EPI, int NA, int NB, bool TWO>
 __global__ __launch_bounds__(256) void k_small(const bf16_t *__restrict__ A0, const bf16_t *__restrict__ A1,
                                                const bf16_t *__restrict__ A2, int64_t lda,
                                                const bf16_t *__restrict__ B0, const bf16_t *__restrict__ B1,
@@ -25,16 +27,13 @@ __global__ __launch_bounds__(256) void k_small(const bf16_t *__restrict__ A0, co
     if (e.gate && *e.gate <= e.gate_thr) return;  // the sparse M-step runs instead
     constexpr int NT = NA > NB ? NA : NB;         // term pairs a + b < NT are multiplied
     __shared__ float red[4][32];
-    __shared__ double reds[4][32];
     __shared__ uint32_t kept_s[2];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int m0 = blockIdx.y * SM, n0 = blockIdx.x * SN;
     if (n0 >= e.n_valid) return;  // a tile of padding (never read)
     if (m0 >= e.m_valid) {
-        if (EPI == EPI_LOGL && wave == 0 && n0 + lane < e.n_valid) {  // the final softmax pass reads every band
+        if (EPI == EPI_LOGL && e.pm && wave == 0 && n0 + lane < e.n_valid)  // k_sm_band reads every group's
             e.pm[(e.band0 + m0 / SM) * e.ldp + n0 + lane] = -1.0e10f;
-            e.ps[(e.band0 + m0 / SM) * e.ldp + n0 + lane] = 0.0;
-        }
         return;
     }
     const int fr = lane & 31, fh = lane >> 5;
@@ -71,9 +70,9 @@ __global__ __launch_bounds__(256) void k_small(const bf16_t *__restrict__ A0, co
                       lds0 + stage * STAGE + g * 1024);
         }
     };
-    f32x16 acc;
+    f32x16 acc, acc1;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+    for (int r = 0; r < 16; ++r) acc[r] = acc1[r] = 0.0f;
     const int sw = (fr >> 1) & 7;
     auto step_mm = [&](int stage) {
         const unsigned char *S = smem + stage * STAGE;
@@ -93,7 +92,10 @@ __global__ __launch_bounds__(256) void k_small(const bf16_t *__restrict__ A0, co
             for (int a = NA - 1; a >= 0; --a)
 #pragma unroll
                 for (int b = NB - 1; b >= 0; --b)
-                    if (a + b < NT) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[a][t], fb[b][t], acc, 0, 0, 0);
+                    if (a + b < NT) {
+                        f32x16 &to = TWO && b == 1 ? acc1 : acc;
+                        to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[a][t], fb[b][t], to, 0, 0, 0);
+                    }
     };
     // step k is in stage k % kST.  Past the last step the loads fetch it again (into a stage nothing reads),
     // so the number of loads in flight is the same in every step.
@@ -109,6 +111,9 @@ __global__ __launch_bounds__(256) void k_small(const bf16_t *__restrict__ A0, co
         st = st + 1 == kST ? 0 : st + 1;
     }
     __builtin_amdgcn_s_waitcnt(kVm0);  // no load is left to write LDS
+    if constexpr (TWO)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[r] += acc1[r];
 
     // accumulator layout: lane holds column lane % 32, rows 8*(r/4) + 4*(lane/32) + r%4, r = 0..15
     const int n = nw + fr;
@@ -123,44 +128,40 @@ __global__ __launch_bounds__(256) void k_small(const bf16_t *__restrict__ A0, co
         }
         return;
     }
-    // logL: the bias, the band's softmax partials (a band = the tile's 64 rows) and the store skipping, by
-    // the rules of the 256-row kernels' epilogue (every logit that is stored is stored in place)
-    float mx = -1.0e10f;
+    // logL: the bias, the maxima of the tile's 64 rows (e.pm; k_sm_band forms the sums, from the stored logits) and
+    // the store skipping by the rules of the 256-row kernels' epilogue (every logit that is stored is stored in place)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const int m = mw + 8 * (r >> 2) + 4 * fh + (r & 3);
         acc[r] = m < e.m_valid ? acc[r] + e.bias[m] : -INFINITY;
-        mx = fmaxf(mx, acc[r]);
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    if (lane < 32) red[wave][lane] = mx;
-    __syncthreads();
-    mx = fmaxf(red[wave & 1][fr], red[2 + (wave & 1)][fr]);
-    constexpr float kLog2e = 1.4426950408889634f;
-    float fs = 0.0f;
+    bool kept = true;
+    if (e.pm) {
+        float mx = -1.0e10f;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) fs += __builtin_amdgcn_exp2f(fmaxf(acc[r] - mx, -1.0e10f) * kLog2e);
-    double ds = (double)fs;
-    ds += __shfl_xor(ds, 32, 64);
-    if (lane < 32) reds[wave][lane] = ds;
-    if (wave < 2) {  // the upper wavefronts read the running maxima: the lower ones take their choice
-        const bool keep = !(e.runmax && nok && (double)mx < (double)float_of_ord(e.runmax[n]) - kSkipStoreNats);
-        const uint64_t kb = __ballot(keep);
-        if (lane == 0) kept_s[wave] = (uint32_t)kb;
-    }
-    __syncthreads();
-    const uint32_t kept_m = kept_s[wave & 1];
-    const bool kept = (kept_m >> fr) & 1u;
-    const int64_t orow = (e.band0 + m0 / SM) * e.ldp;
-    if (wave < 2 && lane < 32 && nok) {
-        e.pm[orow + n] = mx;
-        e.ps[orow + n] = reds[wave][lane] + reds[2 + wave][lane];
-        if (e.blk) e.blk[orow + n] = (int16_t)(kept ? -2 : -1);
-        if (e.runmax && mx == mx) atomicMax(e.runmax + n, ord_of(mx));
-    }
-    if (e.runmax && wave < 2) {
-        const int cnt = __popc(~kept_m & (uint32_t)__ballot(nok));
-        if (lane == 0 && cnt > 0) atomicAdd(e.skipped, (double)cnt);
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, acc[r]);
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        if (lane < 32) red[wave][lane] = mx;
+        __syncthreads();
+        mx = fmaxf(red[wave & 1][fr], red[2 + (wave & 1)][fr]);
+        if (wave < 2) {  // the upper wavefronts read the running maxima: the lower ones take their choice
+            const bool keep = !(e.runmax && nok && (double)mx < (double)float_of_ord(e.runmax[n]) - kSkipStoreNats);
+            const uint64_t kb = __ballot(keep);
+            if (lane == 0) kept_s[wave] = (uint32_t)kb;
+        }
+        __syncthreads();
+        const uint32_t kept_m = kept_s[wave & 1];
+        kept = (kept_m >> fr) & 1u;
+        const int64_t orow = (e.band0 + m0 / SM) * e.ldp;
+        if (wave < 2 && lane < 32 && nok) {
+            e.pm[orow + n] = mx;
+            if (e.blk) e.blk[orow + n] = (int16_t)(kept ? -2 : -1);
+            if (e.runmax && mx == mx) atomicMax(e.runmax + n, ord_of(mx));
+        }
+        if (e.runmax && wave < 2) {
+            const int cnt = __popc(~kept_m & (uint32_t)__ballot(nok));
+            if (lane == 0 && cnt > 0) atomicAdd(e.skipped, (double)cnt);
+        }
     }
     if (kept && nok)
 #pragma unroll
@@ -170,10 +171,10 @@ __global__ __launch_bounds__(256) void k_small(const bf16_t *__restrict__ A0, co
         }
 }
 
-template <int EPI, int NA, int NB>
+template <int EPI, int NA, int NB, bool TWO = false>
 hipError_t launch(const Contraction &g, hipStream_t st)
 {
-    hipLaunchKernelGGL((k_small<EPI, NA, NB>), dim3((g.N + SN - 1) / SN, g.M / SM), dim3(256), 0, st, g.A[0], g.A[1],
+    hipLaunchKernelGGL((k_small<EPI, NA, NB, TWO>), dim3((g.N + SN - 1) / SN, g.M / SM), dim3(256), 0, st, g.A[0], g.A[1],
                        g.A[2], g.lda, g.B[0], g.B[1], g.ldb, g.K, g.e);
     return hipGetLastError();
 }
@@ -189,6 +190,10 @@ hipError_t run_small(int epi, const Contraction &g, hipStream_t st)
         if (k == 10) return launch<EPI_LOGL, 2, 2>(g, st);
         if (k == 13) return launch<EPI_LOGL, 3, 1>(g, st);
         if (k == 14) return launch<EPI_LOGL, 3, 2>(g, st);
+    } else if (g.two_sums && g.nb == 2) {
+        if (g.na == 1) return launch<EPI_STORE, 1, 2, true>(g, st);
+        if (g.na == 2) return launch<EPI_STORE, 2, 2, true>(g, st);
+        if (g.na == 3) return launch<EPI_STORE, 3, 2, true>(g, st);
     } else {
         if (k == 5) return launch<EPI_STORE, 1, 1>(g, st);
         if (k == 6) return launch<EPI_STORE, 1, 2>(g, st);

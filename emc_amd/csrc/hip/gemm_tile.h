@@ -257,10 +257,11 @@ struct Contraction {
     const bf16_t *A[3] = {nullptr, nullptr, nullptr}, *B[2] = {nullptr, nullptr};
     int64_t lda = 0, ldb = 0;
     int M = 0, N = 0, K = 0;
+    bool two_sums = false;  // kTile64 with nb = 2: the products of the two B terms summed apart, then added
     EpiArgs e{};
 };
 
-// Tile for a contraction of this many rows, columns and terms, and its rows (a softmax band of the logL epilogue).
+// Tile for a contraction of this many rows, columns and terms, and its rows (the logL epilogue's maxima are over these).
 GemmTile pick_tile(int64_t rows, int64_t cols, int na, int nb);
 inline int tile_rows_of(GemmTile t) { return t == kTile64 ? 64 : t == kTile128 ? 128 : 256; }
 // epi: EPI_LOGL or EPI_STORE.  run_small: kTile64, every (na, nb); run_dma: the others, the pairs dma_takes names.

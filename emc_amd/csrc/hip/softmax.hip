@@ -24,6 +24,47 @@ __device__ __forceinline__ T wave_sum(T v)
     return v;
 }
 
+// Partials of the 256-row bands where the logL ran on 64-row tiles, whose epilogue wrote the maxima of the 64-row
+// groups (gm, [4 groups per band][I]): the sums of exp(R - max) in the order and arithmetic of the 256-row
+// kernels' epilogue (32 rows of a column in FP32, on the hardware exp2, the pairs and the groups of 64 rows in
+// FP64), so the partials do not depend on the tile.  A group whose logits were left out (gblk, null: none) adds
+// nothing: its terms are below exp(-128) of the pattern's sum.  Bands count from each chunk's first rotation.
+// One workgroup takes 32 columns, a thread 32 rows of one (a launch of 5 us; reading 0.1 to 15 MB).
+__global__ __launch_bounds__(256) void k_sm_band(const float *__restrict__ R, int64_t ldr, int S, int I, int chunk, int bpc,
+                                                 const float *__restrict__ gm, const int16_t *__restrict__ gblk,
+                                                 float *__restrict__ pm, double *__restrict__ ps)
+{
+    __shared__ double red[4][32];
+    constexpr float kLog2e = 1.4426950408889634f;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, hr = 4 * (lane >> 5);
+    const int band = blockIdx.y, i = blockIdx.x * 32 + (lane & 31), ic = min(i, I - 1);
+    const int l0 = (band % bpc) * 256 + 64 * w, s0 = (band / bpc) * chunk + l0;  // this wave's group of 64 rows
+    const int rows = min(min(chunk, S - (band / bpc) * chunk) - l0, 64);
+    float mx = -1.0e10f;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) mx = fmaxf(mx, gm[(size_t)(4 * band + g) * I + ic]);
+    float fs = 0.0f;
+    if (rows > 0 && !(gblk && gblk[(size_t)(4 * band + w) * I + ic] == -1)) {
+        float v[32];
+#pragma unroll
+        for (int k = 0; k < 32; ++k) {
+            const int r = 32 * (k >> 4) + 8 * ((k >> 2) & 3) + (k & 3) + hr;
+            v[k] = R[(size_t)(s0 + min(r, rows - 1)) * ldr + ic];
+            if (r >= rows) v[k] = -INFINITY;
+        }
+#pragma unroll
+        for (int k = 0; k < 32; ++k) fs += __builtin_amdgcn_exp2f(fmaxf(v[k] - mx, -1.0e10f) * kLog2e);
+    }
+    double s = (double)fs;
+    s += __shfl_xor(s, 32, 64);
+    if (lane < 32) red[w][lane] = s;
+    __syncthreads();
+    if (threadIdx.x < 32 && i < I) {
+        pm[(size_t)band * I + i] = mx;
+        ps[(size_t)band * I + i] = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
+    }
+}
+
 constexpr int kPartialRows = 8;
 __global__ __launch_bounds__(256) void k_sm_partial(const float *__restrict__ R, int64_t ldr, int S, int I,
                                                     int rows_per_band, float *__restrict__ pm,
@@ -36,21 +77,22 @@ __global__ __launch_bounds__(256) void k_sm_partial(const float *__restrict__ R,
     float m = -1.0e10f;
     double sum = 0.0;
     const float *col = R + i;
-    for (int s = r0; s < r1; s += kPartialRows) {  // the rows' loads in flight together, one rescale for them
+    for (int s = r0; s < r1; s += kPartialRows) {  // the rows' loads in flight together
         float v[kPartialRows];
 #pragma unroll
         for (int q = 0; q < kPartialRows; ++q) v[q] = col[(size_t)min(s + q, r1 - 1) * ldr];
-        float mx = m;
-#pragma unroll
-        for (int q = 0; q < kPartialRows; ++q) mx = fmaxf(mx, v[q]);
-        if (mx > m) {
-            sum *= (double)expf(m - mx);
-            m = mx;
-        }
 #pragma unroll
         for (int q = 0; q < kPartialRows; ++q) {
-            const float d = v[q] - m;
-            if (d > -1.0e10f && s + q < r1) sum += (double)expf(d);
+            if (s + q >= r1) break;
+            const bool up = v[q] > m;
+            const float d = up ? m - v[q] : v[q] - m;
+            const double ex = (double)expf(d);
+            if (up) {
+                sum = sum * ex + 1.0;
+                m = v[q];
+            } else if (d > -1.0e10f) {
+                sum += ex;
+            }
         }
     }
     pm[(size_t)band * I + i] = m;
@@ -481,7 +523,8 @@ __global__ __launch_bounds__(256) void k_sm_apply(float *__restrict__ R, int64_t
 
 // Partials layout inside c->part:  pm (float, nb*I) | ps (double, nb*I) | blk (double) | Tpart |
 // non-zero counts (one per apply workgroup).
-// nb = the partial pass's band count, or (MFMA logL with fused partials) one band per 256 rows.
+// nb = the partial pass's band count, or (MFMA logL with fused partials) one band per logl_band_rows rows; after
+// 64-row tiles the bands of 256 rows have theirs in the place of ps.
 int softmax_bands(int S, int I)
 {
     return std::max(1, std::min((S + 63) / 64, 4096 / std::max(1, (I + 255) / 256) + 1));
@@ -534,14 +577,23 @@ hipError_t launch_softmax(const emc_ctx *c, hipStream_t st)
     double *Tpart = blk + nfin + 1;
     if (!fused)
         hipLaunchKernelGGL(k_sm_partial, dim3(ncol, nb), dim3(256), 0, st, c->R, (int64_t)c->Ip, S, I, rows, pm, ps);
-    hipLaunchKernelGGL(k_sm_final, dim3(nfin), dim3(256), 0, st, pm, ps, nb, I, c->lse, blk, c->scal);
+    const int16_t *gblk = fused && c->logits_partial ? c->blk : nullptr;
+    if (fused && logl_band_pass(c)) {  // pm: maxima of 64-row groups; the bands' partials take the place of ps
+        const int bands = nb / 4;
+        float *bm = reinterpret_cast<float *>(ps + (int64_t)bands * I);
+        hipLaunchKernelGGL(k_sm_band, dim3((I + 31) / 32, bands), dim3(256), 0, st, c->R, (int64_t)c->Ip, S, I, c->chunk,
+                           c->chunkp / 256, pm, gblk, bm, ps);
+        hipLaunchKernelGGL(k_sm_final, dim3(nfin), dim3(256), 0, st, bm, ps, bands, I, c->lse, blk, c->scal);
+    } else {
+        hipLaunchKernelGGL(k_sm_final, dim3(nfin), dim3(256), 0, st, pm, ps, nb, I, c->lse, blk, c->scal);
+    }
     const int ncb = (I + kApplyCols - 1) / kApplyCols;
     const dim3 ga(ncb, (S + kApplyRows - 1) / kApplyRows);
     double *nzpart = Tpart + (int64_t)ncb * S;  // one non-zero count per apply workgroup
     if (c->mfma)
         hipLaunchKernelGGL(k_sm_apply<1>, ga, dim3(256), 0, st, c->R, (int64_t)c->Ip, S, I, c->lse, c->Ph, c->Pl,
                            Tpart, nzpart, c->opt.scaling ? c->iphi : nullptr, c->pdirty, p_segments(c),
-                           fused ? pm : nullptr, fused && c->logits_partial ? c->blk : nullptr, c->chunk,
+                           fused ? pm : nullptr, gblk, c->chunk,
                            c->chunkp / logl_band_rows(c), logl_band_rows(c), nullptr);
     else
         hipLaunchKernelGGL(k_sm_apply<0>, ga, dim3(256), 0, st, c->R, (int64_t)c->Ip, S, I, c->lse, nullptr, nullptr,

@@ -1,5 +1,5 @@
-"""Binned insertion at its unit sizes (2,048 pairs; 4,096 pairs, two or four units a workgroup), with and without the
-grouping pass, against the atomic insertion of the same slice sums."""
+"""Binned insertion with one unit a workgroup and with blocks of four, with and without the grouping pass, against the
+atomic insertion of the same slice sums."""
 import numpy as np
 import pytest
 
@@ -7,8 +7,8 @@ import emc_amd
 
 pytestmark = pytest.mark.gpu
 
-# L, rotations, chunk: 2,048-pair units without and with a grouping pass and with a ragged last chunk, two units of
-# 4,096 a workgroup, four of them
+# L, rotations, chunk: one unit a workgroup without and with a grouping pass and with a ragged last chunk, then blocks of
+# four units
 CASES = [(6, 3, 0), (12, 60, 0), (24, 420, 0), (17, 420, 100), (32, 3240, 0), (45, 3240, 1300), (64, 12000, 0)]
 
 
