@@ -41,7 +41,11 @@ constexpr int kBrick = 8;
 constexpr int kBrick3 = kBrick * kBrick * kBrick;  // base voxels of a brick
 constexpr int kUnit = 4096;                        // pairs of a unit (positions fit 16 bits)
 constexpr int kUnitsPerBlock = 4;                  // units of a block
-constexpr int kSplitUnits = 1024;                  // up to this many units a chunk: one workgroup each
+// Up to this many units a chunk take a workgroup each (their corner sums, 32 KB a unit, go through memory; with more of
+// them the chip's 512 workgroup slots are filled by the blocks).  Insertion kernel and the pass over the units, us,
+// against a workgroup per block: 24^3 / 420 rotations (60 units) 21 / 36, 32^3 / 3,240 (700) 41 / 56, 45^3 nearest,
+// 1,000 a chunk (400) 26 / 33.
+constexpr int kSplitUnits = 1024;
 constexpr int kVbeg = 520;                         // run starts per unit: kBrick3 + 1, padded to 16 bytes
 constexpr int kGroup = 32;                         // blocks whose partials one grouping workgroup sums
 constexpr int kDirect = 8;                         // up to this many blocks per brick: no grouping pass (a launch;
@@ -49,6 +53,7 @@ constexpr int kDirect = 8;                         // up to this many blocks per
 constexpr int kHalo = kBrick + 1;
 constexpr int kHalo3 = kHalo * kHalo * kHalo;      // voxels a brick's pairs reach
 constexpr int kThreads = 512;  // 8 waves; with 67 KB of LDS and 128 registers two workgroups (16 waves) fit a CU
+constexpr int kReduceThreads = 128;  // of the last pass: all latency, so spread over the chip (32^3: 12.1 us with 512, 10.8)
 constexpr int kPer = kUnit / kThreads;  // positions per thread in step 2
 
 struct BinGeom {
@@ -436,12 +441,12 @@ __global__ __launch_bounds__(kThreads) void k_bin_group(const int32_t *__restric
 // a brick's low face, the neighbour below on that axis (whose halo index there is kBrick); in a
 // fixed order.  gbeg: [key - key0] first group of each brick of the chunk (kBricks + 1 entries);
 // without a grouping pass, blocks and their partials take the place of the groups.
-__global__ __launch_bounds__(kThreads) void k_insert_reduce(const float *__restrict__ gpart,
+__global__ __launch_bounds__(kReduceThreads) void k_insert_reduce(const float *__restrict__ gpart,
                                                             const int32_t *__restrict__ gbeg, BinGeom g,
                                                             float *__restrict__ Mnum, float *__restrict__ Wt,
                                                             bool first, bool direct)
 {
-    const int64_t v = blockIdx.x * (int64_t)kThreads + threadIdx.x;
+    const int64_t v = blockIdx.x * (int64_t)kReduceThreads + threadIdx.x;
     const int L = g.L;
     if (v >= (int64_t)L * L * L) return;
     const int x = (int)(v % L), y = (int)((v / L) % L), z = (int)(v / ((int64_t)L * L));
@@ -728,7 +733,7 @@ hipError_t launch_insert_binned(const emc_ctx *c, int s0, int cs, hipStream_t st
         hipLaunchKernelGGL(k_bin_group, dim3(g1 - g0), dim3(kThreads), 0, st, c->bin_groups + 4 * (size_t)g0, c->bin_part,
                            c->bin_gpart);
     const int nbr = g.nb * g.nb * g.nb;
-    hipLaunchKernelGGL(k_insert_reduce, dim3((unsigned)((c->N3 + kThreads - 1) / kThreads)), dim3(kThreads), 0, st,
+    hipLaunchKernelGGL(k_insert_reduce, dim3((unsigned)((c->N3 + kReduceThreads - 1) / kReduceThreads)), dim3(kReduceThreads), 0, st,
                        c->bin_direct ? c->bin_part : c->bin_gpart, c->bin_gbeg + (size_t)k * (nbr + 1), g, c->Mnum,
                        c->Wt, k == 0, c->bin_direct);
     return hipGetLastError();

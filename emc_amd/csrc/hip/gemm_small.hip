@@ -18,7 +18,7 @@ constexpr int kTerm = 64 * SK * 2;  // LDS bytes of one operand term per stage
 
 // TWO: the products with B[0] and with B[1] are summed apart and added at the end, as two launches of the large
 // tiles' store epilogue would (the second adding to the first).
-template <int EPI, int NA, int NB, bool TWO>
+template <int EPI, int NA, int NB, bool TWO, bool DEEP>
 __global__ __launch_bounds__(256) void k_small(const bf16_t *__restrict__ A0, const bf16_t *__restrict__ A1,
                                                const bf16_t *__restrict__ A2, int64_t lda,
                                                const bf16_t *__restrict__ B0, const bf16_t *__restrict__ B1,
@@ -39,12 +39,14 @@ __global__ __launch_bounds__(256) void k_small(const bf16_t *__restrict__ A0, co
     const int fr = lane & 31, fh = lane >> 5;
     const int mw = m0 + (wave >> 1) * 32, nw = n0 + (wave & 1) * 32;
     constexpr int NTERM = NA + NB, STAGE = NTERM * kTerm;
-    constexpr int kST = NTERM <= 3 ? 3 : 2;  // stages (LDS: two workgroups per CU)
+    // stages: two workgroups per CU, or one with as many as its LDS holds
+    constexpr int kST = DEEP ? (NTERM <= 2 ? 8 : NTERM == 3 ? 6 : NTERM == 4 ? 4 : 3) : NTERM <= 3 ? 3 : 2;
     constexpr int LPW = NTERM * 2;  // DMA instructions per wavefront and stage (8 rows each; 8 per term)
-    constexpr int AHEAD = (kST - 2) * LPW;
-    static_assert(AHEAD < 64);
+    constexpr int AHEAD = (kST - (DEEP ? 3 : 2)) * LPW, FIRST = (kST - 2) * LPW;
+    static_assert(AHEAD >= 0 && FIRST < 64);
     // s_waitcnt encoding: vmcnt in bits 3:0 and 15:14, lgkmcnt and expcnt not waited
     constexpr uint32_t kVmAhead = 0x0F70 | (AHEAD & 15) | ((AHEAD >> 4) << 14), kVm0 = 0x0F70;
+    constexpr uint32_t kVmFirst = 0x0F70 | (FIRST & 15) | ((FIRST >> 4) << 14);
     __shared__ __attribute__((aligned(1024))) unsigned char smem[kST * STAGE];
     // DMA instruction q of this wavefront: rows 8 rb .. 8 rb + 7 of one term; lane l writes chunk l & 7 of row
     // 8 rb + l / 8, which holds logical chunk (l & 7) ^ ((row >> 1) & 7)
@@ -74,18 +76,22 @@ __global__ __launch_bounds__(256) void k_small(const bf16_t *__restrict__ A0, co
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = acc1[r] = 0.0f;
     const int sw = (fr >> 1) & 7;
-    auto step_mm = [&](int stage) {
+    struct Frags {
+        bf16x8 a[NA][4], b[NB][4];
+    };
+    auto fetch = [&](int stage, Frags &f) {
         const unsigned char *S = smem + stage * STAGE;
         const unsigned char *ra = S + ((wave >> 1) * 32 + fr) * 128, *rb = S + NA * kTerm + ((wave & 1) * 32 + fr) * 128;
-        bf16x8 fa[NA][4], fb[NB][4];
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             const int co = ((2 * t + fh) ^ sw) * 16;
 #pragma unroll
-            for (int a = 0; a < NA; ++a) fa[a][t] = *reinterpret_cast<const bf16x8 *>(ra + a * kTerm + co);
+            for (int a = 0; a < NA; ++a) f.a[a][t] = *reinterpret_cast<const bf16x8 *>(ra + a * kTerm + co);
 #pragma unroll
-            for (int b = 0; b < NB; ++b) fb[b][t] = *reinterpret_cast<const bf16x8 *>(rb + b * kTerm + co);
+            for (int b = 0; b < NB; ++b) f.b[b][t] = *reinterpret_cast<const bf16x8 *>(rb + b * kTerm + co);
         }
+    };
+    auto multiply = [&](const Frags &f) {
 #pragma unroll
         for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -94,7 +100,7 @@ __global__ __launch_bounds__(256) void k_small(const bf16_t *__restrict__ A0, co
                 for (int b = NB - 1; b >= 0; --b)
                     if (a + b < NT) {
                         f32x16 &to = TWO && b == 1 ? acc1 : acc;
-                        to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[a][t], fb[b][t], to, 0, 0, 0);
+                        to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[a][t], f.b[b][t], to, 0, 0, 0);
                     }
     };
     // step k is in stage k % kST.  Past the last step the loads fetch it again (into a stage nothing reads),
@@ -102,13 +108,36 @@ __global__ __launch_bounds__(256) void k_small(const bf16_t *__restrict__ A0, co
     const int nk = Kd / SK;
 #pragma unroll
     for (int s = 0; s < kST - 1; ++s) issue(min(s, nk - 1), s);
-    int st = 0;
-    for (int k = 0; k < nk; ++k) {
-        __builtin_amdgcn_s_waitcnt(kVmAhead);  // this wavefront's loads of step k
-        __syncthreads();                       // every wavefront's, and the last reads of step k - 1's stage
-        issue(min(k + kST - 1, nk - 1), st == 0 ? kST - 1 : st - 1);
-        step_mm(st);
-        st = st + 1 == kST ? 0 : st + 1;
+    if constexpr (DEEP) {
+        // step k multiplies the fragments read in step k - 1, while those of step k + 1 are read
+        Frags f[2];
+        __builtin_amdgcn_s_waitcnt(kVmFirst);  // this wavefront's loads of step 0
+        __syncthreads();
+        fetch(0, f[0]);
+        int st = 0;
+        auto step = [&](int k, const Frags &now, Frags &next) {
+            __builtin_amdgcn_s_waitcnt(kVmAhead);  // of step k + 1
+            __syncthreads();                       // every wavefront's, and the last reads of step k - 1's stage
+            issue(min(k + kST - 1, nk - 1), st == 0 ? kST - 1 : st - 1);
+            st = st + 1 == kST ? 0 : st + 1;
+            fetch(st, next);
+            multiply(now);
+        };
+        for (int k = 0; k < nk; k += 2) {
+            step(k, f[0], f[1]);
+            if (k + 1 < nk) step(k + 1, f[1], f[0]);
+        }
+    } else {
+        Frags f;
+        int st = 0;
+        for (int k = 0; k < nk; ++k) {
+            __builtin_amdgcn_s_waitcnt(kVmAhead);  // this wavefront's loads of step k
+            __syncthreads();                       // every wavefront's, and the last reads of step k - 1's stage
+            issue(min(k + kST - 1, nk - 1), st == 0 ? kST - 1 : st - 1);
+            fetch(st, f);
+            multiply(f);
+            st = st + 1 == kST ? 0 : st + 1;
+        }
     }
     __builtin_amdgcn_s_waitcnt(kVm0);  // no load is left to write LDS
     if constexpr (TWO)
@@ -171,11 +200,22 @@ __global__ __launch_bounds__(256) void k_small(const bf16_t *__restrict__ A0, co
         }
 }
 
+// Up to one tile per CU: a workgroup has the CU to itself, all of its LDS for stages, and reads the next step's
+// fragments while it multiplies (three-term slices, 1,000 x 777 x 1,664: 22.4 us with two stages, 21 with four, 17
+// with the fragments ahead too; 420 x 64 x 512 8.2 both ways).  With more tiles two workgroups share a CU and hide each
+// other's waits: 3,240 x 1,000 x 896 two-term counts 30 us, one workgroup with four stages 46.
+constexpr int64_t kDeepTiles = 256;
+
 template <int EPI, int NA, int NB, bool TWO = false>
 hipError_t launch(const Contraction &g, hipStream_t st)
 {
-    hipLaunchKernelGGL((k_small<EPI, NA, NB, TWO>), dim3((g.N + SN - 1) / SN, g.M / SM), dim3(256), 0, st, g.A[0], g.A[1],
-                       g.A[2], g.lda, g.B[0], g.B[1], g.ldb, g.K, g.e);
+    const dim3 grid((g.N + SN - 1) / SN, g.M / SM);
+    const bool deep = (int64_t)grid.x * grid.y <= kDeepTiles;
+    const auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, g.A[0], g.A[1], g.A[2], g.lda, g.B[0], g.B[1], g.ldb, g.K, g.e);
+    };
+    if (deep) run(k_small<EPI, NA, NB, TWO, true>);
+    else run(k_small<EPI, NA, NB, TWO, false>);
     return hipGetLastError();
 }
 

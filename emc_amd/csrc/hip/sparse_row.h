@@ -7,9 +7,9 @@
 // non-zero hi in the whole workgroup ends after one barrier; otherwise its non-zero entries are
 // compacted into an LDS list in ascending order (wave scans and a block prefix sum keep the order,
 // so the result is deterministic), in as many batches as the list needs, and each full list (and
-// the last) has its count rows added to registers, 16 pixels per thread and pass.  Counts as
-// bytes (KT 0), BF16 (KT 1) or BF16 hi + lo (KT 2); NPASS 16-pixel chunks per thread (Pp <=
-// 4096 * NPASS).  FP32 accumulation, one fused multiply-add per entry and pixel, in ascending entry order: the
+// the last) has its count rows added to registers, PX pixels per thread and pass.  Counts as
+// bytes (KT 0), BF16 (KT 1) or BF16 hi + lo (KT 2); NPASS chunks of PX pixels per thread (Pp <=
+// 256 * PX * NPASS).  FP32 accumulation, one fused multiply-add per entry and pixel, in ascending entry order: the
 // chain of the dense FP32 contraction without its zero entries.
 // KT 3 is the FP32 precision: the row is float (ph; pl unused) and so are the counts.
 #pragma once
@@ -26,14 +26,35 @@ constexpr int kStep = 256 * kPer; // entries scanned per step
 static_assert(256 % kPer == 0, "a thread's entries lie in one 256-entry segment");
 
 __device__ __forceinline__ float half16(const u32x4 &v, int k) { return bf2f((bf16_t)(v[k >> 1] >> (16 * (k & 1)))); }
+// N 32-bit words from p (aligned to them, at most 16 bytes)
+template <int N>
+__device__ __forceinline__ void load_words(const void *__restrict__ p, uint32_t (&w)[N])
+{
+    typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+    static_assert(N == 1 || N == 2 || N % 4 == 0);
+    if constexpr (N == 1) {
+        w[0] = *reinterpret_cast<const uint32_t *>(p);
+    } else if constexpr (N == 2) {
+        const u32x2 v = *reinterpret_cast<const u32x2 *>(p);
+        w[0] = v[0];
+        w[1] = v[1];
+    } else {
+#pragma unroll
+        for (int k = 0; k < N; k += 4) {
+            const u32x4 v = reinterpret_cast<const u32x4 *>(p)[k / 4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) w[k + q] = v[q];
+        }
+    }
+}
 __device__ __forceinline__ bool nonzero(const u32x4 &v) { return (v[0] | v[1] | v[2] | v[3]) != 0u; }
 }  // namespace sparse_row_detail
 
 // n entries of the row; pat == nullptr: entry n is pattern n.  Pp is a multiple of 16 and at most
-// 4096 * NPASS; the row holds a multiple of 8 readable entries (padding entries are 0) and starts
+// 256 * PX * NPASS; the row holds a multiple of 8 readable entries (padding entries are 0) and starts
 // 16-byte aligned.  seg (or nullptr): one flag per 256 entries of the row, 0 where those entries are
 // known to be zero (their loads are skipped).
-template <int KT, int NPASS>
+template <int KT, int NPASS, int PX = 16>
 __device__ __forceinline__ void sparse_row(const void *__restrict__ ph, const bf16_t *__restrict__ pl, int n,
                                            const int32_t *__restrict__ pat, const void *__restrict__ Kv,
                                            const bf16_t *__restrict__ Klo, int Pp, float *__restrict__ out,
@@ -56,12 +77,13 @@ __device__ __forceinline__ void sparse_row(const void *__restrict__ ph, const bf
     __shared__ float lp[kCap];
     __shared__ int wsum[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int nch = Pp / 16;
-    float acc[NPASS][16];
+    const int nch = Pp / PX;
+    constexpr int kAhead = PX == 16 ? 4 : 8;
+    float acc[NPASS][PX];
 #pragma unroll
     for (int q = 0; q < NPASS; ++q)
 #pragma unroll
-        for (int k = 0; k < 16; ++k) acc[q][k] = 0.0f;
+        for (int k = 0; k < PX; ++k) acc[q][k] = 0.0f;
 
     auto accumulate = [&](int cnt) {
 #pragma unroll
@@ -70,42 +92,30 @@ __device__ __forceinline__ void sparse_row(const void *__restrict__ ph, const bf
             if (pc >= nch) break;
             // unrolled so that the count-row loads of several entries are in flight together (the
             // sums still add the entries in list order)
-#pragma unroll 4
+#pragma unroll kAhead
             for (int e = 0; e < cnt; ++e) {
-                const size_t row = (size_t)li[e] * Pp + 16 * (size_t)pc;
+                const size_t row = (size_t)li[e] * Pp + PX * (size_t)pc;
                 const float p = lp[e];
-                if (KT == 0) {
-                    const u32x4 v = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const uint8_t *>(Kv) + row);
+                if constexpr (KT == 0) {
+                    uint32_t v[PX / 4];
+                    load_words(reinterpret_cast<const uint8_t *>(Kv) + row, v);
 #pragma unroll
-                    for (int k = 0; k < 16; ++k)
+                    for (int k = 0; k < PX; ++k)
                         acc[q][k] = __builtin_fmaf(p, (float)((v[k >> 2] >> (8 * (k & 3))) & 0xffu), acc[q][k]);
-                } else if (KT == 3) {
-                    const float4 *kr = reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(Kv) + row);
+                } else if constexpr (KT == 3) {
+                    uint32_t v[PX];
+                    load_words(reinterpret_cast<const float *>(Kv) + row, v);
 #pragma unroll
-                    for (int w = 0; w < 4; ++w) {
-                        const float4 v = kr[w];
-                        acc[q][4 * w] = __builtin_fmaf(p, v.x, acc[q][4 * w]);
-                        acc[q][4 * w + 1] = __builtin_fmaf(p, v.y, acc[q][4 * w + 1]);
-                        acc[q][4 * w + 2] = __builtin_fmaf(p, v.z, acc[q][4 * w + 2]);
-                        acc[q][4 * w + 3] = __builtin_fmaf(p, v.w, acc[q][4 * w + 3]);
-                    }
+                    for (int k = 0; k < PX; ++k) acc[q][k] = __builtin_fmaf(p, __uint_as_float(v[k]), acc[q][k]);
                 } else {
-                    const bf16_t *kr = reinterpret_cast<const bf16_t *>(Kv) + row;
-                    const u32x4 a = *reinterpret_cast<const u32x4 *>(kr), b = *reinterpret_cast<const u32x4 *>(kr + 8);
-                    u32x4 al = {0u, 0u, 0u, 0u}, bl = {0u, 0u, 0u, 0u};
-                    if (KT == 2) {
-                        al = *reinterpret_cast<const u32x4 *>(Klo + row);
-                        bl = *reinterpret_cast<const u32x4 *>(Klo + row + 8);
-                    }
+                    uint32_t v[PX / 2], vl[PX / 2];
+                    load_words(reinterpret_cast<const bf16_t *>(Kv) + row, v);
+                    if (KT == 2) load_words(Klo + row, vl);
 #pragma unroll
-                    for (int k = 0; k < 8; ++k) {
-                        float k0 = half16(a, k), k1 = half16(b, k);
-                        if (KT == 2) {
-                            k0 += half16(al, k);
-                            k1 += half16(bl, k);
-                        }
-                        acc[q][k] = __builtin_fmaf(p, k0, acc[q][k]);
-                        acc[q][8 + k] = __builtin_fmaf(p, k1, acc[q][8 + k]);
+                    for (int k = 0; k < PX; ++k) {
+                        float x = bf2f((bf16_t)(v[k >> 1] >> (16 * (k & 1))));
+                        if (KT == 2) x += bf2f((bf16_t)(vl[k >> 1] >> (16 * (k & 1))));
+                        acc[q][k] = __builtin_fmaf(p, x, acc[q][k]);
                     }
                 }
             }
@@ -177,8 +187,8 @@ __device__ __forceinline__ void sparse_row(const void *__restrict__ ph, const bf
         const int pc = tid + q * 256;
         if (pc >= nch) break;
 #pragma unroll
-        for (int k = 0; k < 16; k += 4)
-            *reinterpret_cast<float4 *>(out + 16 * pc + k) = make_float4(acc[q][k], acc[q][k + 1], acc[q][k + 2], acc[q][k + 3]);
+        for (int k = 0; k < PX; k += 4)
+            *reinterpret_cast<float4 *>(out + PX * pc + k) = make_float4(acc[q][k], acc[q][k + 1], acc[q][k + 2], acc[q][k + 3]);
     }
 }
 
