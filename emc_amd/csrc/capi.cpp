@@ -332,7 +332,7 @@ extern "C" emc_status emc_create(const emc_dims *d, const emc_options *o, emc_ct
     if (st == EMC_OK) A(dalloc(&c->Mnum, N3), "Mnum");
     if (st == EMC_OK) A(dalloc(&c->Wt, N3), "Wt");
     if (st == EMC_OK) A(dalloc(&c->tmp3, N3), "tmp3");
-    if (st == EMC_OK) A(dalloc(&c->modelq, N3), "modelq");
+    if (st == EMC_OK) A(dalloc(&c->modelq, quad_model_len(c->L)), "modelq");
     if (st == EMC_OK) A(dalloc(&c->taps, c->L), "taps");
     if (st == EMC_OK) A(dalloc(&c->sumW, Sp), "sumW");
     if (st == EMC_OK) A(dalloc(&c->ns, Sp), "ns");

@@ -156,7 +156,7 @@ struct emc_ctx {
     double *sumK = nullptr;   // [Ip]
     // model
     float *model = nullptr, *Mnum = nullptr, *Wt = nullptr, *tmp3 = nullptr;  // [N3]
-    float4 *modelq = nullptr; // [N3] quad-packed model of the trilinear statistics pass (MFMA path)
+    float4 *modelq = nullptr; // quad-packed model of the trilinear statistics pass
     float *taps = nullptr;    // [L] blur taps
     // slicing stage
     double *sumW = nullptr;   // [Sp]
@@ -244,6 +244,7 @@ hipError_t launch_fill_i32(int32_t *p, int32_t v, int64_t n, hipStream_t st);
 
 // Slicing statistics over rotations [0, S): sumW, ns, the slices that a later pass reads and (BF16
 // Poisson) the column sums of log W; clears the E-step's non-finite flag.  colp / colpart hold colp_len / colpart_len elements.
+int64_t quad_model_len(int L);
 int64_t colp_len(int S, int Pp);
 int64_t colpart_len(int Pp);
 hipError_t launch_slice_stats(const emc_ctx *c, hipStream_t st);

@@ -84,29 +84,42 @@ __device__ __forceinline__ float sample(const float *__restrict__ model, int L, 
     }
 }
 
-// Trilinear sample from the quad-packed model (modelq[v] = model at v, v + 1, v + L, v + L + 1; 0 past
-// an edge): the 8 corners in two 16-byte loads from two cache lines instead of 8 loads from four.  The
-// same corners, test and arithmetic as sample<EMC_INTERP_TRILINEAR>, so the same value bit for bit.
+// The quad-packed model: entry v holds the model at v, v + 1, v + L, v + L + 1 (0 past an edge), so the 8 corners of
+// a trilinear sample are two 16-byte loads.  The entries of 2 x 2 x 2 voxels share a 128-byte line: a slice
+// crosses fewer of those than of lines of 8 voxels along x, whichever way it lies.
+__host__ __device__ __forceinline__ int64_t quad_blocks(int L) { return (L + 1) / 2; }
+__device__ __forceinline__ uint32_t quad_index(int x, int y, int z, uint32_t nb)
+{
+    return (((uint32_t)(z >> 1) * nb + (uint32_t)(y >> 1)) * nb + (uint32_t)(x >> 1)) * 8 +
+           (uint32_t)((z & 1) * 4 + (y & 1) * 2 + (x & 1));
+}
+
+// Trilinear sample from it: the same corners, test and arithmetic as sample<EMC_INTERP_TRILINEAR>, so the same value
+// bit for bit.  The loads do not wait for the test (a point outside reads the nearest cell), so those of
+// several samples are in flight together.
 __device__ __forceinline__ float sample_quad(const float4 *__restrict__ modelq, int L, const float *m, float X,
                                              float Y, float Z)
 {
     float ux, uy, uz;
     rot_point(m, X, Y, Z, model_c(L), ux, uy, uz);
-    int bx, by, bz;
-    float fx, fy, fz;
-    if (!tri_axis(ux, L, bx, fx) || !tri_axis(uy, L, by, fy) || !tri_axis(uz, L, bz, fz)) return -1.0f;
-    const size_t base = ((size_t)bz * L + by) * L + bx;
-    const float4 q0 = modelq[base], q1 = modelq[base + (size_t)L * L];
+    const float hi = (float)(L - 1);
+    const bool ok = ux >= 0.0f && ux <= hi && uy >= 0.0f && uy <= hi && uz >= 0.0f && uz <= hi;
+    const auto cell = [&](float u) { return max(min((int)__builtin_floorf(u), L - 2), 0); };
+    const int bx = cell(ux), by = cell(uy), bz = cell(uz);
+    const float fx = ux - (float)bx, fy = uy - (float)by, fz = uz - (float)bz;
+    const uint32_t nb = (uint32_t)quad_blocks(L);
+    const uint32_t base = quad_index(bx, by, bz, nb);
+    const float4 q0 = modelq[base], q1 = modelq[base + ((bz & 1) ? nb * nb * 8 - 4 : 4)];
     const float v000 = q0.x, v001 = q0.y, v010 = q0.z, v011 = q0.w;
     const float v100 = q1.x, v101 = q1.y, v110 = q1.z, v111 = q1.w;
     const float mn = fminf(fminf(fminf(v000, v001), fminf(v010, v011)),
                            fminf(fminf(v100, v101), fminf(v110, v111)));
-    if (mn < 0.0f) return -1.0f;  // a missing voxel among the corners
     const float gx = 1.0f - fx, gy = 1.0f - fy, gz = 1.0f - fz;
     const float c00 = v000 * gx + v001 * fx, c01 = v010 * gx + v011 * fx;
     const float c10 = v100 * gx + v101 * fx, c11 = v110 * gx + v111 * fx;
     const float c0 = c00 * gy + c01 * fy, c1 = c10 * gy + c11 * fy;
-    return c0 * gz + c1 * fz;
+    const float W = c0 * gz + c1 * fz;
+    return ok && !(mn < 0.0f) ? W : -1.0f;  // outside, or a missing voxel among the corners
 }
 
 // Pixel weight of the chi^2 kinds: poisson (reference chi^2) 1/(W+0.02), absolute 1, relative 1/W^2.

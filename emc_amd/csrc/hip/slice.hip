@@ -16,7 +16,7 @@ namespace {
 
 // rotations per workgroup in the statistics pass: 8 keeps 4 waves per SIMD (16 needed 210 VGPRs,
 // 2 waves per SIMD: 0.77 instead of 0.61 ms at 64^3 / 25,680 rotations)
-constexpr int kStatsG = 8;
+constexpr int kStatsG = 8, kStatsH = 4;  // kStatsH: whose samples' loads are in flight together
 
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v)
@@ -58,6 +58,28 @@ __global__ __launch_bounds__(256) void k_export(const float *__restrict__ a, con
     }
 }
 
+__global__ void k_quad_model(const float *__restrict__ model, int L, float4 *__restrict__ modelq)
+{
+    const int nb = (int)quad_blocks(L);
+    const int64_t n = (int64_t)nb * nb * nb * 8;
+    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x) {
+        const int k = (int)(t & 7);
+        const int64_t b = t >> 3;
+        const int x = (int)(b % nb) * 2 + (k & 1), y = (int)(b / nb % nb) * 2 + ((k >> 1) & 1);
+        const int z = (int)(b / ((int64_t)nb * nb)) * 2 + (k >> 2);
+        float4 q = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (x < L && y < L && z < L) {
+            const int64_t v = ((int64_t)z * L + y) * L + x;
+            const bool xe = x + 1 < L, ye = y + 1 < L;
+            q = make_float4(model[v], xe ? model[v + 1] : 0.0f, ye ? model[v + L] : 0.0f, xe && ye ? model[v + L + 1] : 0.0f);
+        }
+        modelq[t] = q;
+    }
+}
+
+// What the statistics pass keeps of its samples, so that no later pass gathers from the model again.
+enum { KEEP_NONE, KEEP_LOG, KEEP_W, KEEP_WA };
+
 // Per-rotation slice sum over V_s = {active j : W > 0}, |V_s|, and per pixel the workgroup's sum of
 // log W and number of rotations with a valid sample (colp[block][j] = (sum, count); summed over
 // the blocks in a fixed order by k_colsum_*, so the column sums are deterministic).
@@ -66,21 +88,11 @@ __global__ __launch_bounds__(256) void k_export(const float *__restrict__ a, con
 // operand split, KEEP_W keeps W (0 where invalid) for the chi^2 operands, KEEP_WA the FP32 chi^2
 // contraction's operands W and a themselves: a second gather from the model costs as much as this one
 // (64^3 / 6,300 rotations 125 us), reading back what was kept 20 to 50 us.
-// modelq[v] = (model[v], model[v + 1], model[v + L], model[v + L + 1]), 0 past an edge (the trilinear
-// statistics pass reads the 8 corners of a sample as two 16-byte loads).
-__global__ void k_quad_model(const float *__restrict__ model, int L, float4 *__restrict__ modelq)
-{
-    const int64_t n = (int64_t)L * L * L;
-    for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < n; v += (int64_t)gridDim.x * blockDim.x) {
-        const bool xe = (int)(v % L) + 1 < L, ye = (int)((v / L) % L) + 1 < L;
-        modelq[v] = make_float4(model[v], xe ? model[v + 1] : 0.0f, ye ? model[v + L] : 0.0f,
-                                xe && ye ? model[v + L + 1] : 0.0f);
-    }
-}
-
-// What the statistics pass keeps of its samples, so that no later pass gathers from the model again.
-enum { KEEP_NONE, KEEP_LOG, KEEP_W, KEEP_WA };
-
+// What bounds it: the lines that the gathers touch and their latency.  Samples load whether the point is inside or
+// not, four rotations' at once, from a quad-packed model in 2 x 2 x 2 blocks (geom.h), us at 64^3 / 25,680
+// rotations, 128^3 / 6,300 and 64^3 / 6,300: 382, 838, 107 with the loads behind each sample's test and lines along x;
+// 325, 847 with the loads ahead alone; 285, 578, 91 with the blocks too, eight rotations at once (143 registers);
+// 240, 552, 78 four at once (89).
 template <int INTERP, int KEEP>
 __global__ __launch_bounds__(256) void k_slice_stats(const float *__restrict__ model,
                                                      const float4 *__restrict__ modelq, int L,
@@ -90,18 +102,15 @@ __global__ __launch_bounds__(256) void k_slice_stats(const float *__restrict__ m
                                                      float2 *__restrict__ colp, float *__restrict__ out0,
                                                      float *__restrict__ out1, double *__restrict__ scal)
 {
-    __shared__ float rm[kStatsG][9];
     __shared__ double red_w[kStatsG][256];
+    __shared__ __attribute__((aligned(16))) float rm[kStatsG][12];
     __shared__ int red_n[kStatsG][256];
     static_assert(kStatsG * 32 == 256, "32 lanes per rotation in the final sums");
     const int s0 = blockIdx.x * kStatsG;
     const int tid = threadIdx.x;
-    if (tid < kStatsG * 9) {
-        const int g = tid / 9, k = tid % 9;
-        rm[g][k] = (s0 + g < S) ? rotm[12 * (size_t)(s0 + g) + k] : 0.0f;
-    }
-    __syncthreads();
     const int ng = min(kStatsG, S - s0);
+    if (tid < kStatsG * 12) rm[tid / 12][tid % 12] = rotm[12 * (size_t)min(s0 + tid / 12, S - 1) + tid % 12];
+    __syncthreads();
     if (blockIdx.x == 0 && tid == 0) scal[SC_NONFINITE] = 0.0;  // the first kernel of an E-step
     float sw[kStatsG];
     int cnt[kStatsG];
@@ -118,10 +127,21 @@ __global__ __launch_bounds__(256) void k_slice_stats(const float *__restrict__ m
         float col = 0.0f;
         int colv = 0;
 #pragma unroll
-        for (int g = 0; g < kStatsG; ++g) {
-            if (g < ng) {
-                const float W = INTERP == EMC_INTERP_TRILINEAR ? sample_quad(modelq, L, rm[g], X, Y, Z)
-                                                               : sample<INTERP>(model, L, rm[g], X, Y, Z);
+        for (int h = 0; h < kStatsG; h += kStatsH) {
+            float Wh[kStatsH];
+#pragma unroll
+            for (int g = 0; g < kStatsH; ++g) {
+                float m[12];
+#pragma unroll
+                for (int q = 0; q < 12; q += 4)
+                    *reinterpret_cast<float4 *>(m + q) = *reinterpret_cast<const float4 *>(&rm[h + g][q]);
+                Wh[g] = INTERP == EMC_INTERP_TRILINEAR ? sample_quad(modelq, L, m, X, Y, Z) : sample<INTERP>(model, L, m, X, Y, Z);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int g = h; g < h + kStatsH; ++g) {
+                if (g >= ng) continue;
+                const float W = Wh[g - h];
                 const size_t o = (size_t)(s0 + g) * Pp + j;
                 float v0 = KEEP == KEEP_LOG ? -INFINITY : 0.0f, v1 = 0.0f;
                 if (W > 0.0f) {
@@ -488,6 +508,7 @@ hipError_t launch_export(const float *a, const float *b, int64_t N3, int64_t o, 
     return hipGetLastError();
 }
 
+int64_t quad_model_len(int L) { return 8 * quad_blocks(L) * quad_blocks(L) * quad_blocks(L); }
 int64_t colp_len(int S, int Pp) { return (int64_t)((S + kStatsG - 1) / kStatsG) * Pp; }
 int64_t colpart_len(int Pp) { return (int64_t)kColParts * Pp; }
 
@@ -515,7 +536,7 @@ hipError_t launch_slice_stats(const emc_ctx *c, hipStream_t st)
     if (c->opt.interp == EMC_INTERP_NEAREST) {
         slice_stats_interp<EMC_INTERP_NEAREST>(c, st);
     } else {
-        const int64_t n3 = (int64_t)c->L * c->L * c->L;
+        const int64_t n3 = quad_model_len(c->L);
         hipLaunchKernelGGL(k_quad_model, dim3((unsigned)std::min<int64_t>((n3 + 255) / 256, 4096)), dim3(256), 0, st,
                            c->model, c->L, c->modelq);
         slice_stats_interp<EMC_INTERP_TRILINEAR>(c, st);
