@@ -93,7 +93,7 @@ struct Proposal {
     std::vector<double> cap_h;     // per-pattern captured mass of the last measurement
     // recall: cells of largest max logit in each pattern's most recent search, -1 = none
     int32_t *recall = nullptr;     // [Ip][recall]
-    int32_t *recall_h = nullptr;   // [I][recall] pinned host copy taken with each prediction
+    int32_t *recall_h = nullptr;   // [I][recall] pinned, with each prediction: the recalled cells, -1 for those among the top k or given before
     // grouped work lists (built on the host from the prediction)
     int64_t n_slots = 0, n_blk = 0;  // slots, block elements
     int n_fallback = 0;
@@ -361,13 +361,13 @@ hipError_t mlp_colsum(const bf16_t *d, int rows, int ld, int n_valid, float *g, 
 hipError_t mlp_adam(float *w, const float *g, float *m, float *v, bf16_t *w16, int64_t n, float lr, int t,
                     hipStream_t st);
 hipError_t mlp_to_bf16(const float *w, int64_t n, bf16_t *w16, hipStream_t st);
-hipError_t mlp_topk(const float *p, int Cp, int C, int rows, int k, int32_t *cells, float *mass, hipStream_t st);
 // Cell sums Tt of the full responsibilities; with Mx also each cell's largest logit (reads the
 // logits c->R, so only while they are resident: right after a full-search E-step).
 hipError_t mlp_cell_targets(const emc_ctx *c, float *Tt, float *Mx, hipStream_t st);
 hipError_t mlp_captured(const emc_ctx *c, double *cap, hipStream_t st);
-// Adds the recalled cells' predicted probability (those not in the top k) to pmass.
-hipError_t mlp_union_mass(const emc_ctx *c, hipStream_t st);
+// Top cells and pmass (with the recalled cells, those not in the top k) from prob, on the device and in topc_h, pmass_h
+// and recall_h.
+hipError_t mlp_predict_cells(const emc_ctx *c, hipStream_t st);
 hipError_t mlp_gather_batch(const emc_ctx *c, const int32_t *idx, int rows, hipStream_t st);
 hipError_t mlp_synth_counts(const emc_ctx *c, int n, float photons, uint64_t seed, hipStream_t st);
 

@@ -225,13 +225,8 @@ emc_status proposal_predict_enqueue(emc_ctx *c)
     p->pred_valid = false;
     P_TRY(forward(c, p->X, c->Ip, false));
     P_HIP(c, mlp_softmax_ce(p->z, p->Cp, p->C, c->I, c->Ip, nullptr, 0.0f, p->prob, nullptr, nullptr, st));
-    P_HIP(c, mlp_topk(p->prob, p->Cp, p->C, c->I, p->o.top_k, p->topc, p->pmass, st));
-    P_HIP(c, mlp_union_mass(c, st));  // pmass: predicted mass of every cell the iteration would search
-    P_HIP(c, hipMemcpyAsync(p->topc_h, p->topc, sizeof(int32_t) * (size_t)c->I * p->o.top_k, hipMemcpyDeviceToHost, st));
-    P_HIP(c, hipMemcpyAsync(p->pmass_h, p->pmass, sizeof(float) * c->I, hipMemcpyDeviceToHost, st));
-    if (p->o.recall > 0)
-        P_HIP(c, hipMemcpyAsync(p->recall_h, p->recall, sizeof(int32_t) * (size_t)c->I * p->o.recall,
-                                hipMemcpyDeviceToHost, st));
+    // the top cells and pmass, the predicted mass of every cell the iteration would search, also on the host
+    P_HIP(c, mlp_predict_cells(c, st));
     P_HIP(c, hipEventRecord(p->ev_pred, st));
     return EMC_OK;
 }
@@ -257,16 +252,13 @@ emc_status proposal_build_lists(emc_ctx *c, bool *too_many)
     auto nr = [&](int cc) { return rbeg[cc + 1] - rbeg[cc]; };
 
     // cells searched for pattern i (unless it falls back): the predicted top k, then the
-    // recalled cells not among them
+    // recalled cells not among them (the others are -1 in recall_h)
     auto cells_of = [&](int i, int32_t *out) {
         int n = 0;
         for (int q = 0; q < k; ++q) out[n++] = p->topc_h[(size_t)i * k + q];
         for (int q = 0; q < R; ++q) {
             const int32_t cr = p->recall_h[(size_t)i * R + q];
-            if (cr < 0 || cr >= C) continue;
-            bool seen = false;
-            for (int u = 0; u < n; ++u) seen |= out[u] == cr;
-            if (!seen) out[n++] = cr;
+            if (cr >= 0 && cr < C) out[n++] = cr;
         }
         return n;
     };
