@@ -53,7 +53,9 @@ constexpr int kDirect = 8;                         // up to this many blocks per
 constexpr int kHalo = kBrick + 1;
 constexpr int kHalo3 = kHalo * kHalo * kHalo;      // voxels a brick's pairs reach
 constexpr int kThreads = 512;  // 8 waves; with 67 KB of LDS and 128 registers two workgroups (16 waves) fit a CU
-constexpr int kReduceThreads = 128;  // of the last pass: all latency, so spread over the chip (32^3: 12.1 us with 512, 10.8)
+// Threads of a workgroup of the last pass: all latency for few voxels, so spread over the chip (32^3: 12.1 us with 512,
+// 10.8 with 128); larger models read the partials of a brick from fewer places (128^3: 38 us with 512, 49 with 128).
+inline int reduce_threads(int64_t voxels) { return voxels < 256 * kThreads ? 128 : kThreads; }
 constexpr int kPer = kUnit / kThreads;  // positions per thread in step 2
 
 struct BinGeom {
@@ -194,8 +196,9 @@ __global__ __launch_bounds__(kThreads) void k_unit_perm(const int32_t *__restric
 // corner sums are corner-major, the tails value-major.
 //
 // What bounds it: memory, 22 bytes a pair with U, and the latency of list -> U, which the list read one unit ahead
-// halves.  64^3 / 25,680: 820 -> 607 us with that and the swizzle above (k ^ ((k >> 3) & 7) before, which left eight
-// lanes on each bank), 3.0 TB/s.  Forming the fractions here instead of reading them: 985 us (the vector units,
+// halves, and the vector units at the runs' ends, where the lanes part.  64^3 / 25,680: 820 -> 609 us with the list
+// ahead and the swizzle above (k ^ ((k >> 3) & 7) before, which left eight lanes on each bank), 594 with only the last
+// run of a thread looked at for a tail (3.1 TB/s).  The corner sums added by LDS atomics (one instruction for three): 1,110 us.  Forming the fractions here instead of reading them: 985 us (the vector units,
 // then); U, T and the fractions one unit ahead too: 17 to 31 registers spilled, 856 us.
 __device__ __forceinline__ int rswz(int k) { return k ^ ((k >> 6) & (kPer - 1)); }
 
@@ -304,20 +307,19 @@ __global__ __launch_bounds__(kThreads, 4) void k_insert_binned(const int32_t *__
             }
             lv = lo;
         }
-        float acc[2 * NC], own[2 * NC], mine[2 * NC];
+        float acc[2 * NC], own[2 * NC];
 #pragma unroll
-        for (int c = 0; c < 2 * NC; ++c) acc[c] = own[c] = mine[c] = 0.0f;
+        for (int c = 0; c < 2 * NC; ++c) acc[c] = own[c] = 0.0f;
+        // in: svb[lv] <= k0 < end; a run that began before k0 is the first one, and only the last may go on past k1
         int own_lv = -1, my_tail = -1;
-        auto close_run = [&](int kend) {  // the run of lv ends at kend (exclusive)
-            const bool open_left = svb[lv] < k0, open_right = svb[lv + 1] > kend;
-            if (open_right) {  // continues into the next thread: handed over after step 2
-#pragma unroll
-                for (int c = 0; c < 2 * NC; ++c) mine[c] = acc[c];
-                my_tail = lv;
-            } else if (open_left) {  // this thread holds the run's last position: adds the pieces later
+        bool left = k0 < k1 && svb[lv] < k0;
+        int end = k0 < k1 ? svb[lv + 1] : 0;
+        auto close_run = [&] {
+            if (left) {  // this thread holds the run's last position: adds the pieces later
 #pragma unroll
                 for (int c = 0; c < 2 * NC; ++c) own[c] = acc[c];
                 own_lv = lv;
+                left = false;
             } else {  // the whole run: only this thread touches lv in this unit
 #pragma unroll
                 for (int c = 0; c < NC; ++c) {
@@ -325,16 +327,19 @@ __global__ __launch_bounds__(kThreads, 4) void k_insert_binned(const int32_t *__
                     cW[c][lv] += acc[NC + c];
                 }
             }
-#pragma unroll
-            for (int c = 0; c < 2 * NC; ++c) acc[c] = 0.0f;
         };
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
             const int k = k0 + i;
             if (k >= k1) break;
-            if (k >= svb[lv + 1]) {
-                close_run(k);
-                while (svb[lv + 1] <= k) ++lv;  // skip base voxels without pairs
+            if (k >= end) {
+                close_run();
+#pragma unroll
+                for (int c = 0; c < 2 * NC; ++c) acc[c] = 0.0f;
+                do {  // skip base voxels without pairs
+                    ++lv;
+                    end = svb[lv + 1];
+                } while (end <= k);
             }
             const int p = rswz(k);
             const float v = sv[0][p];
@@ -354,12 +359,15 @@ __global__ __launch_bounds__(kThreads, 4) void k_insert_binned(const int32_t *__
                 }
             }
         }
-        if (k0 < k1) close_run(k1);
+        if (k0 < k1) {
+            if (end > k1) my_tail = lv;  // continues into the next thread: acc is handed over
+            else close_run();
+        }
         __syncthreads();  // the staging is consumed: the tails take its space
         tail_lv[tid] = my_tail;
         if (my_tail >= 0)
 #pragma unroll
-            for (int c = 0; c < 2 * NC; ++c) tail[c][tid] = mine[c];
+            for (int c = 0; c < 2 * NC; ++c) tail[c][tid] = acc[c];
         __syncthreads();
         if (own_lv >= 0) {  // the pieces of earlier threads, in thread order, then this thread's
             int t0 = tid;
@@ -441,12 +449,12 @@ __global__ __launch_bounds__(kThreads) void k_bin_group(const int32_t *__restric
 // a brick's low face, the neighbour below on that axis (whose halo index there is kBrick); in a
 // fixed order.  gbeg: [key - key0] first group of each brick of the chunk (kBricks + 1 entries);
 // without a grouping pass, blocks and their partials take the place of the groups.
-__global__ __launch_bounds__(kReduceThreads) void k_insert_reduce(const float *__restrict__ gpart,
+__global__ __launch_bounds__(kThreads) void k_insert_reduce(const float *__restrict__ gpart,
                                                             const int32_t *__restrict__ gbeg, BinGeom g,
                                                             float *__restrict__ Mnum, float *__restrict__ Wt,
                                                             bool first, bool direct)
 {
-    const int64_t v = blockIdx.x * (int64_t)kReduceThreads + threadIdx.x;
+    const int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     const int L = g.L;
     if (v >= (int64_t)L * L * L) return;
     const int x = (int)(v % L), y = (int)((v / L) % L), z = (int)(v / ((int64_t)L * L));
@@ -733,7 +741,8 @@ hipError_t launch_insert_binned(const emc_ctx *c, int s0, int cs, hipStream_t st
         hipLaunchKernelGGL(k_bin_group, dim3(g1 - g0), dim3(kThreads), 0, st, c->bin_groups + 4 * (size_t)g0, c->bin_part,
                            c->bin_gpart);
     const int nbr = g.nb * g.nb * g.nb;
-    hipLaunchKernelGGL(k_insert_reduce, dim3((unsigned)((c->N3 + kReduceThreads - 1) / kReduceThreads)), dim3(kReduceThreads), 0, st,
+    const int rt = reduce_threads(c->N3);
+    hipLaunchKernelGGL(k_insert_reduce, dim3((unsigned)((c->N3 + rt - 1) / rt)), dim3(rt), 0, st,
                        c->bin_direct ? c->bin_part : c->bin_gpart, c->bin_gbeg + (size_t)k * (nbr + 1), g, c->Mnum,
                        c->Wt, k == 0, c->bin_direct);
     return hipGetLastError();
