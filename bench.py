@@ -457,7 +457,7 @@ def main():
     flops = 2.0 * I * S * Pa  # one logical K.logW^T product, counted once (the BF16 split is overhead)
     t_logl = st_mfma["logl_gemm"] * 1e-3
     achieved = flops / t_logl / 1e12
-    kname, kprof = (("k_logl_dma (logL contraction, 256x256 tiles, DMA-staged BF16 operands)", "logl_dma")
+    kname, kprof = (("k_dma (logL contraction, 256x256 tiles, DMA-staged BF16 operands)", "logl_dma")
                     if args.mfma_staging == 0 else
                     ("k_gemm_mfma2 (logL contraction, 256x256 tiles, register-staged byte counts)", "logl_mfma"))
     roof = {"kernel": kname, "bound": "mfma",
