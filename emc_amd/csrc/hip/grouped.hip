@@ -230,7 +230,10 @@ __global__ __launch_bounds__(256) void k_grouped(const bf16_t *__restrict__ A0, 
 }
 
 // Softmax partials: one wavefront per 64 slots of a cell (tiles (cell, s0)); online (max, FP64
-// sum) over the cell's rotation rows, as the dense partial pass does over a band.
+// sum) over the cell's rotation rows, as the dense partial pass does over a band.  All latency: kAheadS rows' loads
+// are in flight together, also in the two passes over a pattern's slots below (64^3, 10,860 rotations in 420 cells,
+// 4,000 patterns: 25, 21 and 25 us with one load after the other, 12, 13 and 21 so).
+constexpr int kAheadS = 8;
 __global__ __launch_bounds__(256) void k_gsm_partial(const float *__restrict__ Lb, GTab g, int n_tiles,
                                                      float *__restrict__ pm, double *__restrict__ ps)
 {
@@ -244,14 +247,21 @@ __global__ __launch_bounds__(256) void k_gsm_partial(const float *__restrict__ L
     const float *col = Lb + g.boff[c] + s;
     float m = -1.0e10f;
     double sum = 0.0;
-    for (int r = 0; r < nr; ++r) {
-        const float v = col[(int64_t)r * nsp];
-        if (v > m) {
-            sum = sum * (double)expf(m - v) + 1.0;
-            m = v;
-        } else {
-            const float d = v - m;
-            if (d > -1.0e10f) sum += (double)expf(d);
+    for (int r0 = 0; r0 < nr; r0 += kAheadS) {
+        float vr[kAheadS];
+#pragma unroll
+        for (int q = 0; q < kAheadS; ++q) vr[q] = col[(int64_t)min(r0 + q, nr - 1) * nsp];
+#pragma unroll
+        for (int q = 0; q < kAheadS; ++q) {
+            if (r0 + q >= nr) break;
+            const float v = vr[q];
+            if (v > m) {
+                sum = sum * (double)expf(m - v) + 1.0;
+                m = v;
+            } else {
+                const float d = v - m;
+                if (d > -1.0e10f) sum += (double)expf(d);
+            }
         }
     }
     pm[sb + s] = m;
@@ -269,12 +279,26 @@ __global__ __launch_bounds__(256) void k_gsm_final(const float *__restrict__ pm,
     if (i < I) {
         const int q0 = g.pbeg[i], q1 = g.pbeg[i + 1];
         float m = -1.0e10f;
-        for (int q = q0; q < q1; ++q) m = fmaxf(m, pm[g.pslot[q]]);
+        for (int q = q0; q < q1; q += kAheadS) {
+            float v[kAheadS];
+#pragma unroll
+            for (int u = 0; u < kAheadS; ++u) v[u] = pm[g.pslot[min(q + u, q1 - 1)]];
+#pragma unroll
+            for (int u = 0; u < kAheadS; ++u) m = fmaxf(m, v[u]);
+        }
         double sum = 0.0;
-        for (int q = q0; q < q1; ++q) {
-            const int sl = g.pslot[q];
-            const double sv = ps[sl];
-            if (sv > 0.0) sum += sv * exp((double)pm[sl] - (double)m);
+        for (int q = q0; q < q1; q += kAheadS) {
+            float v[kAheadS];
+            double sv[kAheadS];
+#pragma unroll
+            for (int u = 0; u < kAheadS; ++u) {
+                const int sl = g.pslot[min(q + u, q1 - 1)];
+                v[u] = pm[sl];
+                sv[u] = ps[sl];
+            }
+#pragma unroll
+            for (int u = 0; u < kAheadS; ++u)
+                if (q + u < q1 && sv[u] > 0.0) sum += sv[u] * exp((double)v[u] - (double)m);
         }
         l = (double)m + log(sum);
         if (!isfinite(l)) scal[SC_NONFINITE] = 1.0;
@@ -407,22 +431,31 @@ __global__ __launch_bounds__(256) void k_recall_dense(const float *__restrict__ 
 
 // Recall after a proposal iteration: the searched cells of largest max logit (the slot partial
 // maximum pm).  The cell of a slot is found by binary search in sbeg.
-__global__ __launch_bounds__(256) void k_recall_slots(const float *__restrict__ pm, GTab g, int I, int C, int R,
+__global__ __launch_bounds__(64) void k_recall_slots(const float *__restrict__ pm, GTab g, int I, int C, int R,
                                                       int32_t *__restrict__ out)
 {
-    const int i = blockIdx.x * 256 + threadIdx.x;
+    const int i = blockIdx.x * 64 + threadIdx.x;
     if (i >= I) return;
     TopCells t;
     t.init();
-    for (int q = g.pbeg[i]; q < g.pbeg[i + 1]; ++q) {
-        const int sl = g.pslot[q];
-        int lo = 0, hi = C;  // largest c with sbeg[c] <= sl
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (g.sbeg[mid] <= sl) lo = mid;
-            else hi = mid;
+    const int q1 = g.pbeg[i + 1];
+    for (int q = g.pbeg[i]; q < q1; q += kAheadS) {
+        int sl[kAheadS], lo[kAheadS];
+        float v[kAheadS];
+#pragma unroll
+        for (int u = 0; u < kAheadS; ++u) {
+            sl[u] = g.pslot[min(q + u, q1 - 1)];
+            v[u] = pm[sl[u]];
+            lo[u] = 0;
         }
-        t.offer(pm[sl], lo);
+        // largest c in [0, C) with sbeg[c] <= sl, for all of them at once
+        for (int step = 1 << (31 - __clz(C)); step > 0; step >>= 1)
+#pragma unroll
+            for (int u = 0; u < kAheadS; ++u)
+                if (lo[u] + step < C && g.sbeg[lo[u] + step] <= sl[u]) lo[u] += step;
+#pragma unroll
+        for (int u = 0; u < kAheadS; ++u)
+            if (q + u < q1) t.offer(v[u], lo[u]);
     }
     t.store(out + (size_t)i * R, R);
 }
@@ -502,7 +535,7 @@ hipError_t launch_recall_grouped(const emc_ctx *c, hipStream_t st)
     const int R = p->o.recall;
     if (R < 1 || R > kMaxRecall) return R == 0 ? hipSuccess : hipErrorInvalidValue;
     const GTab g = tables(c, nullptr);
-    hipLaunchKernelGGL(k_recall_slots, dim3((c->I + 255) / 256), dim3(256), 0, st, p->slot_pm, g, c->I, p->C, R,
+    hipLaunchKernelGGL(k_recall_slots, dim3((c->I + 63) / 64), dim3(64), 0, st, p->slot_pm, g, c->I, p->C, R,
                        p->recall);
     return hipGetLastError();
 }
