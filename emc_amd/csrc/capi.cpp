@@ -356,10 +356,11 @@ extern "C" emc_status emc_create(const emc_dims *d, const emc_options *o, emc_ct
     if (st == EMC_OK && c->side) A(launch_fill_f64(c->scal, 0.0, SC_N, c->side), "side stream");
     if (st == EMC_OK) A(hipHostMalloc((void **)&c->scal_h, sizeof(double) * SC_N, hipHostMallocDefault), "scal_h");
     c->out_slot = std::min<int64_t>(2 * N3, kOutSlot);
-    if (st == EMC_OK)
-        A(hipHostMalloc((void **)&c->out_h, sizeof(float) * c->out_slot * kOutSlots, hipHostMallocDefault), "out_h");
+    // (as many slots as both arrays have pieces; the threaded form, from eight pieces on, has them all)
+    const size_t out_bytes = sizeof(float) * c->out_slot * std::min<int64_t>(kOutSlots, (2 * N3 + c->out_slot - 1) / c->out_slot);
+    if (st == EMC_OK) A(hipHostMalloc((void **)&c->out_h, out_bytes, hipHostMallocDefault), "out_h");
     // its pages are mapped at the first touch (about 1 ms): here, not in the first emc_get_model
-    if (st == EMC_OK) std::memset(c->out_h, 0, sizeof(float) * c->out_slot * kOutSlots);
+    if (st == EMC_OK) std::memset(c->out_h, 0, out_bytes);
     for (auto &e : c->out_ev)
         if (st == EMC_OK) A(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event");
     if (st == EMC_OK) A(hipDeviceSynchronize(), "sync");  // every null-stream fill is done
