@@ -38,7 +38,8 @@ struct Cfg {
     static_assert(STAGE % 1024 == 0 && LPW < 16 && ST * STAGE <= 159744);
 };
 
-template <int EPI, int NA, int NB, int WGM, int TN>
+// SPLIT: the logits of two-term counts; with NB = 1 the sums of the leading count terms are in C already.
+template <int EPI, int NA, int NB, int WGM, int TN, bool SPLIT>
 __global__ __launch_bounds__(128 * WGM) void k_dma(const bf16_t *__restrict__ A0, const bf16_t *__restrict__ A1,
                                              const bf16_t *__restrict__ A2, int64_t lda,
                                              const bf16_t *__restrict__ B0, const bf16_t *__restrict__ B1, int64_t ldb,
@@ -239,7 +240,7 @@ __global__ __launch_bounds__(128 * WGM) void k_dma(const bf16_t *__restrict__ A0
     if (live) kloop(std::true_type{});
     else kloop(std::false_type{});
     __syncthreads();  // the epilogue reuses the LDS
-    if (EPI == EPI_LOGL && e.accumulate) {  // the sums of the term pairs an earlier launch left in C
+    if constexpr (EPI == EPI_LOGL && SPLIT && NB == 1) {  // the sums of the term pairs an earlier launch left in C
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -255,7 +256,7 @@ __global__ __launch_bounds__(128 * WGM) void k_dma(const bf16_t *__restrict__ A0
         __syncthreads();  // packed columns may land on another wave's rows
     }
     if constexpr (EPI == EPI_LOGL) {
-        logl_epilogue<WGM, TN, BN>(acc, e, m0, n0, wm, wn, smem, bias_s, e.runmax ? rm_s : nullptr);
+        logl_epilogue<WGM, TN, BN, SPLIT>(acc, e, m0, n0, wm, wn, smem, bias_s, e.runmax ? rm_s : nullptr);
     } else {
 #pragma unroll
         for (int i = 0; i < 2; ++i)
@@ -275,26 +276,26 @@ __global__ __launch_bounds__(128 * WGM) void k_dma(const bf16_t *__restrict__ A0
     }
 }
 
-template <int EPI, int NA, int NB, int WGM, int TN>
+template <int EPI, int NA, int NB, int WGM, int TN, bool SPLIT>
 hipError_t launch(const Contraction &g, hipStream_t st)
 {
     const int ntm = g.M / (64 * WGM), ntn = (g.N + 64 * TN - 1) / (64 * TN);
     const int gm = std::max(1, std::min(g.e.tile_rows > 0 ? g.e.tile_rows : kTileRows, ntm));
-    hipLaunchKernelGGL((k_dma<EPI, NA, NB, WGM, TN>), dim3(ntm * ntn), dim3(128 * WGM), 0, st, g.A[0], g.A[1], g.A[2], g.lda, g.B[0],
+    hipLaunchKernelGGL((k_dma<EPI, NA, NB, WGM, TN, SPLIT>), dim3(ntm * ntn), dim3(128 * WGM), 0, st, g.A[0], g.A[1], g.A[2], g.lda, g.B[0],
                        g.B[1], g.ldb, g.N, g.K, ntn, gm, g.e);
     return hipGetLastError();
 }
 
-template <int EPI, int NA, int NB>
+template <int EPI, int NA, int NB, bool SPLIT = false>
 hipError_t pick(const Contraction &g, hipStream_t st)
 {
     switch (g.tile) {
-    case kTile256: return launch<EPI, NA, NB, 4, 4>(g, st);
+    case kTile256: return launch<EPI, NA, NB, 4, 4, SPLIT>(g, st);
     case kTile256x320:
-        if constexpr (NA == 2) return launch<EPI, NA, NB, 4, 5>(g, st);
+        if constexpr (NA == 2 && !(SPLIT && NB == 1)) return launch<EPI, NA, NB, 4, 5, SPLIT>(g, st);
         break;
-    case kTile256x128: return launch<EPI, NA, NB, 4, 2>(g, st);
-    case kTile128: return launch<EPI, NA, NB, 2, 2>(g, st);
+    case kTile256x128: return launch<EPI, NA, NB, 4, 2, SPLIT>(g, st);
+    case kTile128: return launch<EPI, NA, NB, 2, 2, SPLIT>(g, st);
     case kTile64: break;
     }
     return hipErrorInvalidValue;
@@ -336,8 +337,9 @@ hipError_t run_dma(int epi, const Contraction &g, hipStream_t st)
         return hipErrorInvalidValue;
     const int k = g.na * 4 + g.nb;
     if (epi == EPI_LOGL) {
+        if (k == 9 && g.split) return pick<EPI_LOGL, 2, 1, true>(g, st);
         if (k == 9) return pick<EPI_LOGL, 2, 1>(g, st);
-        if (k == 10) return pick<EPI_LOGL, 2, 2>(g, st);
+        if (k == 10) return pick<EPI_LOGL, 2, 2, true>(g, st);
         if (k == 13) return pick<EPI_LOGL, 3, 1>(g, st);
     } else {
         if (k == 5) return pick<EPI_STORE, 1, 1>(g, st);

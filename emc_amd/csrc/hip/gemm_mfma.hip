@@ -470,7 +470,7 @@ static hipError_t contract(int epi, const Contraction &g, hipStream_t st)
     h.na = 2;
     h.nb = 1;
     h.B[0] = g.B[1];
-    h.e.accumulate = true;
+    h.split = h.e.accumulate = true;
     return run_dma(epi, h, st);
 }
 

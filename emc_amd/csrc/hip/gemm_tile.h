@@ -41,7 +41,7 @@ struct EpiArgs {
     // once when *gate <= gate_thr (the responsibilities' non-zero count is small)
     const double *gate;
     double gate_thr;
-    bool accumulate;  // store epilogue: C += acc instead of C = acc
+    bool accumulate;  // store epilogue (and the logL's where split names it): C += acc instead of C = acc
     int tile_rows;    // large-tile kernel: row panels per tile group (0 = kTileRows)
 };
 
@@ -84,9 +84,10 @@ constexpr double kSkipStoreNats = 128.0;
 // softmax partials of this 256-row band (e.pm and e.ps: the large-tile logL kernels run only with
 // the softmax fused) restate k_sm_partial's rules: column maxima from the -1e10 floor, over the lane
 // pair, then over the 4 row-waves through LDS; then the sums of exp(R - max), where a term with
-// R - max <= -1e10 (or not a number) adds nothing.  Each lane sums its 32 terms of a column in FP32
-// on the hardware exp2 (the exponent floored at -1e10, whose exp2 is 0); the lane and wave partials
-// are added in FP64.
+// R - max <= -1e10 (or not a number) adds nothing.  With one-term counts each lane sums its 32 terms of a
+// column in FP32 on the hardware exp2 (the exponent floored at -1e10, whose exp2 is 0) and the lane and wave
+// partials are added in FP64; with two-term counts (SPLIT) every term is an expf and is added in FP64, as in
+// k_sm_partial, which forms these sums where the tile is 64 x 64.
 // The logits are stored after the maxima are known.  Without e.blk every logit is stored in place
 // (row-major R).  With e.blk (the iteration's store skipping): a column whose band maximum lies
 // kSkipStoreNats below rmk[column of the tile] (running maxima read when the workgroup started:
@@ -101,7 +102,7 @@ constexpr double kSkipStoreNats = 128.0;
 // the tile's 256 row biases, copied to LDS by the kernel (0 past m_valid), so no vector-memory wait
 // holds up the logit stores (on gfx9 a wait for a load also waits for every store issued before it)
 // and no bias stays in registers between the passes.
-template <int WGM, int TN, int BN2, bool kFull>
+template <int WGM, int TN, int BN2, bool SPLIT, bool kFull>
 __device__ __forceinline__ void logl_epi(const f32x16 (&acc)[2][TN], const EpiArgs &e, int m0, int n0, int wm, int wn,
                                          void *lds, const float *bias_lds, const int32_t *rmk)
 {
@@ -165,17 +166,20 @@ __device__ __forceinline__ void logl_epi(const f32x16 (&acc)[2][TN], const EpiAr
         if (lane == 0 && nskip > 0) atomicAdd(e.skipped, (double)nskip);
     }
     constexpr float kLog2e = 1.4426950408889634f;
-    float fs[TN];
+    std::conditional_t<SPLIT, double, float> fs[TN];
 #pragma unroll
-    for (int j = 0; j < TN; ++j) fs[j] = 0.0f;
+    for (int j = 0; j < TN; ++j) fs[j] = 0;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const float add = bias(i, r);
 #pragma unroll
-            for (int j = 0; j < TN; ++j)
-                fs[j] += __builtin_amdgcn_exp2f(fmaxf((acc[i][j][r] + add) - cmax[j], -1.0e10f) * kLog2e);
+            for (int j = 0; j < TN; ++j) {
+                const float d = fmaxf((acc[i][j][r] + add) - cmax[j], -1.0e10f);
+                if constexpr (SPLIT) fs[j] += (double)expf(d);
+                else fs[j] += __builtin_amdgcn_exp2f(d * kLog2e);
+            }
         }
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
@@ -237,13 +241,13 @@ __device__ __forceinline__ void logl_epi(const f32x16 (&acc)[2][TN], const EpiAr
     }
 }
 
-template <int WGM, int TN, int BN2>
+template <int WGM, int TN, int BN2, bool SPLIT = false>
 __device__ __forceinline__ void logl_epilogue(const f32x16 (&acc)[2][TN], const EpiArgs &e, int m0, int n0, int wm, int wn,
                                               void *lds, const float *bias_lds, const int32_t *rmk = nullptr)
 {
     if (m0 + 64 * WGM <= e.m_valid && n0 + BN2 <= e.n_valid)
-        logl_epi<WGM, TN, BN2, true>(acc, e, m0, n0, wm, wn, lds, bias_lds, rmk);
-    else logl_epi<WGM, TN, BN2, false>(acc, e, m0, n0, wm, wn, lds, bias_lds, rmk);
+        logl_epi<WGM, TN, BN2, SPLIT, true>(acc, e, m0, n0, wm, wn, lds, bias_lds, rmk);
+    else logl_epi<WGM, TN, BN2, SPLIT, false>(acc, e, m0, n0, wm, wn, lds, bias_lds, rmk);
 }
 
 // The contraction C [M][N] (row stride e.ldc) = sum over the term pairs (a, b), a + b < max(na, nb), of
@@ -257,6 +261,7 @@ struct Contraction {
     const bf16_t *A[3] = {nullptr, nullptr, nullptr}, *B[2] = {nullptr, nullptr};
     int64_t lda = 0, ldb = 0;
     int M = 0, N = 0, K = 0;
+    bool split = false;     // run_dma's logits: two-term counts' (the last of the launches that take them, where several do)
     bool two_sums = false;  // kTile64 with nb = 2: the products of the two B terms summed apart, then added
     EpiArgs e{};
 };
