@@ -316,9 +316,10 @@ __device__ __forceinline__ void pattern_const(const bf16_t *__restrict__ K16, co
 
 // Centred log-slice x = (log W + log phi0, or 0 where W <= 0) - colmean[j], from the log W kept by the
 // statistics pass, split into NT BF16 terms (hi, [mid,] lo) whose sum carries ~8*NT significant bits
-// of x.  The workgroups past the first nsplit rows of the grid form the patterns' constants, which
+// of x.  The workgroups past the first gx * nsplit (gx for a row of groups) form the patterns' constants, which
 // depend on the same column means (a launch of their own took 13 us at 32^3 / 1,000 patterns and 60 us with
-// split counts read element by element).  Four pixels per thread and kSplitRows rows per workgroup, whose loads are issued
+// split counts read element by element).  One flat grid: a second dimension is documented to 65,536 groups, which
+// 262,144 patterns of up to 1,024 pixels would pass.  Four pixels per thread and kSplitRows rows per workgroup, whose loads are issued
 // together (the column means are read once for all of them).  Pp is a multiple of 128.
 constexpr int kSplitRows = 8;
 
@@ -326,17 +327,17 @@ template <int NT>
 __global__ __launch_bounds__(256) void k_split_bf16(const float *__restrict__ lw, int s0, int cs, int Pa, int Pp,
                                                     const float *__restrict__ colmean,
                                                     const double *__restrict__ scal, bf16_t *__restrict__ Lh,
-                                                    bf16_t *__restrict__ Lm, bf16_t *__restrict__ Ll, int nsplit,
+                                                    bf16_t *__restrict__ Lm, bf16_t *__restrict__ Ll, int gx, int nsplit,
                                                     const bf16_t *__restrict__ K16, const bf16_t *__restrict__ K16lo,
                                                     const uint8_t *__restrict__ K8, int I, double *__restrict__ cst)
 {
-    if ((int)blockIdx.y >= nsplit) {
-        const int i = (((int)blockIdx.y - nsplit) * (int)gridDim.x + (int)blockIdx.x) * 4 + (int)(threadIdx.x >> 6);
+    if ((int)blockIdx.x >= gx * nsplit) {
+        const int i = ((int)blockIdx.x - gx * nsplit) * 4 + (int)(threadIdx.x >> 6);
         if (i < I) pattern_const(K16, K16lo, K8, i, Pp, colmean, scal[SC_B0], cst);  // a whole wavefront
         return;
     }
-    const int r0 = blockIdx.y * kSplitRows;
-    const int j0 = (blockIdx.x * 256 + threadIdx.x) * 4;
+    const int r0 = blockIdx.x / gx * kSplitRows;
+    const int j0 = (blockIdx.x % gx * 256 + threadIdx.x) * 4;
     if (j0 >= Pp) return;
     const float logphi0 = (float)scal[SC_LOGPHI0];
     float cm[4];
@@ -598,10 +599,10 @@ hipError_t launch_slice_f32(const emc_ctx *c, int s0, int cs, hipStream_t st)
 hipError_t launch_slice_bf16(const emc_ctx *c, int s0, int cs, hipStream_t st)
 {
     const int gx = (c->Pp / 4 + 255) / 256, nsplit = (c->chunkp + kSplitRows - 1) / kSplitRows;
-    const int nconst = s0 == 0 ? ((c->I + 3) / 4 + gx - 1) / gx : 0;  // the constants go with the first chunk
+    const int nconst = s0 == 0 ? (c->I + 3) / 4 : 0;  // the constants go with the first chunk
     const auto run = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(gx, nsplit + nconst), dim3(256), 0, st, c->lw32, s0, cs, c->Pa, c->Pp, c->colmean,
-                           c->scal, c->Lh, c->Lm, c->Ll, nsplit, c->K16, c->k_split ? c->K16lo : nullptr, c->K8, c->I,
+        hipLaunchKernelGGL(kernel, dim3(gx * nsplit + nconst), dim3(256), 0, st, c->lw32, s0, cs, c->Pa, c->Pp, c->colmean,
+                           c->scal, c->Lh, c->Lm, c->Ll, gx, nsplit, c->K16, c->k_split ? c->K16lo : nullptr, c->K8, c->I,
                            c->cst);
     };
     if (c->la_terms == 3) run(k_split_bf16<3>);
