@@ -393,11 +393,13 @@ __global__ __launch_bounds__(256) void k_expand(const float *__restrict__ model,
 
 // Fluence, per-rotation logit terms and pixel column means.  Every workgroup forms the total
 // sum_s sumW_s itself (the same fixed order in each, so the same value) and writes its share of the
-// rotations and pixels; workgroup 0 writes the scalars.
+// rotations and pixels; workgroup 0 writes the scalars.  No more workgroups than the chip holds at once, since each reads
+// every sumW_s (an iteration of 1,000,000 rotations x 64 patterns at 12^3: 6,360 us with one per 256 rotations, 4,790 so).
 //   TRUE_POISSON: phi0 = fluence or (sumK/I)/(sum_s sumW_s / S);
 //                 bias_s = log w_s - phi0 sumW_s + B0, B0 = phi0 * mean_s sumW_s (a global
 //                 shift that keeps the stored logits small; it is returned through cst).
 //   chi^2 kinds:  bias_s = log w_s, rscale_s = 1/(2 n_s sigma^2) (0 when n_s = 0).
+constexpr int kBiasGroups = 512;
 __global__ __launch_bounds__(1024) void k_bias(const double *__restrict__ sumW, const int32_t *__restrict__ ns,
                                                const float *__restrict__ logw, int S, int Sp, int I,
                                                double sumK_total, double fluence, int diff, float sigma,
@@ -550,7 +552,7 @@ hipError_t launch_slice_stats(const emc_ctx *c, hipStream_t st)
 
 hipError_t launch_bias(const emc_ctx *c, float sigma, hipStream_t st)
 {
-    const int nb = std::max(1, (std::max(c->Sp, c->Pp) + 255) / 256);
+    const int nb = std::max(1, std::min((std::max(c->Sp, c->Pp) + 255) / 256, kBiasGroups));
     hipLaunchKernelGGL(k_bias, dim3(nb), dim3(1024), 0, st, c->sumW, c->ns, c->logw, c->S, c->Sp, c->I,
                        c->sumK_total, c->opt.fluence, c->opt.diff, sigma,
                        c->mfma && !c->chi2_mfma ? c->colpart : nullptr, c->Pa, c->Pp, c->bias, c->rscale, c->colmean,
