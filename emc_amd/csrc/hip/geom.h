@@ -94,6 +94,14 @@ __device__ __forceinline__ uint32_t quad_index(int x, int y, int z, uint32_t nb)
            (uint32_t)((z & 1) * 4 + (y & 1) * 2 + (x & 1));
 }
 
+// Lower corner, on one axis, of the cell that holds u or is nearest to it, for any float: it is brought into range before the
+// conversion, which is undefined outside an int's (coordinates of 1e30 are finite and accepted, and their rotated points
+// may overflow).
+__host__ __device__ __forceinline__ int nearest_cell(float u, int L)
+{
+    return (int)__builtin_fminf(__builtin_fmaxf(__builtin_floorf(u), 0.0f), (float)(L - 2));
+}
+
 // Trilinear sample from it: the same corners, test and arithmetic as sample<EMC_INTERP_TRILINEAR>, so the same value
 // bit for bit.  The loads do not wait for the test (a point outside reads the nearest cell), so those of
 // several samples are in flight together.
@@ -104,8 +112,7 @@ __device__ __forceinline__ float sample_quad(const float4 *__restrict__ modelq, 
     rot_point(m, X, Y, Z, model_c(L), ux, uy, uz);
     const float hi = (float)(L - 1);
     const bool ok = ux >= 0.0f && ux <= hi && uy >= 0.0f && uy <= hi && uz >= 0.0f && uz <= hi;
-    const auto cell = [&](float u) { return max(min((int)__builtin_floorf(u), L - 2), 0); };
-    const int bx = cell(ux), by = cell(uy), bz = cell(uz);
+    const int bx = nearest_cell(ux, L), by = nearest_cell(uy, L), bz = nearest_cell(uz, L);
     const float fx = ux - (float)bx, fy = uy - (float)by, fz = uz - (float)bz;
     const uint32_t nb = (uint32_t)quad_blocks(L);
     const uint32_t base = quad_index(bx, by, bz, nb);
