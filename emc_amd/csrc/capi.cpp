@@ -8,12 +8,11 @@
 #include <cstring>
 #include <mutex>
 #include <string>
-#include <system_error>
-#include <thread>
 #include <vector>
 
 #include "emc_internal.h"
 #include "host/host_internal.h"
+#include "host/shared_work.h"
 
 const char *emc_host_last_error();
 
@@ -620,18 +619,7 @@ static hipError_t read_out(emc_ctx *c, const float *a, float *da, const float *b
         }
         err[t] = e;
     };
-    std::thread helper[3];
-    for (int t = 1; t < threads; ++t) {
-        try {
-            helper[t - 1] = std::thread(work, t);
-        } catch (const std::system_error &) {  // no thread to be had: its pieces are copied below
-        }
-    }
-    work(0);
-    for (int t = 1; t < threads; ++t) {
-        if (helper[t - 1].joinable()) helper[t - 1].join();
-        else work(t);
-    }
+    run_shared<4>(threads, work);
     hipError_t e = hipStreamSynchronize(c->stream);  // also after an error: no kernel may still write a slot
     for (int t = 0; t < threads; ++t)
         if (err[t] != hipSuccess) e = err[t];
