@@ -38,9 +38,12 @@ struct Cfg {
     static_assert(STAGE % 1024 == 0 && LPW < 16 && ST * STAGE <= 159744);
 };
 
-// SPLIT: the logits of two-term counts; with NB = 1 the sums of the leading count terms are in C already.
+// SPLIT, logL: the logits of two-term counts; with NB = 1 the sums of the leading count terms are in C already.
+// SPLIT, store: two sums (Contraction::two_sums).  In one chain the low term's products, 2^-8 of the others and less,
+// would each be rounded to the high sum's size: chi^2 log-sum-exps at 64^3, 6,300 x 2,000 were 4 % (absolute, two-term) to
+// 20 % (scaled, normalised patterns, three-term) further from 64 bits so.
 template <int EPI, int NA, int NB, int WGM, int TN, bool SPLIT>
-__global__ __launch_bounds__(128 * WGM) void k_dma(const bf16_t *__restrict__ A0, const bf16_t *__restrict__ A1,
+__global__ __launch_bounds__(128 * WGM, EPI == EPI_STORE && SPLIT ? 2 : 1) void k_dma(const bf16_t *__restrict__ A0, const bf16_t *__restrict__ A1,
                                              const bf16_t *__restrict__ A2, int64_t lda,
                                              const bf16_t *__restrict__ B0, const bf16_t *__restrict__ B1, int64_t ldb,
                                              int N, int Kd, int ntn, int gm, EpiArgs e)
@@ -110,13 +113,14 @@ __global__ __launch_bounds__(128 * WGM) void k_dma(const bf16_t *__restrict__ A0
         }
     };
 
-    f32x16 acc[2][TN];
+    constexpr bool TWO = EPI == EPI_STORE && SPLIT;  // the products with B1 are summed in acc1
+    f32x16 acc[2][TN], acc1[2][TN];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = acc1[i][j][r] = 0.0f;
     const int fr = lane & 31, sw = lds_swz(fr & 15), c0 = lane >> 5;
     struct Frag {
         bf16x8 a[NA][2], b[NB][TN];
@@ -144,8 +148,10 @@ __global__ __launch_bounds__(128 * WGM) void k_dma(const bf16_t *__restrict__ A0
 #pragma unroll
                     for (int i = 0; i < 2; ++i)
 #pragma unroll
-                        for (int j = 0; j < TN; ++j)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(F.a[a][i], F.b[t][j], acc[i][j], 0, 0, 0);
+                        for (int j = 0; j < TN; ++j) {
+                            f32x16 &to = TWO && t == 1 ? acc1[i][j] : acc[i][j];
+                            to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(F.a[a][i], F.b[t][j], to, 0, 0, 0);
+                        }
     };
 
     const int nk = Kd / BK2;
@@ -240,6 +246,13 @@ __global__ __launch_bounds__(128 * WGM) void k_dma(const bf16_t *__restrict__ A0
     if (live) kloop(std::true_type{});
     else kloop(std::false_type{});
     __syncthreads();  // the epilogue reuses the LDS
+    if constexpr (TWO)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[i][j][r] += acc1[i][j][r];
     if constexpr (EPI == EPI_LOGL && SPLIT && NB == 1) {  // the sums of the term pairs an earlier launch left in C
 #pragma unroll
         for (int i = 0; i < 2; ++i)
@@ -289,10 +302,13 @@ hipError_t launch(const Contraction &g, hipStream_t st)
 template <int EPI, int NA, int NB, bool SPLIT = false>
 hipError_t pick(const Contraction &g, hipStream_t st)
 {
+    constexpr bool kWide = !(EPI == EPI_STORE && SPLIT);  // twice the accumulators of 256 x 256 do not fit the registers
     switch (g.tile) {
-    case kTile256: return launch<EPI, NA, NB, 4, 4, SPLIT>(g, st);
+    case kTile256:
+        if constexpr (kWide) return launch<EPI, NA, NB, 4, 4, SPLIT>(g, st);
+        break;
     case kTile256x320:
-        if constexpr (NA == 2 && !(SPLIT && NB == 1)) return launch<EPI, NA, NB, 4, 5, SPLIT>(g, st);
+        if constexpr (kWide && NA == 2 && !(SPLIT && NB == 1)) return launch<EPI, NA, NB, 4, 5, SPLIT>(g, st);
         break;
     case kTile256x128: return launch<EPI, NA, NB, 4, 2, SPLIT>(g, st);
     case kTile128: return launch<EPI, NA, NB, 2, 2, SPLIT>(g, st);
@@ -331,6 +347,18 @@ GemmTile pick_tile(int64_t rows, int64_t cols, int na, int nb)
     return t256 <= t2x1 && t256 <= t128 ? kTile256 : t2x1 <= t128 ? kTile256x128 : kTile128;
 }
 
+// Two sums: the tiles whose two sets of accumulators fit the registers, by the costs above.  An iteration of scaled
+// chi^2, 6,300 x 4,000 at 64^3: 2,180 us on 256 x 128 tiles; 2,090 with one sum on 256 x 256; 2,350 with a launch per
+// term, the second adding to what the first stored.
+GemmTile pick_tile_two(int64_t rows, int64_t cols, int na)
+{
+    const auto tiles = [&](int64_t bm, int64_t bn) { return (rows + bm - 1) / bm * ((cols + bn - 1) / bn); };
+    if (tiles(256, 256) <= kSmallTiles) return kTile64;
+    const double t2x1 = (double)((tiles(256, 128) + 255) / 256) * 0.53;
+    const double t128 = std::max(0.66, (double)tiles(128, 128) / 512.0 * (na == 2 ? 0.74 : 0.80));
+    return t2x1 <= t128 ? kTile256x128 : kTile128;
+}
+
 hipError_t run_dma(int epi, const Contraction &g, hipStream_t st)
 {
     if (g.M % BM2 || g.N % 128 || g.K % BK2 || g.N < 128 || g.lda >= (1 << 26) || g.ldb >= (1 << 26))
@@ -343,8 +371,9 @@ hipError_t run_dma(int epi, const Contraction &g, hipStream_t st)
         if (k == 13) return pick<EPI_LOGL, 3, 1>(g, st);
     } else {
         if (k == 5) return pick<EPI_STORE, 1, 1>(g, st);
-        if (k == 6) return pick<EPI_STORE, 1, 2>(g, st);
         if (k == 9) return pick<EPI_STORE, 2, 1>(g, st);
+        if (k == 6 && g.two_sums) return pick<EPI_STORE, 1, 2, true>(g, st);
+        if (k == 10 && g.two_sums) return pick<EPI_STORE, 2, 2, true>(g, st);
         if (k == 10) return pick<EPI_STORE, 2, 2>(g, st);
         if (k == 13) return pick<EPI_STORE, 3, 1>(g, st);
     }

@@ -460,8 +460,7 @@ bool logl_skips_stores(const emc_ctx *c)
 static hipError_t contract(int epi, const Contraction &g, hipStream_t st)
 {
     if (g.tile == kTile64) return run_small(epi, g, st);
-    if (dma_takes(g.na, g.nb)) return run_dma(epi, g, st);
-    if (g.na != 3 || g.nb != 2) return hipErrorInvalidValue;
+    if (g.na < 3 || g.nb == 1) return run_dma(epi, g, st);
     Contraction h = g;  // (0, 0), (1, 0) and (2, 0), stored; then (0, 1) and (1, 1)
     h.nb = 1;
     hipError_t err = run_dma(EPI_STORE, h, st);
@@ -542,8 +541,8 @@ hipError_t launch_gemm_store_mfma(const emc_ctx *c, int na, const bf16_t *A0, co
     g.e.m_valid = c->chunkp;
     g.e.n_valid = c->Ip;
     g.e.accumulate = accumulate;
-    g.two_sums = true;
-    g.tile = pick_tile(c->chunkp, c->Ip, na, nb);
+    g.two_sums = nb == 2;
+    g.tile = g.two_sums && na < 3 ? pick_tile_two(c->chunkp, c->Ip, na) : pick_tile(c->chunkp, c->Ip, na, nb);
     if (g.tile >= kTile256x128 && c->opt.mfma_staging == 1 && nb == 1)
         return run_large<EPI_STORE>(c->chunkp, c->Ip, st, na, A0, A1, A2, c->Pp, B0, B8, c->Pp, c->Pp, g.e);
     g.na = na;

@@ -236,11 +236,9 @@ hipError_t run_small(int epi, const Contraction &g, hipStream_t st)
         if (g.na == 3) return launch<EPI_STORE, 3, 2, true>(g, st);
     } else {
         if (k == 5) return launch<EPI_STORE, 1, 1>(g, st);
-        if (k == 6) return launch<EPI_STORE, 1, 2>(g, st);
         if (k == 9) return launch<EPI_STORE, 2, 1>(g, st);
         if (k == 10) return launch<EPI_STORE, 2, 2>(g, st);
         if (k == 13) return launch<EPI_STORE, 3, 1>(g, st);
-        if (k == 14) return launch<EPI_STORE, 3, 2>(g, st);
     }
     return hipErrorInvalidValue;
 }

@@ -262,16 +262,16 @@ struct Contraction {
     int64_t lda = 0, ldb = 0;
     int M = 0, N = 0, K = 0;
     bool split = false;     // run_dma's logits: two-term counts' (the last of the launches that take them, where several do)
-    bool two_sums = false;  // kTile64 with nb = 2: the products of the two B terms summed apart, then added
+    bool two_sums = false;  // nb = 2, store epilogue: the products of the two B terms summed apart, then added
     EpiArgs e{};
 };
 
 // Tile for a contraction of this many rows, columns and terms, and its rows (the logL epilogue's maxima are over these).
 GemmTile pick_tile(int64_t rows, int64_t cols, int na, int nb);
+GemmTile pick_tile_two(int64_t rows, int64_t cols, int na);  // two_sums
 inline int tile_rows_of(GemmTile t) { return t == kTile64 ? 64 : t == kTile128 ? 128 : 256; }
-// epi: EPI_LOGL or EPI_STORE.  run_small: kTile64, every (na, nb); run_dma: the others, the pairs dma_takes names.
+// epi: EPI_LOGL or EPI_STORE.  run_small: kTile64; run_dma: the others, na + nb <= 4.
 hipError_t run_small(int epi, const Contraction &g, hipStream_t st);
-inline bool dma_takes(int na, int nb) { return na >= 1 && nb >= 1 && na + nb <= 4 && na <= 3 && nb <= 2; }
 hipError_t run_dma(int epi, const Contraction &g, hipStream_t st);
 
 }  // namespace emc
