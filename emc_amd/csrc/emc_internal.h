@@ -161,7 +161,7 @@ struct emc_ctx {
     // slicing stage
     double *sumW = nullptr;   // [Sp]
     int32_t *ns = nullptr;    // [Sp]
-    float2 *colp = nullptr;   // [ceil(S / 16)][Pp] per statistics block: (sum of log W, valid count)
+    float2 *colp = nullptr;   // [ceil(S / 8)][Pp] per statistics block: (sum of log W, valid count)
     double2 *colpart = nullptr; // [32][Pp] fixed-order partial column sums
     float *colmean = nullptr; // [Pp]
     float *bias = nullptr;    // [Sp] per-rotation additive term of the logits
@@ -274,17 +274,17 @@ hipError_t launch_square_counts(const emc_ctx *c, hipStream_t st);
 hipError_t launch_logl_mfma(const emc_ctx *c, int s0, int cs, hipStream_t st);
 // C [chunkp][Ip] (=, or += with accumulate) sum over pixels of A [chunkp][Pp] (na BF16 terms) and
 // the counts-like operand B [Ip][Pp] (nb BF16 terms; B8: the same as bytes, which the register-staged
-// kernels read), term pairs a + b < max(na, nb).
+// kernels read), term pairs a + b < max(na, nb), the products with each term of B summed apart.
 hipError_t launch_gemm_store_mfma(const emc_ctx *c, int na, const bf16_t *A0, const bf16_t *A1, const bf16_t *A2, int nb,
                                   const bf16_t *B0, const bf16_t *B1, const uint8_t *B8, float *C, bool accumulate,
                                   hipStream_t st);
-// chi^2 logits of rotations [s0, s0+cs) on the MFMA path, from the chunk's FP32 slices (A0 = W,
-// A1 = the pixel weight a): D = sum a W^2 - 2 ip sum a W K + ip^2 sum a K^2 over the valid pixels,
+// chi^2 logits of rotations [s0, s0+cs) on the MFMA path, from the W that the statistics pass kept (lw32; the
+// pixel weight a follows from it): D = sum a W^2 - 2 ip sum a W K + ip^2 sum a K^2 over the valid pixels,
 // ip = 1/phi (options.scaling: sum W K / sum K^2 over W > 1e-10; else 1); R = log w_s - D rscale_s.
 // With scaling, iphi rows [s0, s0+cs) are written for the M-step.
 hipError_t launch_logl_chi2_mfma(const emc_ctx *c, int s0, int cs, hipStream_t st);
-// Ph / Pl segments of 256 patterns tracked by pdirty, and marking every one as possibly non-zero
-// (after anything but the dense softmax wrote Ph / Pl).
+// Segments of 256 patterns of P (Ph / Pl, or R at FP32) tracked by pdirty, and marking every one as possibly
+// non-zero (after anything but the dense softmax wrote P).
 inline int p_segments(const emc_ctx *c) { return (c->I + 255) / 256; }
 hipError_t launch_mark_p_dirty(const emc_ctx *c, hipStream_t st);
 
@@ -328,7 +328,8 @@ hipError_t launch_blur_taps(int L, double sigma, float *taps, hipStream_t st);
 hipError_t launch_compress_buffers(int L, double blur_sigma, bool new_taps, const float *Mnum, const float *Wt,
                                    float *model, float *taps, float *t1, float *t2, double *red, double *scal,
                                    double *avg_out, hipStream_t st);
-// Deterministic single-workgroup sum of n doubles into *out.
+// The E-step's last sums, each in a fixed order: scal[SC_NNZ] of nz[nnz] (non-zero responsibilities), scal[SC_TOTAL] of
+// blk[nblk] (log-sum-exps) and the pattern constants, and, unless Tpart is null, T_s of its ncb rows.
 hipError_t launch_sm_sums(const emc_ctx *c, const double *nz, int nnz, const double *blk, int nblk, const double *Tpart,
                           int ncb, hipStream_t st);
 

@@ -6,7 +6,7 @@
 // two contractions over pixels of split-BF16 slice operands with the counts and the counts
 // squared (both exact in BF16: K, and K^2 as hi + lo), plus a per-rotation constant.  The scaling's
 // sums are two more contractions: sum K^2 over {W > 1e-10} (indicator operand, exact) and sum W K
-// over the same pixels.  The FP32 products go through the large-tile kernel's store epilogue; one
+// over the same pixels.  The FP32 products go through the contraction kernels' store epilogue; one
 // elementwise pass combines them into the logits (in double) and 1/phi.
 #include "../emc_internal.h"
 #include "geom.h"

@@ -348,8 +348,9 @@ GemmTile pick_tile(int64_t rows, int64_t cols, int na, int nb)
 }
 
 // Two sums: the tiles whose two sets of accumulators fit the registers, by the costs above.  An iteration of scaled
-// chi^2, 6,300 x 4,000 at 64^3: 2,180 us on 256 x 128 tiles; 2,090 with one sum on 256 x 256; 2,350 with a launch per
-// term, the second adding to what the first stored.
+// chi^2 at 64^3, us, on 128 x 128 tiles / by this rule: 6,300 x 1,000 1,101/1,051, x 2,000 1,477/1,377, x 4,000 2,323/2,126,
+// 10,860 x 4,000 3,809/3,566, not scaled 6,300 x 3,000 1,649/1,683.  With one sum on any tile 6,300 x 4,000 is 2,105, with a
+// launch per term, the second adding to what the first stored, 2,350.
 GemmTile pick_tile_two(int64_t rows, int64_t cols, int na)
 {
     const auto tiles = [&](int64_t bm, int64_t bn) { return (rows + bm - 1) / bm * ((cols + bn - 1) / bn); };

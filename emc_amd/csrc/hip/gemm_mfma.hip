@@ -1,6 +1,8 @@
 // MFMA contractions for CDNA4 (gfx950): C[m, n] = sum_k sum_{(a,b)} A_a[m, k] B_b[n, k]
 // with A and B given as BF16 terms whose sum carries the operand (A_0 = hi, A_1 = next 8 bits, ...)
-// and FP32 accumulation in the matrix cores.
+// and FP32 accumulation in the matrix cores.  Here are the launchers (which kernel a shape gets, the logL's bands and
+// stores) and the kernels that stage operands through registers: 128 x 128 tiles (mfma_tile = 1, and the fused scatter) and
+// 256-row tiles (mfma_staging = 1).  The default kernels, staged by DMA, are in gemm_dma.hip and gemm_small.hip.
 //
 //   logL   : A = centred log-slices (NA = 2 or 3 terms) [rows = rotations], B = counts
 //            [rows = patterns] (NB = 1, or 2 when a count exceeds 256), k = active pixels.
@@ -8,8 +10,8 @@
 //   M-step : A = responsibilities hi+lo [rows = rotations], B = counts^T [rows = pixels],
 //            k = patterns.  Epilogue: store U, or scatter U straight into the model (fused).
 //
-// Term pairs (a, b) with a + b < NA are accumulated (the dropped pairs are below 2^-8NA of the
-// product).  Tiling: 128 x 128 macro tile, 256 threads = 4 wavefronts of 64 lanes, each wave a
+// Term pairs (a, b) with a + b < NA (max(NA, NB) in the DMA kernels) are accumulated (the dropped pairs are below
+// 2^-8NA of the product).  The 128 x 128 kernel: macro tile, 256 threads = 4 wavefronts of 64 lanes, each wave a
 // 64 x 64 block of 2 x 2 v_mfma_f32_32x32x16_bf16 tiles; BK = 64; operands staged in LDS with
 // rows padded to 72 BF16 (144 B) so the 16-byte fragment reads of 16 lanes hit 64 distinct
 // banks; the next k-tile is fetched into registers while the current one is multiplied.
@@ -205,7 +207,7 @@ hipError_t run(dim3 grid, hipStream_t st, const bf16_t *A0, const bf16_t *A1, co
     return hipGetLastError();
 }
 
-// ---- large-tile variant ---------------------------------------------------------------------
+// ---- 256-row variant ------------------------------------------------------------------------
 // 256 x BN2 macro tile, 512 threads = 8 wavefronts (4 along M x 2 along N), each wave a 64 x BN2/2
 // block of 2 x (BN2/64) 32x32 tiles, so every A fragment (NA terms) feeds BN2/64 MFMAs and every
 // B fragment NA * 2.  BK = 32; two LDS stages (rows padded to 40 BF16 = 80 B: the 16-byte
@@ -215,7 +217,7 @@ hipError_t run(dim3 grid, hipStream_t st, const bf16_t *A0, const bf16_t *A1, co
 // Workgroups are renumbered so that each XCD (round-robin dispatch: workgroup b runs on XCD b % 8)
 // works on a contiguous band of tiles, which share A row panels in that XCD's L2.
 constexpr int BK2 = 32, LDK2 = BK2 + 8;
-constexpr int kTileRows = 1;  // default tile grouping of the large-tile kernel
+constexpr int kTileRows = 1;  // default row panels per group of consecutive tiles
 
 // Counts stored as bytes (exact to 255) widen to BF16 on the way to LDS: 8 bytes -> 8 BF16.
 __device__ __forceinline__ u32x4 widen_u8x8(u32x2 v)

@@ -1,7 +1,8 @@
 // MFMA contractions of small shapes: the 256-row tiles of gemm_dma.hip would leave most of the 256 CUs
 // idle (420 rotations x 64 patterns are two of them: 33 us, all latency), so the tile is 64 x 64, one
-// 32 x 32 block per wavefront.  Each element's products are added in the order of the large tiles
-// (k ascending, low terms first), so the results do not depend on the tile.
+// 32 x 32 block per wavefront.  Each element's products are added in the order of the larger tiles
+// (k ascending, low terms first; two sums where those have two), so the results do not depend on the tile; only the
+// logits of three-term slices with two-term counts do, in which the larger tiles add the low counts' products last.
 //
 // Bound by the latency of the loads along k: the operands go into LDS by DMA (gemm_dma.hip), 64 k at a time,
 // kST stages deep, so kST - 1 blocks are in flight, with one barrier per block.  A DMA instruction
@@ -158,7 +159,7 @@ __global__ __launch_bounds__(256) void k_small(const bf16_t *__restrict__ A0, co
         return;
     }
     // logL: the bias, the maxima of the tile's 64 rows (e.pm; k_sm_band forms the sums, from the stored logits) and
-    // the store skipping by the rules of the 256-row kernels' epilogue (every logit that is stored is stored in place)
+    // the store skipping by the rules of the larger tiles' epilogue (every logit that is stored is stored in place)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const int m = mw + 8 * (r >> 2) + 4 * fh + (r & 3);

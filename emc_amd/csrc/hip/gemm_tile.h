@@ -1,5 +1,5 @@
 // Device code shared by the MFMA contraction kernels (gemm_mfma.hip, gemm_dma.hip, gemm_small.hip):
-// fragment types, the epilogue's arguments and the logL epilogue of the 256-row kernels.
+// fragment types, the epilogue's arguments and the logL epilogue of the tiles of 128 and 256 rows.
 #pragma once
 
 #include <algorithm>
@@ -27,8 +27,8 @@ struct EpiArgs {
     const float *axyz;   // [3][Pp]
     int Pp, Pa, L, interp;
     float *Mnum, *Wt;
-    // softmax partials of the logL epilogue (large-tile kernel): per 256-row band and pattern,
-    // the band maximum pm and sum of exp(R - pm) ps; band = band0 + m-tile
+    // softmax partials of the logL epilogue: per band (the tile's rows) and pattern, the band
+    // maximum pm and (not from 64-row tiles) sum of exp(R - pm) ps; band = band0 + m-tile
     float *pm;
     double *ps;
     int64_t band0, ldp;
@@ -42,7 +42,7 @@ struct EpiArgs {
     const double *gate;
     double gate_thr;
     bool accumulate;  // store epilogue (and the logL's where split names it): C += acc instead of C = acc
-    int tile_rows;    // large-tile kernel: row panels per tile group (0 = kTileRows)
+    int tile_rows;    // row panels per group of consecutive tiles (0 = kTileRows; not 64 x 64 tiles)
 };
 
 constexpr int BM2 = 256;  // rows of the large tiles
@@ -78,12 +78,12 @@ constexpr int32_t kOrdNegInf = (int32_t)0x807fffff;
 // kSkipApplyNats below the pattern's lse as -inf, computes P = 0 there from the band maxima alone.
 constexpr double kSkipStoreNats = 128.0;
 
-// logL epilogue of the 256-row large-tile kernels (8 waves: 4 along M x 2 along N, each a 64-row
+// logL epilogue of the tiles of 256 and 128 rows (WGM = 4 or 2 waves along M x 2 along N, each a 64-row
 // by BN2/2-column block of 2 x TN 32x32 tiles).  Accumulator layout: lane holds column lane % 32
 // of each 32x32 tile and rows 8*(r/4) + 4*(lane/32) + r%4, r = 0..15.  R = acc + bias_s.  The
-// softmax partials of this 256-row band (e.pm and e.ps: the large-tile logL kernels run only with
+// softmax partials of this band, the tile's rows (e.pm and e.ps: these kernels run only with
 // the softmax fused) restate k_sm_partial's rules: column maxima from the -1e10 floor, over the lane
-// pair, then over the 4 row-waves through LDS; then the sums of exp(R - max), where a term with
+// pair, then over the row-waves through LDS; then the sums of exp(R - max), where a term with
 // R - max <= -1e10 (or not a number) adds nothing.  With one-term counts each lane sums its 32 terms of a
 // column in FP32 on the hardware exp2 (the exponent floored at -1e10, whose exp2 is 0) and the lane and wave
 // partials are added in FP64; with two-term counts (SPLIT) every term is an expf and is added in FP64, as in
@@ -91,7 +91,7 @@ constexpr double kSkipStoreNats = 128.0;
 // The logits are stored after the maxima are known.  Without e.blk every logit is stored in place
 // (row-major R).  With e.blk (the iteration's store skipping): a column whose band maximum lies
 // kSkipStoreNats below rmk[column of the tile] (running maxima read when the workgroup started:
-// lower bounds of the pattern's largest logit) is not stored; in a tile inside the valid rows and
+// lower bounds of the pattern's largest logit) is not stored; in a 256 x 256 tile inside the valid rows and
 // columns the kept columns are packed, in column order, as blocks of 256 consecutive floats (the
 // column's rows) in the tile's own rows of R (block k in row m0 + k, columns n0 .. n0 + 255), so the
 // HBM writes are whole lines however few columns are kept; the other tiles store their kept columns
@@ -99,7 +99,7 @@ constexpr double kSkipStoreNats = 128.0;
 // band maximum is merged into e.runmax, and e.skipped counts the columns left out.
 // A tile inside the valid rows and columns (every tile but the last row band and column tile) takes
 // a path without bounds checks.  lds: 48 BN2 + 1056 bytes, free (the main loop's stages).  bias_lds:
-// the tile's 256 row biases, copied to LDS by the kernel (0 past m_valid), so no vector-memory wait
+// the tile's row biases, copied to LDS by the kernel (0 past m_valid), so no vector-memory wait
 // holds up the logit stores (on gfx9 a wait for a load also waits for every store issued before it)
 // and no bias stays in registers between the passes.
 template <int WGM, int TN, int BN2, bool SPLIT, bool kFull>

@@ -24,10 +24,11 @@ __device__ __forceinline__ T wave_sum(T v)
     return v;
 }
 
-// Partials of the 256-row bands where the logL ran on 64-row tiles, whose epilogue wrote the maxima of the 64-row
-// groups (gm, [4 groups per band][I]): the sums of exp(R - max) in the order and arithmetic of the 256-row
-// kernels' epilogue (32 rows of a column in FP32, on the hardware exp2, the pairs and the groups of 64 rows in
-// FP64), so the partials do not depend on the tile.  A group whose logits were left out (gblk, null: none) adds
+// Partials of the 256-row bands where the logL ran on 64-row tiles with one-term counts, whose epilogue wrote the maxima
+// of the 64-row groups (gm, [4 groups per band][I]): the sums of exp(R - max) in the order and arithmetic of the 256-row
+// tiles' epilogue (32 rows of a column in FP32, on the hardware exp2, the pairs and the groups of 64 rows in
+// FP64), so the partials are those of the 256-row tiles bit for bit (128-row tiles have bands of 128 rows, and two-term
+// counts on 64-row tiles take k_sm_partial: other sums, to rounding the same).  A group whose logits were left out (gblk, null: none) adds
 // nothing: its terms are below exp(-128) of the pattern's sum.  Bands count from each chunk's first rotation.
 // One workgroup takes 32 columns, a thread 32 rows of one; all latency: 5.5 us at
 // 3,880 x 777, 10.5 when the logits were read after the group's record.
