@@ -275,8 +275,11 @@ __global__ __launch_bounds__(256) void k_sm_apply(float *__restrict__ R, int64_t
     if (OUT == 1 && pm) {
         const int rl = min(r0 + kApplyRows - 1, S - 1);
         b0 = (r0 / chunk) * bpc + (r0 % chunk) / brows;
-        one_band = b0 == (rl / chunk) * bpc + (rl % chunk) / brows;
-        if (one_band) {  // the workgroup's rows lie in one band (always, when blk is given)
+        const int b1 = (rl / chunk) * bpc + (rl % chunk) / brows;
+        // the workgroup's rows lie in one band (always, when blk is given), or in two smaller ones of the same 256 rows of a
+        // chunk, taken as one: the sparse form, which adds each P in FP64, must not depend on the tile's rows
+        one_band = b0 == b1 || (!blk && r0 / chunk == rl / chunk && (r0 % chunk) / 256 == (rl % chunk) / 256);
+        if (one_band) {
             brow0 = (r0 / chunk) * chunk + ((r0 % chunk) / brows) * brows;
             float pv[4];
             int cv[4] = {-2, -2, -2, -2};
@@ -296,6 +299,10 @@ __global__ __launch_bounds__(256) void k_sm_apply(float *__restrict__ R, int64_t
                     if (blk && c0 + k < I) cv[k] = blk[o + k];
                 }
             }
+            if (b1 != b0)
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (c0 + k < I) pv[k] = fmaxf(pv[k], pm[(size_t)b1 * I + c0 + k]);
 #pragma unroll
             for (int k = 0; k < 4; ++k)
                 if (c0 + k < I) {
