@@ -17,7 +17,7 @@
 //
 // Launches: divide + statistics, then one pass per axis; the first axis pass finishes the statistics itself
 // (every workgroup adds the 256 block partials in the same order, so all get the same normaliser) and
-// scales what it reads, the last scales the missing voxels it keeps.  At small sides the launches are
+// scales what it reads, the last scales what it keeps.  At small sides the launches are
 // the time (about 4.6 us each in a stream).  emc_compress_device at 41^3 27 us, and 128^3 62 us (its passes 10,
 // 22, 16 and 20 us against 25 MB of traffic and 1.6 GFLOP); with a voxel per thread and axis, separate
 // divide, scale and average launches and a thread per tap 41 and 222 us.
@@ -202,7 +202,7 @@ __global__ __launch_bounds__(256) void k_scale(float *__restrict__ M, int64_t n,
 // vector ALU bounds it (a thread per voxel with its inputs from L2 took 56 us per axis at 128^3).
 // AXIS 0: lines are rows (x); it reads the divided model, finishes the statistics, scales and takes negatives
 // as 0.  AXIS 1 (y) and 2 (z): lines are columns, neighbouring lines contiguous in x.  AXIS 2 writes into the
-// model, where a negative (missing) voxel keeps its value, scaled.
+// model, where a voxel that is negative once scaled (a missing one) keeps that value.
 constexpr int kBlurThreads = 128;
 template <int AXIS, int NL>
 __global__ __launch_bounds__(kBlurThreads) void k_blur(const float *__restrict__ in, float *__restrict__ out,
@@ -230,6 +230,11 @@ __global__ __launch_bounds__(kBlurThreads) void k_blur(const float *__restrict__
         }
     };
     double inv = 1.0;
+    const auto kept = [&inv](float m, float x) {  // AXIS 2: the scaled value where it is negative, else the blurred one
+        if (!(m < 0.0f)) return x;
+        const float s = scaled(m, inv);
+        return s < 0.0f ? s : x;
+    };
     if constexpr (AXIS == 0) {
         const StatLoads<kBlurThreads> sl = load_stats<kBlurThreads>(part);
         for (int r = tid >> 6; r < NL; r += kBlurThreads / 64)
@@ -288,10 +293,7 @@ __global__ __launch_bounds__(kBlurThreads) void k_blur(const float *__restrict__
                     float4 v = make_float4(acc[0][i], acc[1][i], acc[2][i], acc[3][i]);
                     if (AXIS == 2) {
                         const float4 m = *o;
-                        v.x = m.x < 0.0f ? scaled(m.x, inv) : v.x;
-                        v.y = m.y < 0.0f ? scaled(m.y, inv) : v.y;
-                        v.z = m.z < 0.0f ? scaled(m.z, inv) : v.z;
-                        v.w = m.w < 0.0f ? scaled(m.w, inv) : v.w;
+                        v = make_float4(kept(m.x, v.x), kept(m.y, v.y), kept(m.z, v.z), kept(m.w, v.w));
                     }
                     *o = v;
                 }
@@ -309,7 +311,7 @@ __global__ __launch_bounds__(kBlurThreads) void k_blur(const float *__restrict__
 #pragma unroll
             for (int r = 0; r < 4; ++r)
                 if (c0 + i < L && 4 * lg + r < nl)
-                    out[f[r] + i * step] = AXIS == 2 && m[r][i] < 0.0f ? scaled(m[r][i], inv) : acc[r][i];
+                    out[f[r] + i * step] = AXIS == 2 ? kept(m[r][i], acc[r][i]) : acc[r][i];
     }
 }
 
