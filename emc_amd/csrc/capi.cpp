@@ -626,6 +626,19 @@ static hipError_t read_out(emc_ctx *c, const float *a, float *da, const float *b
     return e;
 }
 
+// Memory that the runtime knows (pinned, managed): the device copies into it directly.
+static bool known_memory(const void *p)
+{
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();  // this call's own: the pointer is not known
+        return false;
+    }
+    return a.type != hipMemoryTypeUnregistered;
+}
+
+// An array whose destination the runtime knows is copied directly (through the slots it took 1.3 to 2 times as long: both
+// arrays 53 and 107 us at 64^3, 311 and 520 at 128^3), the others through the slots.
 extern "C" emc_status emc_get_model(emc_ctx *c, float *model, float *weight)
 {
     if (!c) return fail(c, EMC_E_INVALID, "get_model: null context");
@@ -633,9 +646,24 @@ extern "C" emc_status emc_get_model(emc_ctx *c, float *model, float *weight)
     const float *src[2];
     float *dst[2];
     int n = 0;
-    if (model) { src[n] = c->model; dst[n++] = model; }
-    if (weight) { src[n] = c->Wt; dst[n++] = weight; }
-    if (n > 0) HIP_TRY(c, read_out(c, src[0], dst[0], n > 1 ? src[1] : nullptr, n > 1 ? dst[1] : nullptr));
+    hipError_t e = hipSuccess;
+    const auto take = [&](const float *s, float *d) {
+        if (!d) return;
+        if (!known_memory(d)) {
+            src[n] = s;
+            dst[n++] = d;
+        } else if (e == hipSuccess) {
+            e = hipMemcpyAsync(d, s, sizeof(float) * c->N3, hipMemcpyDeviceToHost, c->stream);
+        }
+    };
+    take(c->model, model);
+    take(c->Wt, weight);
+    if (e == hipSuccess && n > 0) e = read_out(c, src[0], dst[0], n > 1 ? src[1] : nullptr, n > 1 ? dst[1] : nullptr);
+    else {
+        const hipError_t e2 = hipStreamSynchronize(c->stream);  // also after an error: no copy may still be under way
+        if (e == hipSuccess) e = e2;
+    }
+    HIP_TRY(c, e);
     return EMC_OK;
 }
 
