@@ -872,18 +872,19 @@ extern "C" emc_status emc_set_resp(emc_ctx *c, const float *resp)
     HIP_TRY(c, hipSetDevice(c->opt.device));
     const int S = c->S, I = c->I;
     std::vector<double> T(c->Sp, 0.0);
+    size_t set = 0;  // entries that are not zero, counted in the pass that checks them
     for (int s = 0; s < S; ++s) {
         double t = 0.0;
         for (int i = 0; i < I; ++i) {
             const float p = resp[(size_t)s * I + i];
             if (!(p >= 0.0f) || !std::isfinite(p)) return fail(c, EMC_E_INVALID, "set_resp: values must be finite and >= 0");
             t += p;
+            set += p != 0.0f;
         }
         T[s] = t;
     }
     if (!c->mfma) {
-        double nnz = 0.0;  // read by the M-step's choice of form, as after an E-step
-        for (size_t k = 0; k < (size_t)S * I; ++k) nnz += resp[k] != 0.0f;
+        const double nnz = (double)set;  // read by the M-step's choice of form, as after an E-step
         HIP_TRY(c, hipMemcpy(c->scal + SC_NNZ, &nnz, sizeof(double), hipMemcpyHostToDevice));
         HIP_TRY(c, hipMemcpy2D(c->R, sizeof(float) * c->Ip, resp, sizeof(float) * I, sizeof(float) * I, S,
                                hipMemcpyHostToDevice));
