@@ -223,6 +223,7 @@ struct emc_ctx {
     int32_t *bin_groups = nullptr;                     // [n_groups][4] = key, first block, end block (per chunk), 0
     int32_t *bin_gbeg = nullptr;                       // [chunks][bricks + 1] first group (bin_direct: block) of each brick
     float *bin_usum = nullptr;                         // [units of a chunk][2][corners][512] unit sums (null: a workgroup per block)
+    size_t bin_usum_bytes = 0;
     float *bin_part = nullptr;                         // [blocks of a chunk][2][9^3] block partials
     float *bin_gpart = nullptr;                        // [groups of a chunk][2][9^3] group partials
     std::vector<int> bin_chunk_units, bin_chunk_blocks, bin_chunk_groups; // unit / block / group range of each rotation chunk

@@ -558,7 +558,6 @@ hipError_t build_bins(emc_ctx *c, std::string &err)
     release(c->bin_groups);
     release(c->bin_gbeg);
     release(c->bin_part);
-    release(c->bin_usum);
     release(c->bin_gpart);
     chk(hipMalloc((void **)&kin, sizeof(uint32_t) * n));
     chk(hipMalloc((void **)&vin, sizeof(uint32_t) * n));
@@ -643,9 +642,16 @@ hipError_t build_bins(emc_ctx *c, std::string &err)
         chk(hipMalloc((void **)&c->bin_groups, sizeof(int32_t) * groups.size()));
         chk(hipMalloc((void **)&c->bin_gbeg, sizeof(int32_t) * gbeg.size()));
         chk(hipMalloc((void **)&c->bin_part, sizeof(float) * 2 * kHalo3 * (size_t)max_blocks));
-        if (split)
-            chk(hipMalloc((void **)&c->bin_usum,
-                          sizeof(float) * 2 * kBrick3 * (c->opt.interp == EMC_INTERP_NEAREST ? 1 : 8) * (size_t)max_units));
+        // Kept from one build to the next while it is large enough (it is at most 32 MB): freeing and allocating it again
+        // made a new mask or new rotations 0.2 to 0.3 ms slower (32^3 / 3,240: 1.9 -> 2.2 ms).
+        const size_t usum =
+            split ? sizeof(float) * 2 * kBrick3 * (c->opt.interp == EMC_INTERP_NEAREST ? 1 : 8) * (size_t)max_units : 0;
+        if (!split || usum > c->bin_usum_bytes) {
+            release(c->bin_usum);
+            c->bin_usum_bytes = 0;
+            if (split) chk(hipMalloc((void **)&c->bin_usum, usum));
+            if (c->bin_usum) c->bin_usum_bytes = usum;
+        }
         if (!c->bin_direct) chk(hipMalloc((void **)&c->bin_gpart, sizeof(float) * 2 * kHalo3 * (size_t)max_groups));
         chk(hipMalloc((void **)&c->bin_perm, sizeof(uint16_t) * n));
         chk(hipMalloc((void **)&c->bin_vbeg, sizeof(uint16_t) * kVbeg * (size_t)n_units));
